@@ -60,6 +60,12 @@ int tbf16_quantize_rows(const void* x, int64_t R, int64_t K, int64_t ldx, int t,
 int tbf16_quantize_rows_t(const void* x, int64_t R, int64_t K, int64_t ldx, int t, void* yT, int64_t ldyT,
                           float* s_inv, int32_t* exps_ws, void* stream);
 
+/* tbf16_quantize_rows (max scales) and tbf16_quantize_rows_t in one call: y16 (R, K),
+ * row stride ldy, and yT (K, R), row stride ldyT. For the training forward, whose own
+ * product reads y16 and whose dW reads yT (tbf16/autograd.py:60-68). */
+int tbf16_quantize_rows_both(const void* x, int64_t R, int64_t K, int64_t ldx, int t, void* y16, int64_t ldy, void* yT,
+                             int64_t ldyT, float* s_inv, int32_t* exps_ws, void* stream);
+
 /* Column quantisation: amax[c] = max_r |x[r,c] * row_mul[r]|, y = fp16((x * row_mul)
  * * 2^p[c]), s_inv[c] = 2^-p[c]; row_mul (R,) fp32 powers of two or NULL. The fp16
  * result is written transposed: yT (K, R), row stride ldyT >= R.
@@ -75,13 +81,12 @@ int tbf16_quantize_cols_t(const void* x, int64_t R, int64_t K, int64_t ldx, int 
  * x bf16 (M, K); w16 fp16 (N, K); ws fp32 (N,); bias bf16 (N,) or NULL; y bf16
  * (M, N). cfg < 0 picks the tile shape. workspace: tbf16_linear_ws_bytes(M, K, N,
  * cfg) bytes, 16-byte aligned; its first M int32 receive the row exponents p.
- * With the decode configurations, and with tiles of at most 128 columns at K >=
- * 1024, x is quantised once, as the reference's small-M path does: the row
- * inverse scales and x's scaled fp16 copy go into the workspace too, and the
- * GEMM runs on fp16 operands (the same output as converting x inside it). Where
- * the tiles would leave half of the CUs idle (K >= 2048, at most 8 MiB of partial
- * sums), K is split in two: fp32 partial sums go into the workspace and a second
- * kernel adds them in a fixed order and applies the epilogue. Replaces linear (tbf16/csrc/gemm_sm75.cu:257-284) and, at
+ * x is quantised once, as the reference's small-M path does: the row inverse scales
+ * and x's scaled fp16 copy go into the workspace too, and the GEMM runs on fp16
+ * operands (some pinned configurations convert x inside the GEMM instead). Where the
+ * tiles would leave CUs idle and K is long (at most 8 MiB of partial sums), K is split
+ * in up to eight: fp32 partial sums go into the workspace and a second kernel adds
+ * them in a fixed order and applies the epilogue. Replaces linear (tbf16/csrc/gemm_sm75.cu:257-284) and, at
  * 2 <= M < 256, quantize_rows + cuBLAS + epilogue (tbf16/ops.py:163-178) without
  * its fp16 intermediate. */
 size_t tbf16_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int cfg);

@@ -149,6 +149,46 @@ def test_gemm_small_integers_bit_exact(dev, cfg, K):
     assert np.array_equal(e.cpu().numpy(), O.row_exps(a.bfloat16(), 15))
 
 
+@pytest.mark.parametrize("K", [8, 64, 128, 200, 1000, 3040])
+@pytest.mark.parametrize("cfg", range(20, 31))
+def test_gemm_pingpong_small_integers_bit_exact(dev, cfg, K):
+    """The ping-pong configurations as above: exact integer products at one k tile (whole
+    and partial), two, an odd and an even number of tiles with a partial last one (the
+    group without a last tile reads zeros); rows and columns past whole tiles, and one
+    row of tiles against few columns (fewer columns per block than the tile has)."""
+    g = torch.Generator().manual_seed(11)
+    for M, N in ((523, 264), (29, 1032), (1, 8)):
+        a = torch.randint(-1, 2, (M, K), generator=g)
+        b = torch.randint(-1, 2, (N, K), generator=g)
+        bias = torch.randint(-8, 9, (N,), generator=g)
+        sa = torch.ldexp(torch.ones(M), torch.randint(-3, 4, (M,), generator=g).float())
+        sb = torch.ldexp(torch.ones(N), torch.randint(-3, 4, (N,), generator=g).float())
+        want = ((a @ b.t()).double() * sa.double()[:, None] * sb.double()[None, :] + bias.double()).bfloat16()
+        a16, b16, sad, sbd, bd = (t.to(dev) for t in (a.half(), b.half(), sa, sb, bias.bfloat16()))
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        _ext.call("tbf16_gemm_f16", a16.data_ptr(), M, K, K, sad.data_ptr(), b16.data_ptr(), N, K, sbd.data_ptr(),
+                  bd.data_ptr(), y.data_ptr(), N, cfg, _ext.stream())
+        assert torch.equal(y.cpu(), want), (M, N)
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 8, 1000), (64, 256, 8200), (130, 72, 4096), (260, 8, 30000), (2, 264, 130000)])
+def test_linear_dispatch_splits_bit_exact(dev, M, N, K):
+    """The dispatcher's own choice where few tiles meet a long K (2, 4 or 8 splits, a K
+    tail in the last one) and where x16 would not fit the no-allocation array (kernels
+    that add over k in order): exact products, so any order gives the same bits; the
+    no-allocation entry point gives them too."""
+    g = torch.Generator().manual_seed(12)
+    a, b = torch.randint(-1, 2, (M, K), generator=g), torch.randint(-1, 2, (N, K), generator=g)
+    xb, b16, ones = a.bfloat16().to(dev), b.half().to(dev), torch.ones(N, device=dev)
+    want = (a @ b.t()).double().bfloat16()
+    work, _ = linear_ws(M, K, N, -1, dev)
+    for name, tail in (("tbf16_linear", (work.data_ptr(), _ext.stream())), ("tbf16_linear_noalloc", (_ext.stream(),))):
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        _ext.call(name, xb.data_ptr(), M, K, K, b16.data_ptr(), N, K, ones.data_ptr(), None, y.data_ptr(), N, 15, 0, -1,
+                  *tail)
+        assert torch.equal(y.cpu(), want), name
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (200, 768, 2560), (300, 264, 3040)])
 def test_linear_split_k(dev, M, N, K):
     """K split over two blocks per tile (what tbf16_linear picks where the tiles leave

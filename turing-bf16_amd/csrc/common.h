@@ -204,6 +204,8 @@ __device__ __forceinline__ void wait_vmem_n() {
   static_assert(N >= 0 && N <= 63, "vmcnt immediate");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
+// s_waitcnt lgkmcnt(0): this wave's LDS reads and writes are done
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 // Workgroup barrier without the memory fence of __syncthreads (which waits for
 // every outstanding load, direct-to-LDS loads in flight included). The caller
 // waits for whatever the other waves must see (s_waitcnt) before it; the empty

@@ -59,6 +59,122 @@ __device__ __forceinline__ int swz(int row, int chunk) {
   else return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4);
 }
 
+// Epilogue of a wave's TM x TN sub-tile at (m0 + wm TM, n0 + wn TN):
+// (acc * sa[m]) * sb[n] + bias[n] -> bf16 straight from registers, or (part) the raw
+// fp32 sums. acc[i][j] is the 32x32 block of columns 32 i and rows 32 j; sa_l, sb_l
+// and bias_l are the block's factors in LDS.
+// Lane l holds columns 8 q + 4 (l / 32) .. + 3 of row l % 32 for q = 0..3.
+// Exchanges regroup them without LDS or a barrier: v_permlane32_swap pairs q = 2p
+// (kept by lanes < 32) with q = 2p + 1 (kept by lanes >= 32), so a lane holds 8
+// columns (16 bytes) of its row; v_permlane16_swap then pairs p = 0 with p = 1
+// between 16-lane rows (lane l: row l % 16, or + 16, columns 0 / 16 / 8 / 24 of
+// the 32-column block for l / 16 = 0 / 1 / 2 / 3); where FN is even, a DPP
+// row_ror:8 exchange between lanes l and l ^ 8 then pairs blocks i - 1 and i, so
+// each store instruction writes whole 128-byte rows (8 rows x 64 columns) and L2
+// writes back exactly y (WRITE_SIZE = y; 64-byte runs had read 1.38 x).
+template <int TM, int TN>
+__device__ __forceinline__ void store_tile(const floatx16 (&acc)[TN / 32][TM / 32], const float* sa_l, const float* sb_l,
+                                           const uint16_t* bias_l, int wm, int wn, int lane, int m0, int n0,
+                                           uint16_t* __restrict__ C, int64_t ldc, int M, int N, float* part) {
+  constexpr int FM = TM / 32, FN = TN / 32;
+  const int fr = lane & 31, fk = lane >> 5;
+  if (part) {
+    // raw fp32 sums: acc[i][j][4 q + r] is row wm TM + 32 j + fr, column
+    // wn TN + 32 i + 8 q + 4 fk + r of the tile (N is a multiple of 8)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      const int m = m0 + wm * TM + j * 32 + fr;
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int n = n0 + wn * TN + i * 32 + 8 * q + 4 * fk;
+          if (m < M && n < N)
+            *reinterpret_cast<float4*>(part + (int64_t)m * N + n) =
+                make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        }
+    }
+    return;
+  }
+  const int rl = lane & 15, cq = lane >> 4;
+  const int cl = ((cq & 1) << 4) | ((cq >> 1) << 3);
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int ml = wm * TM + j * 32 + fr;  // this lane's row before the exchanges
+    const float sa = sa_l[ml];
+    const int r0 = m0 + wm * TM + j * 32 + rl;  // rows stored by this lane
+    uint32_t xa[4], ya[4];  // block i - 1's x / y, held for the third exchange
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      uint32_t w[4][2];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int nl = wn * TN + i * 32 + 8 * q + 4 * fk;
+        const float4 sb = *reinterpret_cast<const float4*>(sb_l + nl);
+        const uint2 bw = *reinterpret_cast<const uint2*>(bias_l + nl);
+        const float y0 = fmaf(acc[i][j][4 * q + 0] * sa, sb.x, bf16_lo(bw.x));
+        const float y1 = fmaf(acc[i][j][4 * q + 1] * sa, sb.y, bf16_hi(bw.x));
+        const float y2 = fmaf(acc[i][j][4 * q + 2] * sa, sb.z, bf16_lo(bw.y));
+        const float y3 = fmaf(acc[i][j][4 * q + 3] * sa, sb.w, bf16_hi(bw.y));
+        w[q][0] = pack_bf16(y0, y1);
+        w[q][1] = pack_bf16(y2, y3);
+      }
+      // v[p]: 16 bytes of row l % 32, columns 16 p + 8 (l / 32) .. + 7
+      uint32_t v[2][4];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const auto d0 = __builtin_amdgcn_permlane32_swap(w[2 * p][0], w[2 * p + 1][0], false, false);
+        const auto d1 = __builtin_amdgcn_permlane32_swap(w[2 * p][1], w[2 * p + 1][1], false, false);
+        v[p][0] = d0[0]; v[p][1] = d1[0]; v[p][2] = d0[1]; v[p][3] = d1[1];
+      }
+      // x: rows 0..15 of the 32-row block, y: rows 16..31
+      uint32_t x[4], y[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const auto e = __builtin_amdgcn_permlane16_swap(v[0][d], v[1][d], false, false);
+        x[d] = e[0];
+        y[d] = e[1];
+      }
+      if constexpr (FN % 2 == 0) {
+        if (i % 2 == 0) {
+#pragma unroll
+          for (int d = 0; d < 4; ++d) { xa[d] = x[d]; ya[d] = y[d]; }
+          continue;
+        }
+        // third exchange: lane l and lane l ^ 8 (DPP row_ror:8) trade so that one
+        // store writes rows 0..7 (or 8..15) with blocks i - 1 and i side by side
+        const bool hi8 = (lane & 8) != 0;
+        uint32_t f[4], s2[4], g[4], s3[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const uint32_t tx = __builtin_amdgcn_mov_dpp((int)xa[d], 0x128, 0xF, 0xF, false);
+          const uint32_t tb = __builtin_amdgcn_mov_dpp((int)x[d], 0x128, 0xF, 0xF, false);
+          f[d] = hi8 ? tb : xa[d];
+          s2[d] = hi8 ? x[d] : tx;
+          const uint32_t uy = __builtin_amdgcn_mov_dpp((int)ya[d], 0x128, 0xF, 0xF, false);
+          const uint32_t ub = __builtin_amdgcn_mov_dpp((int)y[d], 0x128, 0xF, 0xF, false);
+          g[d] = hi8 ? ub : ya[d];
+          s3[d] = hi8 ? y[d] : uy;
+        }
+        const int rb = m0 + wm * TM + j * 32 + (lane & 7);
+        const int n = n0 + wn * TN + (i - 1 + (hi8 ? 1 : 0)) * 32 + cl;
+        if (n < N) {
+          if (rb < M) stg16(C + (int64_t)rb * ldc + n, make_uint4(f[0], f[1], f[2], f[3]));
+          if (rb + 8 < M) stg16(C + (int64_t)(rb + 8) * ldc + n, make_uint4(s2[0], s2[1], s2[2], s2[3]));
+          if (rb + 16 < M) stg16(C + (int64_t)(rb + 16) * ldc + n, make_uint4(g[0], g[1], g[2], g[3]));
+          if (rb + 24 < M) stg16(C + (int64_t)(rb + 24) * ldc + n, make_uint4(s3[0], s3[1], s3[2], s3[3]));
+        }
+      } else {
+        const int n = n0 + wn * TN + i * 32 + cl;
+        if (n < N) {
+          if (r0 < M) stg16(C + (int64_t)r0 * ldc + n, make_uint4(x[0], x[1], x[2], x[3]));
+          if (r0 + 16 < M) stg16(C + (int64_t)(r0 + 16) * ldc + n, make_uint4(y[0], y[1], y[2], y[3]));
+        }
+      }
+    }
+  }
+}
+
 template <int BM, int BN, int WM, int WN, int BK, int PF, int NS, bool A_BF16, bool KEVEN>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(const uint16_t* __restrict__ A, int64_t lda,
                                                            const int32_t* __restrict__ a_exp,
@@ -444,112 +560,475 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(const uint16_t* __res
     }
   }
 
-  // ---- epilogue: (acc * sa[m]) * sb[n] + bias[n] -> bf16 straight from registers ----
-  // Lane l holds columns 8 q + 4 (l / 32) .. + 3 of row l % 32 for q = 0..3.
-  // Exchanges regroup them without LDS or a barrier: v_permlane32_swap pairs q = 2p
-  // (kept by lanes < 32) with q = 2p + 1 (kept by lanes >= 32), so a lane holds 8
-  // columns (16 bytes) of its row; v_permlane16_swap then pairs p = 0 with p = 1
-  // between 16-lane rows (lane l: row l % 16, or + 16, columns 0 / 16 / 8 / 24 of
-  // the 32-column block for l / 16 = 0 / 1 / 2 / 3); where FN is even, a DPP
-  // row_ror:8 exchange between lanes l and l ^ 8 then pairs blocks i - 1 and i, so
-  // each store instruction writes whole 128-byte rows (8 rows x 64 columns) and L2
-  // writes back exactly y (WRITE_SIZE = y; 64-byte runs had read 1.38 x).
+  store_tile<BM / WM, BN / WN>(acc, sa_l, sb_l, bias_l, wm, wn, lane, m0, n0, C, ldc, M, N,
+                               part ? part + (int64_t)ks * M * N : nullptr);
+}
+
+// Epilogue of a wave's TM x TN sub-tile made of 16x16 MFMA blocks: acc[i][j] holds
+// columns 16 i and rows 16 j, lane l columns 4 (l / 16) .. + 3 of row l % 16. The same
+// fp32 arithmetic as store_tile; part: the raw fp32 sums, row stride ldp. v_permlane16_swap pairs column blocks 2 p and 2 p + 1
+// between 16-lane rows, so a lane holds 16 bytes of its row (columns 0 / 16 / 8 / 24 of
+// the 32-column pair for l / 16 = 0 / 1 / 2 / 3); with two pairs, a DPP row_ror:8
+// exchange between lanes l and l ^ 8 makes each store write whole 128-byte rows.
+template <int TM, int TN>
+__device__ __forceinline__ void store_tile16(const floatx4 (&acc)[TN / 16][TM / 16], const float* sa_l, const float* sb_l,
+                                             const uint16_t* bias_l, int wm, int wn, int lane, int m0, int n0,
+                                             uint16_t* __restrict__ C, int64_t ldc, int M, int N, float* part, int ldp) {
+  constexpr int FM = TM / 16, FN = TN / 16, NP = FN / 2;
+  static_assert(FN == 2 || FN == 4, "sub-tile columns");
+  const int fr = lane & 15, fk = lane >> 4;
   if (part) {
-    // raw fp32 sums: acc[i][j][4 q + r] is row wm TM + 32 j + fr, column
-    // wn TN + 32 i + 8 q + 4 fk + r of the tile (N is a multiple of 8)
-    float* const pk = part + (int64_t)ks * M * N;
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
-      const int m = m0 + wm * TM + j * 32 + fr;
+      const int m = m0 + wm * TM + j * 16 + fr;
 #pragma unroll
-      for (int i = 0; i < FN; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wn * TN + i * 32 + 8 * q + 4 * fk;
-          if (m < M && n < N)
-            *reinterpret_cast<float4*>(pk + (int64_t)m * N + n) =
-                make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-        }
+      for (int i = 0; i < FN; ++i) {
+        const int n = n0 + wn * TN + i * 16 + 4 * fk;
+        if (m < M && n < N)
+          *reinterpret_cast<float4*>(part + (int64_t)m * ldp + n) =
+              make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+      }
     }
     return;
   }
-  const int rl = lane & 15, cq = lane >> 4;
-  const int cl = ((cq & 1) << 4) | ((cq >> 1) << 3);
+  const int cl = ((fk & 1) << 4) | ((fk >> 1) << 3);
+  const bool hi8 = (lane & 8) != 0;
 #pragma unroll
   for (int j = 0; j < FM; ++j) {
-    const int ml = wm * TM + j * 32 + fr;  // this lane's row before the exchanges
-    const float sa = sa_l[ml];
-    const int r0 = m0 + wm * TM + j * 32 + rl;  // rows stored by this lane
-    uint32_t xa[4], ya[4];  // block i - 1's x / y, held for the third exchange
+    const float sa = sa_l[wm * TM + j * 16 + fr];
+    uint32_t v[NP][4];
 #pragma unroll
-    for (int i = 0; i < FN; ++i) {
-      uint32_t w[4][2];
+    for (int p = 0; p < NP; ++p) {
+      uint32_t w[2][2];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int nl = wn * TN + i * 32 + 8 * q + 4 * fk;
+      for (int i = 0; i < 2; ++i) {
+        const int nl = wn * TN + (2 * p + i) * 16 + 4 * fk;
         const float4 sb = *reinterpret_cast<const float4*>(sb_l + nl);
         const uint2 bw = *reinterpret_cast<const uint2*>(bias_l + nl);
-        const float y0 = fmaf(acc[i][j][4 * q + 0] * sa, sb.x, bf16_lo(bw.x));
-        const float y1 = fmaf(acc[i][j][4 * q + 1] * sa, sb.y, bf16_hi(bw.x));
-        const float y2 = fmaf(acc[i][j][4 * q + 2] * sa, sb.z, bf16_lo(bw.y));
-        const float y3 = fmaf(acc[i][j][4 * q + 3] * sa, sb.w, bf16_hi(bw.y));
-        w[q][0] = pack_bf16(y0, y1);
-        w[q][1] = pack_bf16(y2, y3);
+        const floatx4 c = acc[2 * p + i][j];
+        w[i][0] = pack_bf16(fmaf(c[0] * sa, sb.x, bf16_lo(bw.x)), fmaf(c[1] * sa, sb.y, bf16_hi(bw.x)));
+        w[i][1] = pack_bf16(fmaf(c[2] * sa, sb.z, bf16_lo(bw.y)), fmaf(c[3] * sa, sb.w, bf16_hi(bw.y)));
       }
-      // v[p]: 16 bytes of row l % 32, columns 16 p + 8 (l / 32) .. + 7
-      uint32_t v[2][4];
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const auto d0 = __builtin_amdgcn_permlane32_swap(w[2 * p][0], w[2 * p + 1][0], false, false);
-        const auto d1 = __builtin_amdgcn_permlane32_swap(w[2 * p][1], w[2 * p + 1][1], false, false);
-        v[p][0] = d0[0]; v[p][1] = d1[0]; v[p][2] = d0[1]; v[p][3] = d1[1];
-      }
-      // x: rows 0..15 of the 32-row block, y: rows 16..31
-      uint32_t x[4], y[4];
+      const auto d0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+      const auto d1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+      v[p][0] = d0[0]; v[p][1] = d1[0]; v[p][2] = d0[1]; v[p][3] = d1[1];
+    }
+    const int row0 = m0 + wm * TM + j * 16, col0 = n0 + wn * TN + cl;
+    if constexpr (NP == 2) {
+      uint32_t f[4], g[4];
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        const auto e = __builtin_amdgcn_permlane16_swap(v[0][d], v[1][d], false, false);
-        x[d] = e[0];
-        y[d] = e[1];
+        const uint32_t t0 = __builtin_amdgcn_mov_dpp((int)v[0][d], 0x128, 0xF, 0xF, false);
+        const uint32_t t1 = __builtin_amdgcn_mov_dpp((int)v[1][d], 0x128, 0xF, 0xF, false);
+        f[d] = hi8 ? t1 : v[0][d];
+        g[d] = hi8 ? v[1][d] : t0;
       }
-      if constexpr (FN % 2 == 0) {
-        if (i % 2 == 0) {
-#pragma unroll
-          for (int d = 0; d < 4; ++d) { xa[d] = x[d]; ya[d] = y[d]; }
-          continue;
-        }
-        // third exchange: lane l and lane l ^ 8 (DPP row_ror:8) trade so that one
-        // store writes rows 0..7 (or 8..15) with blocks i - 1 and i side by side
-        const bool hi8 = (lane & 8) != 0;
-        uint32_t f[4], s2[4], g[4], s3[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          const uint32_t tx = __builtin_amdgcn_mov_dpp((int)xa[d], 0x128, 0xF, 0xF, false);
-          const uint32_t tb = __builtin_amdgcn_mov_dpp((int)x[d], 0x128, 0xF, 0xF, false);
-          f[d] = hi8 ? tb : xa[d];
-          s2[d] = hi8 ? x[d] : tx;
-          const uint32_t uy = __builtin_amdgcn_mov_dpp((int)ya[d], 0x128, 0xF, 0xF, false);
-          const uint32_t ub = __builtin_amdgcn_mov_dpp((int)y[d], 0x128, 0xF, 0xF, false);
-          g[d] = hi8 ? ub : ya[d];
-          s3[d] = hi8 ? y[d] : uy;
-        }
-        const int rb = m0 + wm * TM + j * 32 + (lane & 7);
-        const int n = n0 + wn * TN + (i - 1 + (hi8 ? 1 : 0)) * 32 + cl;
-        if (n < N) {
-          if (rb < M) stg16(C + (int64_t)rb * ldc + n, make_uint4(f[0], f[1], f[2], f[3]));
-          if (rb + 8 < M) stg16(C + (int64_t)(rb + 8) * ldc + n, make_uint4(s2[0], s2[1], s2[2], s2[3]));
-          if (rb + 16 < M) stg16(C + (int64_t)(rb + 16) * ldc + n, make_uint4(g[0], g[1], g[2], g[3]));
-          if (rb + 24 < M) stg16(C + (int64_t)(rb + 24) * ldc + n, make_uint4(s3[0], s3[1], s3[2], s3[3]));
-        }
-      } else {
-        const int n = n0 + wn * TN + i * 32 + cl;
-        if (n < N) {
-          if (r0 < M) stg16(C + (int64_t)r0 * ldc + n, make_uint4(x[0], x[1], x[2], x[3]));
-          if (r0 + 16 < M) stg16(C + (int64_t)(r0 + 16) * ldc + n, make_uint4(y[0], y[1], y[2], y[3]));
-        }
+      const int m = row0 + (lane & 7), n = col0 + (hi8 ? 32 : 0);
+      if (n < N) {
+        if (m < M) stg16(C + (int64_t)m * ldc + n, make_uint4(f[0], f[1], f[2], f[3]));
+        if (m + 8 < M) stg16(C + (int64_t)(m + 8) * ldc + n, make_uint4(g[0], g[1], g[2], g[3]));
       }
+    } else {
+      if (row0 + fr < M && col0 < N)
+        stg16(C + (int64_t)(row0 + fr) * ldc + col0, make_uint4(v[0][0], v[0][1], v[0][2], v[0][3]));
     }
   }
+}
+
+// Ping-pong GEMM on fp16 operands: 8 waves in two groups of four, one wave of each
+// group per SIMD (waves w and w + 4 share a SIMD), half a phase apart: while one
+// group's MFMAs run, the other reads its next fragments from LDS and issues direct
+// global -> LDS loads; a bare barrier ends each such interval. Group g owns rows
+// [BM / 2 g, + BM / 2) of the tile, wave w % 4 of it BN / 4 columns. k tile 64.
+//  - MFMA 16x16x32: under this kernel the chip's clock is set by power, and the 16x16
+//    form costs less of it than 32x32x16 (4096^3: 1.92 GHz and 101.8 us against 1.63
+//    GHz and 113.4 us with the same schedule, same output bits).
+//  - a k tile is staged as four half tiles, each its own __shared__ object: A half h
+//    holds rows RA h .. + RA of each group's 2 RA, B half h columns CB h .. + CB of each
+//    wave's 2 CB. S stages in a ring (tile kt in stage kt % S).
+//  - a k tile is two phases, each one half of A against both of B (256x256: 32 MFMAs,
+//    512 cycles). The B half 0 of a tile is read one phase early, which evens out
+//    the LDS reads of the phases:
+//      phase  MFMAs     reads                    loads
+//      0      A0 B0 B1  A0, B1                   A1 of tile kt + S - 1, B0 of kt + S
+//      1      A1 B0 B1  A1, B0 of tile kt + 1    A0, B1 of tile kt + S
+//    A wave waits for its fragment reads (lgkmcnt 0) before the barrier that starts
+//    its MFMAs; the other group's reads of the same phase are complete one barrier
+//    later, so the next phase's loads may overwrite what this phase read.
+//  - a half tile is loaded 2 S - 1 phases before it is read. Before each phase's first
+//    barrier a wave waits until only the last 2 S - 2 phases' loads are left: what the
+//    next phase reads has then landed for every wave of both groups. S = 2 is all
+//    that fits at 256x256 and 192x256 (their phases are long enough to cover a load);
+//    the smaller tiles' shorter phases need the deeper ring.
+// Loads of tiles past the last go to a resource of length 0 (no memory traffic, zeros
+// nobody reads). The fp32 additions run over k in ascending order.
+// HA, FB: 16-row and 16-column blocks per wave and half (BM = 64 HA, BN = 128 FB).
+// part / kt_per: split K, as gemm_kernel.
+template <int HA, int FB, int S, bool KEVEN>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void pingpong_kernel(
+    const uint16_t* __restrict__ A, int64_t lda, const float* __restrict__ a_sinv, const uint16_t* __restrict__ B,
+    int64_t ldb, const float* __restrict__ b_sinv, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C,
+    int64_t ldc, int M, int N, int K_all, float* __restrict__ part, int kt_per) {
+  constexpr int BM = 64 * HA, BN = 128 * FB, RA = 16 * HA, CB = 16 * FB;
+  constexpr int AB = 4 * HA, BB = 8 * FB;  // 1 KB blocks (8 rows of 128 bytes) of a half tile
+  constexpr int AL = (AB + 7) / 8, BL = BB / 8;
+  constexpr int INFLIGHT = (S - 1) * (HA + 2 * FB);  // a wave's loads of 2 S - 2 phases
+  static_assert(HA >= 2 && HA <= 4 && (FB == 1 || FB == 2) && S >= 2 && S <= 4, "tile");
+  __shared__ __align__(1024) uint8_t a00[AB * 1024], a01[AB * 1024], a10[AB * 1024], a11[AB * 1024];  // [stage][half]
+  __shared__ __align__(1024) uint8_t b00[BB * 1024], b01[BB * 1024], b10[BB * 1024], b11[BB * 1024];
+  constexpr int A2 = S > 2 ? AB * 1024 : 16, B2 = S > 2 ? BB * 1024 : 16, A3 = S > 3 ? AB * 1024 : 16,
+                B3 = S > 3 ? BB * 1024 : 16;
+  __shared__ __align__(1024) uint8_t a20[A2], a21[A2], a30[A3], a31[A3], b20[B2], b21[B2], b30[B3], b31[B3];
+  uint8_t* const sa0[4] = {a00, a10, a20, a30};
+  uint8_t* const sa1[4] = {a01, a11, a21, a31};
+  uint8_t* const sb0[4] = {b00, b10, b20, b30};
+  uint8_t* const sb1[4] = {b01, b11, b21, b31};
+  __shared__ __align__(16) float sa_l[BM], sb_l[BN];
+  __shared__ __align__(16) uint16_t bias_l[BN];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;  // wm: the group
+
+  // tile assignment: XCD-contiguous ranges, then grouped raster (as gemm_kernel)
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  int bid = blockIdx.x;
+  const int nblk = gridDim.x;
+  if ((nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);
+  constexpr int GM = 8;
+  const int group = bid / (GM * tiles_n), first = group * GM, gsize = min(tiles_m - first, GM);
+  const int within = bid % (GM * tiles_n);
+  const int m0 = (first + within % gsize) * BM;
+  const int n0 = (within / gsize) * BN;
+  const int ks = part ? (int)blockIdx.y : 0;
+  const int kbase = ks * kt_per * 64;
+  const int K = part ? min(K_all - kbase, kt_per * 64) : K_all;
+
+  // the epilogue's factors, one a thread, loaded ahead of the direct loads (rows past M
+  // and columns past N take the last one's and are not stored)
+  const int fc = tid - 256;
+  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, N - 1)];
+  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), N - 1)] : (uint16_t)0;
+
+  // direct loads: lane l of the load of 1 KB block b lands at row 8 b + l / 8 of the
+  // half tile, physical chunk l % 8, so it fetches the logical chunk `chunk` (the XOR
+  // swizzle on the source side; a wave's blocks all have its own parity). Wave w loads
+  // blocks w and w + 8; of 12 blocks (HA = 3) the last four are waves 0-3's in half 0
+  // and waves 4-7's in half 1, so that every wave has the same loads in two phases.
+  const int l8 = lane >> 3, chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
+  int aoff[2][AL], boff[2][BL];  // [half][block]
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int i = 0; i < AL; ++i) {
+      const int r = 8 * (i == 0 ? wave : AB == 12 ? 8 + (wave & 3) : 8 + wave) + l8;
+      aoff[h][i] = ((r / RA * 2 * RA + RA * h + r % RA) * (int)lda + chunk * 8) * 2;
+    }
+#pragma unroll
+    for (int i = 0; i < BL; ++i) {
+      const int r = 8 * (wave + 8 * i) + l8;
+      boff[h][i] = ((r / CB * 2 * CB + CB * h + r % CB) * (int)ldb + chunk * 8) * 2;
+    }
+  }
+  const BufRes ares =
+      make_res(A + (int64_t)m0 * lda + kbase, min<int64_t>((int64_t)(M - m0) * lda * 2 - kbase * 2, 0x7fffffff));
+  const BufRes bres =
+      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(N - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
+  const int KT = (K + 63) / 64;
+  auto aload = [&](int h, uint8_t* half, int kt) {
+    const BufRes rt{ares.lo, ares.hi, kt < KT ? ares.bytes : 0};
+    const uint32_t base = lds_addr(half);
+    const bool kok = KEVEN || kt * 64 + chunk * 8 < K;  // a k tail reads zeros
+    buf_load16_lds(rt, base + wave * 1024, kok ? aoff[h][0] : (int)0x80000000, kt * 128);
+    if constexpr (AB == 12) {
+      if (wm == h) buf_load16_lds(rt, base + (8 + wn) * 1024, kok ? aoff[h][AL - 1] : (int)0x80000000, kt * 128);
+    } else if constexpr (AB == 16) {
+      buf_load16_lds(rt, base + (8 + wave) * 1024, kok ? aoff[h][AL - 1] : (int)0x80000000, kt * 128);
+    }
+  };
+  auto bload = [&](int h, uint8_t* half, int kt) {
+    const BufRes rt{bres.lo, bres.hi, kt < KT ? bres.bytes : 0};
+    const uint32_t base = lds_addr(half);
+    const bool kok = KEVEN || kt * 64 + chunk * 8 < K;
+#pragma unroll
+    for (int i = 0; i < BL; ++i)
+      buf_load16_lds(rt, base + (wave + 8 * i) * 1024, kok ? boff[h][i] : (int)0x80000000, kt * 128);
+  };
+
+  floatx4 acc[2 * FB][2 * HA];  // [16 columns][16 rows]
+#pragma unroll
+  for (int i = 0; i < 2 * FB; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * HA; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+
+  const int fr = lane & 15, fk = lane >> 4;
+  half8 fa[2][HA], fb0[2][2][FB], fb1[2][FB];  // [k step][block]; B0 of the current and the next tile
+  auto areads = [&](const uint8_t* half) {
+#pragma unroll
+    for (int j = 0; j < HA; ++j)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        fa[s][j] = *reinterpret_cast<const half8*>(half + swz<64>(wm * RA + j * 16 + fr, 4 * s + fk));
+  };
+  auto breads = [&](half8(&f)[2][FB], const uint8_t* half) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < FB; ++i)
+        f[s][i] = *reinterpret_cast<const half8*>(half + swz<64>(wn * CB + i * 16 + fr, 4 * s + fk));
+  };
+  // a phase's MFMAs between its two barriers
+  auto mma = [&](const half8(&b0)[2][FB], int ha) {
+    wait_vmem_n<INFLIGHT>();
+    wait_lds();
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_no_fence();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int j = 0; j < HA; ++j)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int i = 0; i < 2 * FB; ++i)
+          acc[i][HA * ha + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(i < FB ? b0[s][i] : fb1[s][i - FB], fa[s][j],
+                                                                       acc[i][HA * ha + j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_no_fence();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // prologue: tiles 0 .. S - 2 whole, three half tiles of tile S - 1
+#pragma unroll
+  for (int t = 0; t < S; ++t) {
+    bload(0, sb0[t], t);
+    aload(0, sa0[t], t);
+    bload(1, sb1[t], t);
+    if (t + 1 < S) aload(1, sa1[t], t);
+  }
+  if (fc < 0) {
+    if (tid < BM) sa_l[tid] = fsc;
+  } else if (fc < BN) {
+    sb_l[fc] = fsc;
+    bias_l[fc] = fbias;
+  }
+  wait_vmem_n<INFLIGHT>();
+  wait_lds();
+  __builtin_amdgcn_sched_barrier(0);
+  barrier_no_fence();
+  __builtin_amdgcn_sched_barrier(0);
+  breads(fb0[0], sb0[0]);
+  wait_lds();
+  __builtin_amdgcn_sched_barrier(0);
+  barrier_no_fence();  // every wave has read B0 of tile 0: phase 0 loads over it
+  if (wm == 1) barrier_no_fence();
+  __builtin_amdgcn_sched_barrier(0);
+
+  // tile kt in stage u % S; fb0[u % 2] holds its B0 fragments, fb0[(u + 1) % 2] takes tile kt + 1's
+  constexpr int UN = S == 3 ? 6 : S;
+  for (int kt0 = 0; kt0 < KT; kt0 += UN) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int kt = kt0 + u, c = u % S;
+      if (u > 0 && kt >= KT) break;
+      areads(sa0[c]);
+      breads(fb1, sb1[c]);
+      aload(1, sa1[(c + S - 1) % S], kt + S - 1);
+      bload(0, sb0[c], kt + S);
+      mma(fb0[u & 1], 0);
+      areads(sa1[c]);
+      breads(fb0[(u + 1) & 1], sb0[(c + 1) % S]);
+      aload(0, sa0[c], kt + S);
+      bload(1, sb1[c], kt + S);
+      mma(fb0[u & 1], 1);
+    }
+  }
+  if (wm == 0) barrier_no_fence();
+  wait_vmem_n<0>();  // the loads of tiles past the last have ended before the block's LDS is given back
+  store_tile16<2 * RA, 2 * CB>(acc, sa_l, sb_l, bias_l, wm, wn, lane, m0, n0, C, ldc, M, N,
+                               part ? part + (int64_t)ks * M * N : nullptr, N);
+}
+
+// Ping-pong GEMM on fp16 operands for tiles too small for pingpong_kernel's phases:
+// both groups of four waves (2 x 2 sub-tiles of 16 RM x 16 RN) cover the whole BM x BN
+// tile, group 0 with the even k tiles, group 1 with the odd ones, and their sums meet
+// in LDS at the end. Interval t (between two bare barriers): group t % 2 reads its
+// fragments of tile t while the other group multiplies tile t - 1; every wave issues
+// its share of the direct loads of tile t + S - 1 into the stage of tile t - 1, whose
+// reads ended before the interval began, and before the interval's barrier waits until
+// tile t + 1 has landed (the loads of S - 2 later tiles are left in flight).
+//  - a wave's sub-tile is twice as wide as with eight waves side by side: a third
+//    less LDS traffic per product, and an interval holds a whole k tile of one group
+//    (128x128: 32 MFMAs, 512 cycles) instead of a quarter.
+//  - an odd number of k tiles is padded with one of zeros (a resource of length 0).
+// The two groups' fp32 sums are added even + odd: another order than k ascending,
+// the same for every launch. part / kt_per: split K, as gemm_kernel. R <= BN: columns
+// per block (a multiple of 8); below BN the weights of a single row of tiles are
+// spread over every CU, the rest of the tile is zeros.
+template <int RM, int RN, int S, bool KEVEN>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void ksplit_kernel(
+    const uint16_t* __restrict__ A, int64_t lda, const float* __restrict__ a_sinv, const uint16_t* __restrict__ B,
+    int64_t ldb, const float* __restrict__ b_sinv, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C,
+    int64_t ldc, int M, int N_all, int K_all, float* __restrict__ part, int kt_per, int R) {
+  constexpr int BM = 32 * RM, BN = 32 * RN, TM = 16 * RM, TN = 16 * RN;
+  constexpr int STG = (BM + BN) * 128, NL = (BM + BN) / 64, AL = BM / 64;  // loads per wave and tile; the first AL are A's
+  constexpr int XB = RM / 2 * RN * 16 * 64;  // bytes of the half sub-tile a wave hands over
+  static_assert(RM % 2 == 0 && (RN == 2 || RN == 4) && S >= 3 && S <= 9 && 3 * (STG / XB) >= 8 && NL * 64 == BM + BN, "tile");
+  __shared__ __align__(1024) uint8_t st0[STG], st1[STG], st2[STG];
+  __shared__ __align__(1024) uint8_t st3[S > 3 ? STG : 16], st4[S > 4 ? STG : 16], st5[S > 5 ? STG : 16];
+  __shared__ __align__(1024) uint8_t st6[S > 6 ? STG : 16], st7[S > 7 ? STG : 16], st8[S > 8 ? STG : 16];
+  __shared__ __align__(16) float sa_l[BM], sb_l[BN];
+  __shared__ __align__(16) uint16_t bias_l[BN];
+  uint8_t* const stages[9] = {st0, st1, st2, st3, st4, st5, st6, st7, st8};
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave >> 1) & 1, wn = wave & 1;
+
+  // tile assignment: XCD-contiguous ranges, then grouped raster (as gemm_kernel)
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N_all + R - 1) / R;
+  int bid = blockIdx.x;
+  const int nblk = gridDim.x;
+  if ((nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);
+  constexpr int GM = 8;
+  const int group = bid / (GM * tiles_n), first = group * GM, gsize = min(tiles_m - first, GM);
+  const int within = bid % (GM * tiles_n);
+  const int m0 = (first + within % gsize) * BM;
+  const int n0 = (within / gsize) * R, N = min(N_all, n0 + R);
+  const int ks = part ? (int)blockIdx.y : 0;
+  const int kbase = ks * kt_per * 64;
+  const int K = part ? min(K_all - kbase, kt_per * 64) : K_all;
+
+  // the epilogue's factors (see pingpong_kernel)
+  const int fc = tid - 256;
+  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, N - 1)];
+  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), N - 1)] : (uint16_t)0;
+
+  // direct loads: 1 KB block wave + 8 i of the stage (rows of A, then of B)
+  const int chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
+  int off[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int r = 8 * (wave + 8 * (i < AL ? i : i - AL)) + (lane >> 3);
+    off[i] = (r * (int)(i < AL ? lda : ldb) + chunk * 8) * 2;
+  }
+  const BufRes ares =
+      make_res(A + (int64_t)m0 * lda + kbase, min<int64_t>((int64_t)(M - m0) * lda * 2 - kbase * 2, 0x7fffffff));
+  const BufRes bres =
+      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(N - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
+  const int KT = (K + 63) / 64;
+  auto load = [&](uint8_t* stage, int kt) {
+    const BufRes ra{ares.lo, ares.hi, kt < KT ? ares.bytes : 0}, rb{bres.lo, bres.hi, kt < KT ? bres.bytes : 0};
+    const uint32_t base = lds_addr(stage) + wave * 1024;
+    const bool kok = KEVEN || kt * 64 + chunk * 8 < K;  // a k tail reads zeros
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      buf_load16_lds(i < AL ? ra : rb, base + i * 8192, kok ? off[i] : (int)0x80000000, kt * 128);
+  };
+
+  floatx4 acc[RN][RM];  // [16 columns][16 rows]
+#pragma unroll
+  for (int i = 0; i < RN; ++i)
+#pragma unroll
+    for (int j = 0; j < RM; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+  const int fr = lane & 15, fk = lane >> 4;
+  half8 fa[2][RM], fb[2][RN];
+  auto settle = [&]() {  // the end of an interval
+    wait_vmem_n<NL*(S - 2)>();
+    wait_lds();
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_no_fence();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+#pragma unroll
+  for (int t = 0; t < S - 1; ++t) load(stages[t], t);
+  if (fc < 0) {
+    if (tid < BM) sa_l[tid] = fsc;
+  } else if (fc < BN) {
+    sb_l[fc] = fsc;
+    bias_l[fc] = fbias;
+  }
+  settle();
+
+  const int J = (KT + 1) / 2;  // k tiles per group
+  auto run = [&](auto g_c) {
+    constexpr int g = decltype(g_c)::value;
+    if constexpr (g == 1) {
+      load(stages[S - 1], S - 1);
+      settle();
+    }
+    constexpr int UN = S % 2 ? S : S / 2;
+    for (int j0 = 0; j0 < J; j0 += UN) {
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        if (u > 0 && j0 + u >= J) break;
+        const int kt = 2 * (j0 + u) + g;
+        const int c = (2 * u + g) % S;
+        const uint8_t* stage = stages[c];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+          for (int i = 0; i < RN; ++i)
+            fb[s][i] = *reinterpret_cast<const half8*>(stage + swz<64>(BM + wn * TN + i * 16 + fr, 4 * s + fk));
+#pragma unroll
+          for (int j = 0; j < RM; ++j)
+            fa[s][j] = *reinterpret_cast<const half8*>(stage + swz<64>(wm * TM + j * 16 + fr, 4 * s + fk));
+        }
+        load(stages[(c + S - 1) % S], kt + S - 1);
+        settle();
+        load(stages[c], kt + S);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int j = 0; j < RM; ++j)
+#pragma unroll
+            for (int i = 0; i < RN; ++i)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[s][i], fa[s][j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        settle();
+      }
+    }
+    if constexpr (g == 0) settle();
+    // hand the other group half of the rows' sums, take its sums of the rest
+    wait_vmem_n<0>();
+    __syncthreads();
+    constexpr int H = RM / 2;
+    constexpr int PER = STG / XB;  // waves' regions per stage
+    auto region = [&](int w) {
+      return reinterpret_cast<float4*>((w < PER ? st0 : w < 2 * PER ? st1 : st2) + (w % PER) * XB) + lane;
+    };
+    float4* const out = region(wave);
+    const float4* const in = region(wave ^ 4);
+#pragma unroll
+    for (int i = 0; i < RN; ++i)
+#pragma unroll
+      for (int j = 0; j < H; ++j) {
+        const floatx4 v = acc[i][g ? j : H + j];
+        out[(i * H + j) * 64] = make_float4(v[0], v[1], v[2], v[3]);
+      }
+    __syncthreads();
+    floatx4 sum[RN][H];
+#pragma unroll
+    for (int i = 0; i < RN; ++i)
+#pragma unroll
+      for (int j = 0; j < H; ++j) {
+        const float4 v = in[(i * H + j) * 64];
+        const floatx4 o = acc[i][g ? H + j : j];
+        sum[i][j][0] = o[0] + v.x;  // even + odd (commutative: the same bits in either group)
+        sum[i][j][1] = o[1] + v.y;
+        sum[i][j][2] = o[2] + v.z;
+        sum[i][j][3] = o[3] + v.w;
+      }
+    // rows wm TM + g TM / 2 of the tile: sub-tile row 2 wm + g of height TM / 2
+    store_tile16<TM / 2, TN>(sum, sa_l, sb_l, bias_l, 2 * wm + g, wn, lane, m0, n0, C, ldc, M, N,
+                             part ? part + (int64_t)ks * M * N_all : nullptr, N_all);
+  };
+  if (wave < 4) run(std::integral_constant<int, 0>{});
+  else run(std::integral_constant<int, 1>{});
 }
 
 // Split-K reduction and epilogue: y = bf16((p_0 + p_1 + ...) * sa[m] * sb[n] +
@@ -967,6 +1446,8 @@ struct TileCfg {
   int bm, bn, bk;  // skinny configurations: bm = the largest M they take
   bool skinny;
   bool stream;  // fp16 a only (stream_kernel); bm = rows of a per block
+  bool pingpong;  // fp16 a only (pingpong_kernel, ksplit_kernel)
+  bool ksplit;    // ksplit_kernel: two groups of waves take alternate k tiles
 };
 // Tiled configurations (block tile, waves, k tile, register sets in flight, LDS stages):
 // 0: 256x256, 8 waves of 64x128 (2 per SIMD), k 32, 3 sets, 3 stages, grouped MFMA schedule
@@ -992,13 +1473,22 @@ struct TileCfg {
 // 18: 256 rows, 3 stages
 // Two-stage k 64 loop as 9: 19: 192x256, 8 waves of 96x64 (a tile count that fills
 // the CUs where 256-row tiles leave some idle, e.g. M = 6144: 32 rows of tiles)
+// Ping-pong on fp16 a: 20: 256x256, 21: 192x256 (2 stages), 22: 128x256, 23: 256x128,
+// 24: 128x128 (3 stages). Ping-pong with alternate k tiles, fp16 a: 25: 256x128,
+// 26: 192x128 (3 stages), 27: 128x128 (4), 28: 128x64, 29: 64x128, 30: 64x64 (6)
 constexpr TileCfg kCfgs[] = {{256, 256, 32}, {128, 128, 64}, {64, 64, 64},       {128, 128, 64},    {256, 256, 32},
                              {32, 32, 64, true}, {32, 32, 64, true}, {64, 32, 64, true}, {64, 64, 64, true},
                              {256, 256, 64}, {256, 128, 64}, {256, 64, 64}, {128, 64, 64}, {32, 64, 64, true},
                              {64, 64, 64, true}, {32, 64, 64, false, true}, {64, 64, 64, false, true},
                              {128, 64, 64, false, true}, {256, 64, 64, false, true},
-                             {192, 256, 64}};
-constexpr int kNumCfgs = 20;
+                             {192, 256, 64},
+                             {256, 256, 64, false, false, true}, {192, 256, 64, false, false, true},
+                             {128, 256, 64, false, false, true}, {256, 128, 64, false, false, true},
+                             {128, 128, 64, false, false, true},
+                             {256, 128, 64, false, false, true, true}, {192, 128, 64, false, false, true, true},
+                             {128, 128, 64, false, false, true, true}, {128, 64, 64, false, false, true, true},
+                             {64, 128, 64, false, false, true, true}, {64, 64, 64, false, false, true, true}};
+constexpr int kNumCfgs = 31;
 
 // Compute units of the current device (cached per device).
 int64_t num_cus() {
@@ -1013,37 +1503,30 @@ int64_t num_cus() {
   return cache[dev];
 }
 
-// Configuration choice, fitted to measurements on MI355X (256 CUs). f16a: the caller
-// can supply fp16 a (the decode configurations need it). Otherwise, for M <= 64
-// with enough b rows for 160 blocks, the 64-row skinny block (8 waves splitting
-// K, 3 chunks in flight: 17.6 -> 16.4 us at M = 16, K = 2560, N = 10240) up to M = 32 and
-// the LDS-staged 64x64 tile above (every skinny block re-reads all of a, which
-// costs more than the weights from M ~ 40 on). Otherwise the tile that maximises
-// eff x (blocks / whole rounds of 256 blocks) x (M / M rounded up to the tile):
-// larger tiles run faster per CU (eff), but a partial last round of blocks or a
-// mostly empty row of tiles wastes CUs.
-// Split K in two (tile configurations, workspace entry points): where a tile
-// configuration leaves at least half the CUs without a tile, K >= 2048 and the
-// fp32 partial sums take at most kSplitPartBytes, two blocks per tile each sum half
-// of K into the workspace and a reduction applies the epilogue (256x4096x4096:
-// 128 tiles of 128x64 -> 256 blocks). The output differs from the unsplit one only
-// by the order of the fp32 additions (exact for integer-valued products).
+// Split K in two for a pinned tile configuration that converts x in the GEMM or takes
+// x16 (workspace entry points): where it leaves at least half the CUs without a tile,
+// K >= 2048 and the fp32 partial sums take at most kSplitPartBytes, two blocks per
+// tile each sum half of K into the workspace and a reduction applies the epilogue.
+// The output differs from the unsplit one only by the order of the fp32 additions
+// (exact for integer-valued products).
 constexpr size_t kSplitPartBytes = (size_t)8 << 20;
 int pick_split(int cfg, int64_t M, int64_t N, int64_t K) {
-  if (cfg < 0 || cfg >= kNumCfgs || kCfgs[cfg].skinny || kCfgs[cfg].stream || K < 2048) return 1;
+  if (cfg < 0 || cfg >= kNumCfgs || kCfgs[cfg].skinny || kCfgs[cfg].stream || kCfgs[cfg].pingpong || K < 2048) return 1;
   const int64_t tiles = cdiv(M, kCfgs[cfg].bm) * cdiv(N, kCfgs[cfg].bn);
   if (2 * tiles > num_cus() || (size_t)2 * (size_t)M * (size_t)N * 4 > kSplitPartBytes) return 1;
   return 2;
 }
 
-// K > 0: the caller can split K (pick_split), which the score accounts for.
-int pick_cfg(int64_t M, int64_t N, bool f16a, int64_t K = 0) {
-  // decode on fp16 a (a16 given, or tbf16_linear's workspace copy): the direct-to-LDS
-  // ring for M <= 128 once N fills every CU with at least 32 b rows (M = 16 / 64 /
-  // 128 at K = 2560, N = 10240: 13.3 / 18.2 / 23.0 us against 13.6 / 24.1 / 26.9 for
-  // the kernels below; at M = 255 the two tie, and the 256-row tiles skip the copy)
-  if (f16a && M <= 128 && N >= 32 * num_cus()) return M <= 32 ? 15 : M <= 64 ? 16 : 17;
-  if (M <= 64) {
+// Tile configuration that converts bf16 a inside the GEMM (tbf16_linear_exps, and the
+// no-allocation entry point where x16 does not fit its array). For M <= 64 with enough
+// b rows for 160 blocks, the 64-row skinny block up to M = 32 and the LDS-staged 64x64
+// tile above (every skinny block re-reads all of a). Otherwise the tile that maximises
+// eff x (blocks / whole rounds of CU-count blocks) x (M / M rounded up to the tile):
+// larger tiles run faster per CU (eff), but a partial last round of blocks or a mostly
+// empty row of tiles wastes CUs. tiles_only: no skinny blocks (which add over k in
+// another order).
+int pick_fused(int64_t M, int64_t N, bool tiles_only) {
+  if (M <= 64 && !tiles_only) {
     if (cdiv(N, 64) >= 160) return M <= 32 ? 13 : 2;
     return M <= 32 ? 6 : 7;
   }
@@ -1057,19 +1540,81 @@ int pick_cfg(int64_t M, int64_t N, bool f16a, int64_t K = 0) {
   float best_score = -1.f;
   for (int i = 0; i < ncand; ++i) {
     const TileCfg& t = kCfgs[cand[i]];
-    const int s = K > 0 ? pick_split(cand[i], M, N, K) : 1;
-    const int64_t mt = cdiv(M, t.bm), tiles = mt * cdiv(N, t.bn) * s;
+    const int64_t mt = cdiv(M, t.bm), tiles = mt * cdiv(N, t.bn);
     const float util = (float)tiles / (float)(cdiv(tiles, kCUs) * kCUs);
     const float mutil = (float)M / (float)(mt * t.bm);
-    // the partial sums' round trip and the reduction launch: 0.9 (17.3 + ~3 us
-    // against 25.2 us unsplit for 256x4096x4096)
-    const float score = eff[i] * util * mutil * (s > 1 ? 0.9f : 1.0f);
+    const float score = eff[i] * util * mutil;
     if (score > best_score) {
       best_score = score;
       best = cand[i];
     }
   }
   return best;
+}
+
+// Configuration of a GEMM on fp16 operands: the one with the least estimated time.
+// A round of at most CU-count blocks takes c1 + KT x slope us, c1 the first loads and
+// the epilogue, slope the time of a 64-deep k tile, which grows from `light` (few
+// blocks: latencies) to `full` (every CU busy: LDS, L2 and the power the chip may
+// draw). Measured on MI355X in us, light / full: 256x256 1.03 / 1.38 (4096^3 in
+// 100, 256x4096x4096 in 67), 256x128 0.54 / 0.80, 128x128 0.30 / 0.43
+// (1024x4096x4096 in 34), 64x64 0.15 / 0.175 (256x4096x4096 in 16); the estimates are
+// within 10% of 14 other shapes' times. Splitting K over s blocks per tile adds the
+// partial sums' round trip and a launch.
+// can_split: the caller has a workspace, of which the partial sums may take part_bytes.
+// k_ascending: only kernels that add over k in ascending order, in at
+// most two splits, whose output bits the converting kernels reproduce.
+struct F16Cand {
+  int cfg;
+  float c1, light, full;
+};
+constexpr F16Cand kF16Cands[] = {{20, 7.5f, 1.03f, 1.38f}, {21, 6.0f, 0.79f, 1.14f}, {22, 6.0f, 0.58f, 0.80f},
+                                 {23, 6.0f, 0.58f, 0.80f}, {24, 3.4f, 0.43f, 0.49f}, {25, 6.0f, 0.54f, 0.80f},
+                                 {26, 4.5f, 0.44f, 0.62f}, {27, 3.4f, 0.30f, 0.43f}, {28, 2.3f, 0.22f, 0.265f},
+                                 {29, 2.3f, 0.22f, 0.265f}, {30, 1.6f, 0.15f, 0.175f}};
+struct F16Pick {
+  int cfg, splits;
+};
+F16Pick search_f16(int64_t M, int64_t N, int64_t K, int64_t cus, bool can_split, size_t part_bytes, bool k_ascending) {
+  const int64_t KT = std::max<int64_t>(1, cdiv(K, 64));
+  F16Pick best{20, 1};
+  float best_us = INFINITY;
+  for (const F16Cand& c : kF16Cands) {
+    const TileCfg& t = kCfgs[c.cfg];
+    if (k_ascending && t.ksplit) continue;
+    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
+    for (int s = 1; s <= (!can_split ? 1 : k_ascending ? 2 : 8); s *= 2) {
+      const int64_t kt = cdiv(KT, s);
+      if (s > 1 && (kt < 8 || (s - 1) * kt >= KT || (size_t)s * (size_t)M * (size_t)N * 4 > part_bytes)) break;
+      const float load = std::min(1.f, (float)(tiles * s) / (float)cus);
+      const float slope = c.light + (c.full - c.light) * load;
+      float us = (float)cdiv(tiles * s, cus) * (c.c1 + (float)kt * slope);
+      if (s > 1) us += 3.5f + (float)s * (float)M * (float)N * 8.f / 4e6f;
+      if (us < best_us) {
+        best_us = us;
+        best = F16Pick{c.cfg, s};
+      }
+    }
+  }
+  return best;
+}
+// The last picks of this thread by shape: the search costs about as much host time as
+// a launch does of a decode-sized call.
+F16Pick pick_f16(int64_t M, int64_t N, int64_t K, bool can_split = false, size_t part_bytes = 0, bool k_ascending = false) {
+  struct Entry {
+    int64_t M, N, K, cus;
+    size_t part_bytes;
+    bool can_split, k_ascending;
+    F16Pick pick;
+  };
+  constexpr int kEntries = 64;
+  static thread_local Entry cache[kEntries] = {};  // M = 0: empty (no call has M = 0)
+  Entry& e = cache[(uint64_t)(M * 31 + N * 7 + K) % kEntries];
+  const int64_t cus = num_cus();
+  if (e.M != M || e.N != N || e.K != K || e.cus != cus || e.part_bytes != part_bytes || e.can_split != can_split ||
+      e.k_ascending != k_ascending)
+    e = Entry{M, N, K, cus, part_bytes, can_split, k_ascending, search_f16(M, N, K, cus, can_split, part_bytes, k_ascending)};
+  return e.pick;
 }
 
 template <int BM, int BN, int WM, int WN, int BK, int PF, int NS, bool A_BF16>
@@ -1094,11 +1639,11 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
                 int64_t K, hipStream_t st, float* part = nullptr, int splits = 1) {
   const int bm = kCfgs[cfg].bm, bn = kCfgs[cfg].bn;
   TB_CHECK(splits == 1 || (part != nullptr && splits > 1 && !kCfgs[cfg].skinny && !kCfgs[cfg].stream &&
-                           (int64_t)splits * kCfgs[cfg].bk <= K),
-           "gemm: split K needs a tile configuration, a partial-sum buffer and K >= splits k tiles");
+                           (splits - 1) * cdiv(cdiv(K, kCfgs[cfg].bk), splits) * kCfgs[cfg].bk < K),
+           "gemm: split K needs a tile configuration, a partial-sum buffer and k tiles for every split");
   if (splits == 1) part = nullptr;
   TB_CHECK(!kCfgs[cfg].skinny || M <= bm, "gemm: configuration %d takes M <= %d", cfg, bm);
-  TB_CHECK(!kCfgs[cfg].stream || !A_BF16, "gemm: configuration %d needs fp16 a (tbf16_gemm_f16 or tbf16_linear)", cfg);
+  TB_CHECK(!(kCfgs[cfg].stream || kCfgs[cfg].pingpong) || !A_BF16, "gemm: configuration %d needs fp16 a (tbf16_gemm_f16 or tbf16_linear)", cfg);
   // skinny and stream blocks take `rows` weight rows each: as many as fit (bn)
   // when that already fills whole rounds of blocks over the CUs, else fewer, so
   // that the weight stream is spread over every CU in as few rounds as possible
@@ -1108,7 +1653,10 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
     const int64_t rounds = cdiv(cdiv(N, bn), ncu);
     rows = (int)std::min<int64_t>(bn, std::max<int64_t>(8, cdiv(cdiv(N, rounds * ncu), 8) * 8));
   }
-  const int64_t blocks = kCfgs[cfg].skinny || kCfgs[cfg].stream ? cdiv(N, rows) : cdiv(M, bm) * cdiv(N, bn);
+  // a single row of ksplit tiles that leaves CUs idle: fewer columns per block, as above
+  if (kCfgs[cfg].ksplit && M <= bm && splits == 1 && cdiv(N, bn) < num_cus())
+    rows = (int)std::min<int64_t>(bn, std::max<int64_t>(8, cdiv(cdiv(N, num_cus()), 8) * 8));
+  const int64_t blocks = cdiv(N, rows) * (kCfgs[cfg].skinny || kCfgs[cfg].stream ? 1 : cdiv(M, bm));
   TB_CHECK(blocks < (int64_t)1 << 31 && cdiv(M, bm) < 65536, "gemm: grid too large");
   const bool even = K % kCfgs[cfg].bk == 0;  // no k-tail selects on loaded values
   const auto a = (const uint16_t*)A;
@@ -1146,7 +1694,42 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
     case 16: STREAM(64, 9); break;
     case 17: STREAM(128, 6); break;
     case 18: STREAM(256, 3); break;
+#define PINGPONG(HA_, FB_, S_)                                                                               \
+  if constexpr (!A_BF16) {                                                                             \
+    const int kt_per = (int)cdiv(cdiv(K, 64), splits);                                                 \
+    const dim3 grid(g, part ? (unsigned)splits : 1u);                                                  \
+    if (even)                                                                                          \
+      pingpong_kernel<HA_, FB_, S_, true><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, \
+                                                            M, N, K, part, kt_per);                    \
+    else                                                                                               \
+      pingpong_kernel<HA_, FB_, S_, false><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, \
+                                                             M, N, K, part, kt_per);                   \
+  }
+    case 20: PINGPONG(4, 2, 2); break;
+    case 21: PINGPONG(3, 2, 2); break;
+    case 22: PINGPONG(2, 2, 3); break;
+    case 23: PINGPONG(4, 1, 3); break;
+    case 24: PINGPONG(2, 1, 3); break;
+#define KSPLIT(RM_, RN_, S_)                                                                                  \
+  if constexpr (!A_BF16) {                                                                                  \
+    const int kt_per = (int)cdiv(cdiv(K, 64), splits);                                                      \
+    const dim3 grid(g, part ? (unsigned)splits : 1u);                                                       \
+    if (even)                                                                                               \
+      ksplit_kernel<RM_, RN_, S_, true><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, M, \
+                                                              N, K, part, kt_per, rows);                    \
+    else                                                                                                    \
+      ksplit_kernel<RM_, RN_, S_, false><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, M, \
+                                                               N, K, part, kt_per, rows);                   \
+  }
+    case 25: KSPLIT(8, 4, 3); break;
+    case 26: KSPLIT(6, 4, 3); break;
+    case 27: KSPLIT(4, 4, 4); break;
+    case 28: KSPLIT(4, 2, 6); break;
+    case 29: KSPLIT(2, 4, 6); break;
+    case 30: KSPLIT(2, 2, 6); break;
     default: SKINNY(2, 2, 4, 2, true); break;
+#undef PINGPONG
+#undef KSPLIT
 #undef STREAM
 #undef SKINNY
 #undef CFG
@@ -1186,71 +1769,82 @@ int launch_quantize_rows(const void* x, int64_t R, int64_t K, int64_t ldx, int t
 
 namespace {
 
-// Whether tbf16_linear quantises x once (row exponents, inverse scales and the
-// fp16 rows into its workspace) and runs the GEMM on fp16 operands, instead of
-// converting x inside the GEMM. The decode kernel takes fp16 a only. Tiles of at
-// most 128 columns convert each x tile once per column block (64 times at N =
-// 4096 with 64-column tiles), which the one pass saves: bit-identical output,
-// 256x4096x4096 34.6 -> 27.7 us, 1024x4096x4096 56.9 -> 50.3, 2048x4096x4096 84.4
-// -> 77.1 (128-column tiles). 256-column tiles convert x 16 times at N = 4096
-// and gain nothing there (4096^3: the extra pass costs more than it saves), and
-// at K < 1024 the pass costs about what it saves (200x2560x768: 10.0 vs 10.6 us).
+// Whether tbf16_linear with a pinned configuration quantises x once (row exponents,
+// inverse scales and the fp16 rows into its workspace) and runs the GEMM on fp16
+// operands, instead of converting x inside the GEMM: the kernels that take fp16 a only,
+// and the tiles of at most 128 columns at K >= 1024, which convert each x tile once per
+// column block.
 bool quantize_once(int cfg, int64_t K) {
   if (cfg < 0 || cfg >= kNumCfgs) return false;
   const TileCfg& c = kCfgs[cfg];
-  return c.stream || (!c.skinny && c.bn <= 128 && K >= 1024);
+  return c.stream || c.pingpong || (!c.skinny && c.bn <= 128 && K >= 1024);
 }
 
-// Workspace of tbf16_linear: the row exponents (int32 (M,)); where x is quantised
-// once (`quantize_once`, unless `fused` asks for the conversion inside the GEMM,
-// which the decode kernel cannot do), the row inverse scales (fp32 (M,)) and the
-// scaled fp16 copy of x (M, K); where K is split (`pick_split`), the fp32 partial
-// sums (splits x M x N). Each part 256-byte aligned.
+// How tbf16_linear runs a call, and its workspace: the row exponents (int32 (M,)); with
+// q16, the row inverse scales (fp32 (M,)) and the scaled fp16 copy of x (M, K); where K
+// is split, the fp32 partial sums (splits x M x N). Each part 256-byte aligned.
 struct LinearWs {
   size_t exps, sinv, x16, part, bytes;
-  int splits;
+  int cfg, splits;
   bool q16;
 };
-LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg, bool fused = false) {
-  LinearWs w{0, 0, 0, 0, align_up((size_t)M * 4, 256), 1, false};
-  w.q16 = quantize_once(cfg, K) && !(fused && !kCfgs[cfg].stream);
-  if (w.q16) {
+LinearWs layout_ws(int64_t M, int64_t K, int64_t N, int cfg, int splits, bool q16) {
+  LinearWs w{0, 0, 0, 0, align_up((size_t)M * 4, 256), cfg, splits, q16};
+  if (q16) {
     w.sinv = w.bytes;
     w.x16 = w.sinv + align_up((size_t)M * 4, 256);
     w.bytes = align_up(w.x16 + (size_t)M * (size_t)K * 2, 256);
   }
-  w.splits = pick_split(cfg, M, N, K);
-  if (w.splits > 1) {
+  if (splits > 1) {
     w.part = w.bytes;
-    w.bytes = w.part + (size_t)w.splits * (size_t)M * (size_t)N * 4;
+    w.bytes = w.part + (size_t)splits * (size_t)M * (size_t)N * 4;
   }
   return w;
 }
+// The dispatcher's choice (cfg < 0): x quantised once and a kernel on fp16 operands,
+// also for wide tiles (4096^3: 101 us + 9 us of row pass against 118 + 5 with the
+// conversion in the GEMM). Where that workspace would not fit the no-allocation entry
+// point's array, only kernels whose output the converting tiles reproduce bit for bit,
+// which that entry point then runs.
+LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg) {
+  if (cfg >= 0) return layout_ws(M, K, N, cfg, pick_split(cfg, M, N, K), quantize_once(cfg, K));
+  const size_t base = layout_ws(M, K, N, 20, 1, true).bytes;
+  const bool bounded = base > TBF16_NOALLOC_SCRATCH_BYTES;
+  const F16Pick p = pick_f16(M, N, K, true,
+                             bounded ? kSplitPartBytes : std::min<size_t>(kSplitPartBytes, TBF16_NOALLOC_SCRATCH_BYTES - base),
+                             bounded);
+  return layout_ws(M, K, N, p.cfg, p.splits, true);
+}
+// The form that converts x inside the GEMM, the same output bits: the pinned
+// configuration, or a tile with the splits of the dispatcher's choice (all of them
+// have k tiles of 64 and so the same split points).
+LinearWs fused_ws(int64_t M, int64_t K, int64_t N, int cfg) {
+  if (cfg >= 0) return layout_ws(M, K, N, cfg, pick_split(cfg, M, N, K), false);
+  return layout_ws(M, K, N, pick_fused(M, N, true), linear_ws(M, K, N, cfg).splits, false);
+}
 
-// fused: convert x inside the GEMM even where `quantize_once` holds (same output;
-// for a workspace too small for the fp16 copy of x). The decode kernel cannot.
-int linear_into(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N, int64_t ldw,
-                const float* ws, const void* bias, void* y, int64_t ldy, int t, int l1, int cfg, uint8_t* wsp,
-                bool fused, hipStream_t st) {
-  const LinearWs w = linear_ws(M, K, N, cfg, fused);
+int linear_into(const LinearWs& w, const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N,
+                int64_t ldw, const float* ws, const void* bias, void* y, int64_t ldy, int t, int l1, uint8_t* wsp,
+                hipStream_t st) {
   int32_t* exps = reinterpret_cast<int32_t*>(wsp + w.exps);
   float* part = w.splits > 1 ? reinterpret_cast<float*>(wsp + w.part) : nullptr;
   if (!w.q16) {
     if (int rc = launch_row_exps(x, M, K, ldx, t, l1, exps, nullptr, st)) return rc;
-    return launch_gemm<true>(cfg, x, ldx, exps, nullptr, w16, ldw, ws, bias, y, ldy, M, N, K, st, part, w.splits);
+    return launch_gemm<true>(w.cfg, x, ldx, exps, nullptr, w16, ldw, ws, bias, y, ldy, M, N, K, st, part, w.splits);
   }
   // x quantised once (exponents, inverse scales, fp16 rows), then the GEMM on fp16
   // operands: the same fp16 values the fused kernels convert in registers
   float* sinv = reinterpret_cast<float*>(wsp + w.sinv);
   void* x16 = wsp + w.x16;
   if (int rc = launch_quantize_rows(x, M, K, ldx, t, l1, x16, K, sinv, exps, st)) return rc;
-  return launch_gemm<false>(cfg, x16, K, nullptr, sinv, w16, ldw, ws, bias, y, ldy, M, N, K, st, part, w.splits);
+  return launch_gemm<false>(w.cfg, x16, K, nullptr, sinv, w16, ldw, ws, bias, y, ldy, M, N, K, st, part, w.splits);
 }
 }  // namespace
 
 extern "C" size_t tbf16_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int cfg) {
   if (M <= 0 || K < 0 || N <= 0 || cfg >= kNumCfgs) return M > 0 ? (size_t)M * 4 : 0;
-  return linear_ws(M, K, N, cfg < 0 ? pick_cfg(M, N, true, K) : cfg).bytes;
+  // enough for either form of the call
+  return std::max(linear_ws(M, K, N, cfg).bytes, layout_ws(M, K, N, 0, cfg < 0 ? pick_split(12, M, N, K) : 1, false).bytes);
 }
 
 extern "C" int tbf16_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N,
@@ -1261,8 +1855,8 @@ extern "C" int tbf16_linear(const void* x, int64_t M, int64_t K, int64_t ldx, co
   TB_CHECK(aligned16(workspace), "linear: workspace must be 16-byte aligned");
   TB_CHECK(cfg < kNumCfgs, "bad cfg");
   if (M == 0 || N == 0) return 0;
-  return linear_into(x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1, cfg < 0 ? pick_cfg(M, N, true, K) : cfg,
-                     static_cast<uint8_t*>(workspace), false, as_stream(stream));
+  return linear_into(linear_ws(M, K, N, cfg), x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1,
+                     static_cast<uint8_t*>(workspace), as_stream(stream));
 }
 
 // ---- tbf16_linear_noalloc: the workspace in a static device array ---------------
@@ -1313,17 +1907,18 @@ extern "C" int tbf16_linear_noalloc(const void* x, int64_t M, int64_t K, int64_t
              "linear_noalloc: cannot query the stream's device");
     TB_CHECK(sd == cur, "linear_noalloc: the stream belongs to device %d, the current device is %d", (int)sd, cur);
   }
-  const int c = cfg < 0 ? pick_cfg(M, N, true, K) : cfg;
   // where the fp16 copy of x does not fit, a tile configuration converts x inside
-  // the GEMM instead (the same output); the decode kernel needs the copy
-  const bool fused = !kCfgs[c].stream && linear_ws(M, K, N, c).bytes > TBF16_NOALLOC_SCRATCH_BYTES;
-  const size_t need = linear_ws(M, K, N, c, fused).bytes;
-  TB_CHECK(need <= TBF16_NOALLOC_SCRATCH_BYTES,
+  // the GEMM instead (the same output), except at decode sizes and in the kernels that
+  // take fp16 a only, whose calls are rejected
+  LinearWs w = linear_ws(M, K, N, cfg);
+  const bool f16_only = cfg >= 0 ? kCfgs[cfg].stream || kCfgs[cfg].pingpong : M <= 128 && N >= 32 * num_cus();
+  if (w.bytes > TBF16_NOALLOC_SCRATCH_BYTES && !f16_only) w = fused_ws(M, K, N, cfg);
+  TB_CHECK(w.bytes <= TBF16_NOALLOC_SCRATCH_BYTES,
            "linear_noalloc: %lld x %lld needs %zu workspace bytes, beyond the scratch limit of %d bytes", (long long)M,
-           (long long)K, need, TBF16_NOALLOC_SCRATCH_BYTES);
+           (long long)K, w.bytes, TBF16_NOALLOC_SCRATCH_BYTES);
   uint8_t* wsp = nullptr;
   if (int rc = scratch_ptr(&wsp)) return rc;
-  return linear_into(x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1, c, wsp, fused, st);
+  return linear_into(w, x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1, wsp, st);
 }
 
 extern "C" int tbf16_linear_exps(const void* x, int64_t M, int64_t K, int64_t ldx, const int32_t* exps,
@@ -1333,7 +1928,7 @@ extern "C" int tbf16_linear_exps(const void* x, int64_t M, int64_t K, int64_t ld
   TB_CHECK(exps != nullptr || M == 0, "linear_exps: exps missing");
   TB_CHECK(cfg < kNumCfgs, "bad cfg");
   if (M == 0 || N == 0) return 0;
-  return launch_gemm<true>(cfg < 0 ? pick_cfg(M, N, false) : cfg, x, ldx, exps, nullptr, w16, ldw, ws, bias, y, ldy, M, N, K,
+  return launch_gemm<true>(cfg < 0 ? pick_fused(M, N, false) : cfg, x, ldx, exps, nullptr, w16, ldw, ws, bias, y, ldy, M, N, K,
                            as_stream(stream));
 }
 
@@ -1344,6 +1939,6 @@ extern "C" int tbf16_gemm_f16(const void* a16, int64_t M, int64_t K, int64_t lda
   TB_CHECK(sa != nullptr || M == 0, "gemm_f16: sa missing");
   TB_CHECK(cfg < kNumCfgs, "bad cfg");
   if (M == 0 || N == 0) return 0;
-  return launch_gemm<false>(cfg < 0 ? pick_cfg(M, N, true) : cfg, a16, lda, nullptr, sa, b16, ldb, sb, bias, y, ldy, M, N,
+  return launch_gemm<false>(cfg < 0 ? pick_f16(M, N, K).cfg : cfg, a16, lda, nullptr, sa, b16, ldb, sb, bias, y, ldy, M, N,
                             K, as_stream(stream));
 }

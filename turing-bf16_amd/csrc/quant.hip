@@ -462,6 +462,21 @@ extern "C" int tbf16_quantize_rows_t(const void* x, int64_t R, int64_t K, int64_
   return 0;
 }
 
+extern "C" int tbf16_quantize_rows_both(const void* x, int64_t R, int64_t K, int64_t ldx, int t, void* y16, int64_t ldy,
+                                        void* yT, int64_t ldyT, float* s_inv, int32_t* exps_ws, void* stream) {
+  if (int rc = check_rows("quantize_rows_both", x, R, K, ldx)) return rc;
+  TB_CHECK(ldy % 8 == 0 && ldy >= K && aligned16(y16), "quantize_rows_both: bad output");
+  TB_CHECK(ldyT % 8 == 0 && ldyT >= R && aligned16(yT) && s_inv && exps_ws, "quantize_rows_both: bad output");
+  hipStream_t st = as_stream(stream);
+  if (int rc = launch_quantize_rows(x, R, K, ldx, t, 0, y16, ldy, s_inv, exps_ws, st)) return rc;
+  if (K == 0 || ldyT == 0) return 0;
+  dim3 grid((unsigned)cdiv(K, 256), (unsigned)cdiv(ldyT, 64));
+  transpose_convert_kernel<<<grid, 256, 0, st>>>((const uint16_t*)x, R, K, ldx, exps_ws, nullptr, nullptr,
+                                                 (uint16_t*)yT, ldyT);
+  TB_LAUNCH_CHECK("quantize_rows_both");
+  return 0;
+}
+
 extern "C" size_t tbf16_quantize_cols_ws_bytes(int64_t R, int64_t K) {
   const int64_t ch = col_chunks(R, K);
   return align_up((size_t)(ch * K) * sizeof(float), 256) + align_up((size_t)K * sizeof(int32_t), 256);

@@ -36,6 +36,7 @@ _SIGS = {
     "tbf16_row_exps": (I, [P, I64, I64, I64, I, I, P, P, P]),
     "tbf16_quantize_rows": (I, [P, I64, I64, I64, I, I, P, I64, P, P]),
     "tbf16_quantize_rows_t": (I, [P, I64, I64, I64, I, P, I64, P, P, P]),
+    "tbf16_quantize_rows_both": (I, [P, I64, I64, I64, I, P, I64, P, I64, P, P, P]),
     "tbf16_quantize_cols_ws_bytes": (SZ, [I64, I64]),
     "tbf16_quantize_cols_t": (I, [P, I64, I64, I64, I, P, P, I64, P, P, I64, P]),
     "tbf16_linear_ws_bytes": (SZ, [I64, I64, I64, I]),
