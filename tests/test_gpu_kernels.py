@@ -4,6 +4,8 @@ relative Frobenius error <= 2e-3 and no worse than the reference's own error,
 which the oracle emulates)."""
 import ctypes
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -359,6 +361,29 @@ def test_attention_causal_block_forms(dev, monkeypatch, B, H, S, D, layout, spli
     if layout == "bshd":  # permuted views: row stride H * D
         q, k, v = (t.transpose(1, 2) for t in (q, k, v))
     _attn_checks(q, k, v, dev, label=f"split={split} k={kform} {layout} B={B} H={H} S={S} D={D}")
+
+
+@pytest.mark.parametrize("split", ["0", "1"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Sq,Sk,D", [(33, 65, 64), (130, 257, 128), (200, 127, 96), (257, 64, 64), (16, 3, 128)])
+def test_attention_bias_forms(dev, monkeypatch, Sq, Sk, D, causal, split):
+    """Bias rows read four keys at a time at any alignment (odd row strides and a
+    broadcast padding row), with whole and cut key tiles, in plain and split-key blocks
+    (with fewer key tiles than groups too): within the bound of the unbiased forms of
+    fp64 softmax(q k^T scale + bias) v."""
+    monkeypatch.setenv("TBF16_ATTN_SPLIT", split)
+    g = torch.Generator().manual_seed(Sq + Sk)
+    q = torch.randn(2, 3, Sq, D, generator=g).bfloat16()
+    k, v = (torch.randn(2, 3, Sk, D, generator=g).bfloat16() for _ in range(2))
+    rows = torch.randn(2, 3, Sq, Sk, generator=g).half()
+    pad = torch.arange(Sk).view(1, 1, 1, Sk) < torch.tensor([Sk, (Sk + 2) // 2]).view(2, 1, 1, 1)
+    for mask in (rows, pad):
+        got = tbf16.sdpa(q.to(dev), k.to(dev), v.to(dev), attn_mask=mask.to(dev), is_causal=causal)
+        s = q.double() @ k.double().transpose(-1, -2) * D ** -0.5
+        s = s + mask.double() if mask.dtype == torch.float16 else s.masked_fill(~mask, -math.inf)
+        if causal:
+            s = s.masked_fill(torch.ones(Sq, Sk, dtype=torch.bool).triu(1), -math.inf)
+        assert rel(got.cpu(), torch.softmax(s, -1) @ v.double()) < TOL
 
 
 @pytest.mark.parametrize("kform", ["bf16", "fp16"])

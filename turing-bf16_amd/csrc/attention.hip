@@ -16,13 +16,16 @@
 //
 // Block = 4 or 8 waves, 32 query rows per wave; key tiles of 64.
 //  - a wave keeps its 32 q rows as MFMA fragments in registers for the whole
-//    kernel and computes S^T = K Q^T with v_mfma_f32_32x32x16_f16 (K from LDS), so
-//    each lane owns ONE query row: row max / sum need one exchange with lane ^ 32.
+//    kernel and computes S^T = K Q^T with 16x16x32 MFMAs (K from LDS), so each lane
+//    owns two query rows, 16 apart: row max / sum need exchanges with lanes ^ 16 and
+//    ^ 32. Long sequences run at the clock that the chip's power allows, and this MFMA
+//    shape costs less of it than 32x32x16: 16k causal, 16 heads, D = 128, 1.85 -> 1.90
+//    GHz and 1035 -> 984 us a call.
 //  - online softmax in fp32, base 2 (logit * scale * log2 e), P rounded to fp16.
 //  - O^T = V^T P^T: V is stored transposed in LDS (d-major, keys permuted within
-//    each 16-key group by swapping index bits 2 and 3) so that the A fragment of
-//    a lane is one 16-byte read and P's fragment comes straight from S^T's
-//    accumulators without any cross-lane shuffle.
+//    each 32-key group, vt_run) so that the A fragment of a lane is one 16-byte read
+//    and P's fragment comes straight from S^T's accumulators without any cross-lane
+//    shuffle.
 //  - row sums l come from the fp16 P that enters the PV product (v_dot2 with
 //    ones), so the normalisation matches the weights actually applied.
 //  - output bf16(O / l * 2^ev) written from registers: one rounding.
@@ -33,6 +36,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <atomic>
 #include <math.h>
 
 #include <type_traits>
@@ -78,9 +82,10 @@ struct FwdParams {
   float drop_scale;
 };
 
-__device__ __forceinline__ int perm16(int key) {  // swap bits 2 and 3 of a key index
-  return (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1);
-}
+// Position of key 4 kg's run of four in its 64-key tile of V^T: within each 32 keys,
+// k slots 8 f + r of the PV operand are keys 4 f + r, slots 8 f + 4 + r keys 16 + 4 f + r
+// (what a lane's S^T accumulators of two 16-key blocks hold).
+__device__ __forceinline__ int vt_run(int kg) { return 32 * (kg >> 3) + 8 * (kg & 3) + 4 * ((kg >> 2) & 1); }
 
 template <int DP>
 __device__ __forceinline__ int swz_k(int row, int chunk) {
@@ -93,17 +98,43 @@ __device__ __forceinline__ int swz_vt(int d, int chunk) { return d * 128 + ((chu
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// One 32x32x16 step of S^T = K Q^T: fp16 operands (k16, q 2^a), or with KBF the
-// raw bf16 rows of k and q (v_mfma_f32_32x32x16_bf16, the same rate on gfx950).
+// One 16x16x32 step of S^T = K Q^T: fp16 operands (k16, q 2^a), or with KBF the
+// raw bf16 rows of k and q (v_mfma_f32_16x16x32_bf16, the same rate on gfx950).
 // Scaling a bf16 value by 2^a into fp16 is exact unless it leaves fp16's normal
 // range, so both forms multiply the same values: q.k 2^(a - a).
 template <bool KBF>
-__device__ __forceinline__ floatx16 mfma_qk(half8 k, half8 q, floatx16 c) {
+__device__ __forceinline__ floatx4 mfma_qk(half8 k, half8 q, floatx4 c) {
   if constexpr (KBF)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, k), __builtin_bit_cast(bf16x8, q), c, 0,
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k), __builtin_bit_cast(bf16x8, q), c, 0,
                                                     0, 0);
-  else return __builtin_amdgcn_mfma_f32_32x32x16_f16(k, q, c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_f16(k, q, c, 0, 0, 0);
 }
+
+// O^T accumulators of one 16-query column: NB blocks of 16 d (4 values a lane each) in
+// vectors of up to 32 registers. As separate 4-register values the compiler gives each
+// MFMA a new destination and copies all of them around the rarely taken rescale (32
+// moves per tile, a sixth of the softmax's instructions); parts of one wide value stay
+// where they are.
+template <int NB>
+struct AccCol {
+  static constexpr int W = NB * 4 < 32 ? NB * 4 : 32, NV = NB * 4 / W;
+  typedef float vec __attribute__((ext_vector_type(W)));
+  vec v[NV];
+  __device__ __forceinline__ float at(int db, int r) const { return v[db * 4 / W][db * 4 % W + r]; }
+  __device__ __forceinline__ floatx4 get(int db) const { return floatx4{at(db, 0), at(db, 1), at(db, 2), at(db, 3)}; }
+  __device__ __forceinline__ void set(int db, floatx4 x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[db * 4 / W][db * 4 % W + r] = x[r];
+  }
+  __device__ __forceinline__ void scale(float f) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] *= f;
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = 0.f;
+  }
+};
 
 // Block-wide max of an int (NT threads, one slot per wave in red).
 template <int NT>
@@ -119,17 +150,21 @@ __device__ __forceinline__ int block_max_int(int v, int* red) {
   return r;
 }
 
-// Masks the scores of a key tile that crosses the end of the keys or (causal)
-// the diagonal: keys >= Sk or > qmax become -inf. Lane layout of S^T: key
-// key0 + 32 kh + 8 (r / 4) + 4 fk + r % 4 in accumulator r of half kh. Called
-// from a wave-uniform branch, so interior tiles skip it.
-__device__ __forceinline__ void mask_tile(floatx16 (&sacc)[2], int key0, int Sk, int qmax, int fk) {
-  const int lim = min(Sk - 1, qmax) - key0 - 4 * fk;  // keep offsets <= lim
+// Masks the scores of a key tile that crosses the end of the keys or (CAUSAL) the
+// diagonal: keys >= Sk or past the query become -inf. Lane layout of S^T: key
+// key0 + 16 i + 4 fk + r of query row qrow[qb] in sacc[i][qb][r]. Called from a
+// wave-uniform branch, so interior tiles skip it.
+template <bool CAUSAL>
+__device__ __forceinline__ void mask_tile(floatx4 (&sacc)[4][2], int key0, int Sk, const int (&qrow)[2], int fk) {
 #pragma unroll
-  for (int kh = 0; kh < 2; ++kh)
+  for (int qb = 0; qb < 2; ++qb) {
+    const int lim = (CAUSAL ? min(Sk - 1, qrow[qb]) : Sk - 1) - key0 - 4 * fk;  // keep offsets <= lim
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if (kh * 32 + 8 * (r >> 2) + (r & 3) > lim) sacc[kh][r] = -INFINITY;
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (16 * i + r > lim) sacc[i][qb][r] = -INFINITY;
+  }
 }
 
 // Halves j of four rows (packed fp16 words w0..w3 holding halves 2i, 2i+1) -> the
@@ -172,7 +207,7 @@ __device__ __forceinline__ void heads_max(const float* part, int nbh, int nch, F
 // (row c / (DP / 8), chunk c % (DP / 8)). V: thread t takes blocks t + 256 i of 4
 // keys x 8 columns (kg = block % 16, dc = block / 16), converts the four 16-byte
 // row pieces and writes, for each of its 8 columns d, the 4-key run at position
-// perm16(4 kg) of row d of the tile's V^T block (8 bytes; the 16 threads of one dc
+// vt_run(kg) of row d of the tile's V^T block (8 bytes; the 16 threads of one dc
 // fill each 128-byte row; the tile's DP rows are one contiguous block, which the
 // forward kernel then copies to LDS 1 KB at a time). Keys past Sk and columns
 // past D are written as zeros.
@@ -265,7 +300,7 @@ __global__ __launch_bounds__(256) void kv_prep_kernel(FwdParams p) {
     uint4 cv[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) cv[r] = cvt_bf16x8_f16x8(vr[i][r], sv);
-    const int pos = perm16(4 * kg);
+    const int pos = vt_run(kg);
     const uint32_t* w0 = reinterpret_cast<const uint32_t*>(&cv[0]);
     const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&cv[1]);
     const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&cv[2]);
@@ -283,31 +318,34 @@ __global__ __launch_bounds__(256) void kv_prep_kernel(FwdParams p) {
 // SPLIT (NW = 8): waves w and w + 4 take the same 32 query rows (BQ = 128) and
 // the even and the odd key tiles respectively, from four LDS stages (a pair of
 // tiles in flight while the other pair is read); the odd group hands its O^T,
-// running max and row sums to its partner through LDS at the end. A causal grid
-// of few blocks then gets both the heavy/light pairing (every block the same
-// work) and two waves per SIMD.
+// running max and row sums to its partner through LDS at the end. A grid of few
+// blocks then gets two waves per SIMD, a causal one with the heavy/light pairing
+// (every block the same work).
 // KBF: S^T = K Q^T on the raw bf16 rows of k and q (bf16 MFMA), K tiles copied
 // straight from k (head dim = DP); only V goes through the conversion pass.
+// HAS_BIAS: the rows are read four keys at a time (one by one they had bound the
+// kernel: key-padding mask, B = 2, H = 12, S = 1111, D = 64, 84 -> 58 us a call).
 template <int DP, int NW, bool CAUSAL, bool HAS_BIAS, bool DROP, bool SPLIT = false, bool KBF = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP > 128 ? 1 : 2, DP > 128 ? 1 : 2))) void
 attn_fwd_kernel(FwdParams p) {
-  static_assert(!SPLIT || (NW == 8 && DP <= 128 && !HAS_BIAS && !DROP), "split-key blocks: 8 waves, no bias or dropout");
-  static_assert(!KBF || (DP <= 128 && !HAS_BIAS && !DROP), "bf16 K rows: head dim <= 128, no bias or dropout");
+  static_assert(!SPLIT || (NW == 8 && DP <= 128 && !DROP), "split-key blocks: 8 waves, no dropout");
+  static_assert(!KBF || (DP <= 128 && !DROP), "bf16 K rows: head dim <= 128, no dropout");
   constexpr int RB = SPLIT ? NW / 2 : NW;  // 32-row query blocks per block
   constexpr int NT = NW * 64, BQW = 32 * RB;
-  constexpr int KS = DP / 16;            // MFMA k-steps over the head dim
-  constexpr int DB = DP / 32;            // 32-wide d blocks of O^T
+  constexpr int KS = DP / 32;            // MFMA k-steps over the head dim
+  constexpr int DB = DP / 16;            // 16-wide d blocks of O^T
   constexpr int CPR = DP / 8;            // 16-byte chunks per K row
   constexpr int KBYTES = BKV * DP * 2;
   constexpr int STAGE = KBYTES + DP * 128;
-  // V^T fragments read during the QK product (registers allow it up to DP = 128
-  // without the bias rows or the dropout hashing)
-  constexpr bool VPRE = DP <= 128 && !HAS_BIAS && !DROP;
+  // fragment reads run ahead under an instruction-group schedule (registers allow it
+  // up to DP = 128 without the dropout hashing)
+  constexpr bool VPRE = DP <= 128 && !DROP;
   // K and V^T tiles go global -> LDS directly, 1 KB per wave instruction: BPW
   // such blocks per wave per tile, the first KPW of them K, the rest V^T
   constexpr int KBLK = KBYTES / 1024, NBLK = STAGE / 1024;
   static_assert(NBLK % NW == 0 && KBLK % NW == 0, "K/V staging blocks");
   constexpr int BPW = NBLK / NW, KPW = KBLK / NW;
+  (void)NT; (void)CPR;
   // two stages as separate objects, so that the compiler's LDS alias analysis
   // sees that reads of one stage never wait for the loads into the other (a
   // third stage, loads two tiles ahead, measured no faster)
@@ -317,7 +355,7 @@ attn_fwd_kernel(FwdParams p) {
   __shared__ __align__(1024) uint8_t smem3[SPLIT ? STAGE : 16];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 31, fk = lane >> 5;
+  const int fr = lane & 15, fk = lane >> 4;
   const int rw = SPLIT ? wave % RB : wave;  // this wave's 32-row query block
   const int grp = SPLIT ? wave / RB : 0;    // SPLIT: key tiles of this parity
   // grid (heads, query blocks): dispatch runs over heads first, so the heaviest
@@ -338,18 +376,22 @@ attn_fwd_kernel(FwdParams p) {
   for (int pass = 0; pass < npass; ++pass) {
     const int qt = !CAUSAL ? bx : p.pair ? (pass == 0 ? ntiles - 1 - bx : bx) : (int)gridDim.y - 1 - bx;
     const int q0 = qt * BQW;
-    // ---- Q fragments in registers (fp16, scaled by 2^a) ----
-    const int qrow = q0 + rw * 32 + fr;
-    const uint32_t drow = DROP ? drop_row((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qrow, p.drop_lo) : 0u;
-    half8 qf[KS];
-    {
-      const uint16_t* qp = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)min(qrow, p.Sq - 1) * p.q_ss;
+    // ---- Q fragments in registers (fp16, scaled by 2^a; KBF: bf16): this lane's rows
+    // are qrow[0] and qrow[1], 16 apart ----
+    int qrow[2];
+    uint32_t drow[2];
+    half8 qf[2][KS];
+  #pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      qrow[qb] = q0 + rw * 32 + qb * 16 + fr;
+      drow[qb] = DROP ? drop_row((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qrow[qb], p.drop_lo) : 0u;
+      const uint16_t* qp = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)min(qrow[qb], p.Sq - 1) * p.q_ss;
   #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        const int d = 16 * s + 8 * fk;
+        const int d = 32 * s + 8 * fk;
         uint4 v = make_uint4(0, 0, 0, 0);
-        if (qrow < p.Sq && d < p.D) v = KBF ? ldg16(qp + d) : cvt_bf16x8_f16x8(ldg16(qp + d), sq);
-        qf[s] = __builtin_bit_cast(half8, v);
+        if (qrow[qb] < p.Sq && d < p.D) v = KBF ? ldg16(qp + d) : cvt_bf16x8_f16x8(ldg16(qp + d), sq);
+        qf[qb][s] = __builtin_bit_cast(half8, v);
       }
     }
 
@@ -396,89 +438,95 @@ attn_fwd_kernel(FwdParams p) {
       }
     };
 
-    floatx16 acc_o[DB];
-  #pragma unroll
-    for (int i = 0; i < DB; ++i)
-  #pragma unroll
-      for (int r = 0; r < 16; ++r) acc_o[i][r] = 0.f;
+    AccCol<DB> acc_o[2];  // [16 queries]
+    acc_o[0].clear();
+    acc_o[1].clear();
     // running max in log2 units; stays stale until a row's max grows by more than
     // 2^8, so exp2 arguments are <= 8 and P <= 256 (fp16-safe)
-    float m_run = -INFINITY, l_run = 0.f;
+    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
     const float c = HAS_BIAS ? 1.f : p.scale_log2;
 
     const int nkb_all = (p.Sk + BKV - 1) / BKV;
     int nkb = nkb_all;
     if constexpr (CAUSAL) nkb = min(nkb_all, (min(q0 + BQW, p.Sq) + BKV - 1) / BKV);
-    const uint16_t* brow = nullptr;
-    if constexpr (HAS_BIAS)
-      brow = p.bias + (int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh + (int64_t)min(qrow, p.Sq - 1) * p.bias_sq;
-
-    // The last PV step of each tile runs at the start of the next tile, after its
-    // first K reads have gone out (its fragments were read before the barrier),
-    // so the barrier's drain and those reads' latency hide behind 4 MFMAs. It
-    // starts as zeros (adds nothing) and is flushed after the last tile.
-    half8 dpf, dvf[DB];
-    for (int e = 0; e < 8; ++e) dpf[e] = (_Float16)0.f;
+    const uint16_t* brow[2] = {nullptr, nullptr};
+    if constexpr (HAS_BIAS) {
   #pragma unroll
-    for (int db = 0; db < DB; ++db) dvf[db] = dpf;
+      for (int qb = 0; qb < 2; ++qb)
+        brow[qb] = p.bias + (int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh + (int64_t)min(qrow[qb], p.Sq - 1) * p.bias_sq;
+    }
+
+    // The last quarter of each tile's PV product runs at the start of the next tile,
+    // after its first K reads have gone out (its fragments were read before the
+    // barrier), so the barrier's drain and those reads' latency hide behind its MFMAs.
+    // It starts as zeros (adds nothing) and is flushed after the last tile.
+    constexpr int DQ = DB / 2;  // d blocks of the deferred quarter: DB - DQ .. of the second 32 keys
+    half8 dpf[2], dvf[DQ];
+    for (int e = 0; e < 8; ++e) dpf[0][e] = (_Float16)0.f;
+    dpf[1] = dpf[0];
+  #pragma unroll
+    for (int i = 0; i < DQ; ++i) dvf[i] = dpf[0];
+    auto pv = [&](const half8& vf, const half8(&pf)[2], int db) {
+  #pragma unroll
+      for (int qb = 0; qb < 2; ++qb)
+        acc_o[qb].set(db, __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[qb], acc_o[qb].get(db), 0, 0, 0));
+    };
     auto deferred = [&]() {
   #pragma unroll
-      for (int db = 0; db < DB; ++db) acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(dvf[db], dpf, acc_o[db], 0, 0, 0);
+      for (int i = 0; i < DQ; ++i) pv(dvf[i], dpf, DB - DQ + i);
     };
     auto step = [&](int kb, const uint8_t* sK, auto masked_c) {
       constexpr bool MASKED = decltype(masked_c)::value;
       const uint8_t* sV = sK + KBYTES;
-      // S^T = K Q^T for two 32-key halves: lane = one query row, 16 keys each.
-      // Fragment reads run ahead of their MFMAs (the compiler otherwise reads each
-      // fragment at its use and waits on it): the first half's K fragments, then
-      // the second half's K fragments between the first half's MFMAs, then the V^T
-      // fragments of the first two PV steps between the second half's MFMAs; the
-      // remaining V^T fragments are read during the PV MFMAs two steps ahead.
-      // Pinned by instruction-group schedules (DP <= 128 without bias rows; else
-      // each fragment is read at its use).
-      floatx16 sacc[2];
+      // S^T = K Q^T for four 16-key blocks: lane = two query rows (16 apart), 4 keys of
+      // each block. Fragment reads run ahead of their MFMAs (the compiler otherwise
+      // reads each fragment at its use and waits on it): the K fragments, then the
+      // V^T fragments of the first 32 keys between the last K MFMAs; the other V^T
+      // fragments are read during the PV MFMAs. Pinned by instruction-group schedules
+      // (VPRE; else each fragment is read at its use).
+      floatx4 sacc[4][2];
   #pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
+      for (int i = 0; i < 4; ++i)
   #pragma unroll
-        for (int r = 0; r < 16; ++r) sacc[kh][r] = 0.f;
-      auto kread = [&](int kh, int s) {
-        return *reinterpret_cast<const half8*>(sK + swz_k<DP>(kh * 32 + fr, 2 * s + fk));
+        for (int qb = 0; qb < 2; ++qb)
+  #pragma unroll
+          for (int r = 0; r < 4; ++r) sacc[i][qb][r] = 0.f;
+      auto kread = [&](int i, int s) {
+        return *reinterpret_cast<const half8*>(sK + swz_k<DP>(i * 16 + fr, 4 * s + fk));
       };
-      auto vread = [&](int ks, int db) {
-        return *reinterpret_cast<const half8*>(sV + swz_vt(db * 32 + fr, 2 * ks + fk));
+      auto vread = [&](int g, int db) {
+        return *reinterpret_cast<const half8*>(sV + swz_vt(db * 16 + fr, 4 * g + fk));
       };
-      half8 vf[VPRE ? 4 : 1][DB];
+      half8 vf[VPRE ? DB : 1];
       if constexpr (VPRE) {
-        // One read queue: the K fragments in MFMA order, the two halves' chains
-        // alternating (consecutive MFMAs never depend on each other: a dependent
-        // MFMA waits for its predecessor's result), then the V^T fragments of PV
-        // steps 0 and 1; reads run LA MFMAs ahead, two per MFMA at first.
-        constexpr int LA = 4, NK = 2 * KS, NQ = NK + 2 * DB, EXTRA = NQ - LA - NK;
+        // One read queue: the K fragments in MFMA order (k step by k step, so that
+        // consecutive MFMAs never depend on each other), then the V^T fragments of the
+        // first 32 keys; reads run LA fragments ahead, two per fragment at first.
+        constexpr int LA = 4, NK = 4 * KS, NQ = NK + DB, EXTRA = NQ - LA - NK;
         static_assert(EXTRA >= 0 && EXTRA <= NK, "read queue");
         half8 fq[NQ];
   #pragma unroll
         for (int j = 0; j < NQ; ++j) {
-          if (j < NK) fq[j] = kread(j & 1, j >> 1);
-          else fq[j] = vread((j - NK) / DB, (j - NK) % DB);
+          if (j < NK) fq[j] = kread(j & 3, j >> 2);
+          else fq[j] = vread(0, j - NK);
         }
         deferred();
   #pragma unroll
         for (int j = 0; j < NK; ++j)
-          sacc[j & 1] = mfma_qk<KBF>(fq[j], qf[j >> 1], sacc[j & 1]);
   #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+          for (int qb = 0; qb < 2; ++qb) sacc[j & 3][qb] = mfma_qk<KBF>(fq[j], qf[qb][j >> 2], sacc[j & 3][qb]);
   #pragma unroll
-          for (int db = 0; db < DB; ++db) vf[ks][db] = fq[NK + ks * DB + db];
+        for (int db = 0; db < DB; ++db) vf[db] = fq[NK + db];
         __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, DB, 0);  // the previous tile's deferred step
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * DQ, 0);  // the previous tile's deferred quarter
   #pragma unroll
         for (int i = 0; i < EXTRA; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
   #pragma unroll
         for (int i = EXTRA; i < NK; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -487,84 +535,115 @@ attn_fwd_kernel(FwdParams p) {
   #pragma unroll
         for (int s = 0; s < KS; ++s)
   #pragma unroll
-          for (int kh = 0; kh < 2; ++kh) sacc[kh] = mfma_qk<KBF>(kread(kh, s), qf[s], sacc[kh]);
+          for (int i = 0; i < 4; ++i) {
+            const half8 kf = kread(i, s);
+  #pragma unroll
+            for (int qb = 0; qb < 2; ++qb) sacc[i][qb] = mfma_qk<KBF>(kf, qf[qb][s], sacc[i][qb]);
+          }
       }
       const int key0 = kb * BKV;
       const bool edge = (key0 + BKV > p.Sk) || (CAUSAL && key0 + BKV - 1 > q0 + rw * 32);
       if constexpr (HAS_BIAS) {
+        // four keys' bias in one 8-byte load (rows need not be aligned), one by one
+        // where the tile crosses the end of the keys
+        const bool whole = key0 + BKV <= p.Sk;
   #pragma unroll
-        for (int kh = 0; kh < 2; ++kh)
+        for (int i = 0; i < 4; ++i)
   #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = key0 + kh * 32 + 8 * (r >> 2) + 4 * fk + (r & 3);
-            sacc[kh][r] = sacc[kh][r] * p.scale_log2 +
-                          (key < p.Sk ? (float)__builtin_bit_cast(_Float16, brow[key]) * kLog2e : 0.f);
+          for (int qb = 0; qb < 2; ++qb) {
+            const int key = key0 + i * 16 + 4 * fk;
+            half4 bv;
+            if (whole) {
+              __builtin_memcpy(&bv, brow[qb] + key, 8);
+            } else {
+  #pragma unroll
+              for (int r = 0; r < 4; ++r)
+                bv[r] = key + r < p.Sk ? __builtin_bit_cast(_Float16, brow[qb][key + r]) : (_Float16)0.f;
+            }
+  #pragma unroll
+            for (int r = 0; r < 4; ++r) sacc[i][qb][r] = sacc[i][qb][r] * p.scale_log2 + (float)bv[r] * kLog2e;
           }
       }
-      if (MASKED && edge) mask_tile(sacc, key0, p.Sk, CAUSAL ? qrow : INT_MAX, fk);
-      float mx = -INFINITY;
+      if (MASKED && edge) mask_tile<CAUSAL>(sacc, key0, p.Sk, qrow, fk);
+      float mx[2];
   #pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
+      for (int qb = 0; qb < 2; ++qb) {
+        mx[qb] = -INFINITY;
   #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[kh][r]);
-      mx = max_xor32(mx) * c;
-      if (__any(mx > m_run + 8.f)) {  // wave-uniform: rescale O and l only when some row needs it
-        const float m_new = fmaxf(m_run, mx);
-        const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
-        l_run *= alpha;
+        for (int i = 0; i < 4; ++i)
   #pragma unroll
-        for (int i = 0; i < DB; ++i)
-  #pragma unroll
-          for (int r = 0; r < 16; ++r) acc_o[i][r] *= alpha;
+          for (int r = 0; r < 4; ++r) mx[qb] = fmaxf(mx[qb], sacc[i][qb][r]);
+        mx[qb] = max_xor32(max_xor16(mx[qb])) * c;
       }
-      const float mneg = (m_run == -INFINITY) ? 0.f : -m_run;
-      // row sums from the fp16 P that the PV product uses (v_dot2 with ones)
+      if (__any(mx[0] > m_run[0] + 8.f || mx[1] > m_run[1] + 8.f)) {  // wave-uniform: rescale only when some row needs it
+  #pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+          const float m_new = fmaxf(m_run[qb], mx[qb]);
+          const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run[qb] - m_new);
+          m_run[qb] = m_new;
+          l_run[qb] *= alpha;
+          acc_o[qb].scale(alpha);
+        }
+      }
+      // row sums from the fp16 P that the PV product uses (v_dot2 with ones); pf[g]:
+      // P^T of 32 keys, k slots 8 fk + r = key 4 fk + r of block 2 g, + 4 = of block 2 g + 1
       const half2v ones = {(_Float16)1.f, (_Float16)1.f};
-      float lsum = 0.f;
-      uint32_t pk[2][8];
+      half8 pf[2][2];
   #pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
+      for (int qb = 0; qb < 2; ++qb) {
+        const float mneg = (m_run[qb] == -INFINITY) ? 0.f : -m_run[qb];
+        float lsum = 0.f;
   #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[kh][r], c, mneg));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[kh][r + 1], c, mneg));
-          pk[kh][r >> 1] = pack_f16(p0, p1);
-          lsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, pk[kh][r >> 1]), ones, lsum, false);
-          if constexpr (DROP) {  // l keeps the undropped weights; the PV product gets the kept ones,
-            // unscaled (P reaches 2^8 under the lazy rescale: P / (1 - p) would leave fp16
-            // for p near 1), and the epilogue applies 1 / (1 - p) in fp32
-            const int key = key0 + kh * 32 + 8 * (r >> 2) + 4 * fk + (r & 3);  // even
-            const uint32_t u = drop_pair(drow, key, p.drop_hi);
-            pk[kh][r >> 1] = pack_f16(drop_keep(u, key, p.drop_thr) ? p0 : 0.f,
-                                      drop_keep(u, key + 1, p.drop_thr) ? p1 : 0.f);
+        for (int g = 0; g < 2; ++g) {
+          uint32_t w[4];
+  #pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int i = 2 * g + (j >> 1), r = 2 * (j & 1);
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[i][qb][r], c, mneg));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[i][qb][r + 1], c, mneg));
+            w[j] = pack_f16(p0, p1);
+            lsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, w[j]), ones, lsum, false);
+            if constexpr (DROP) {  // l keeps the undropped weights; the PV product gets the kept ones,
+              // unscaled (P reaches 2^8 under the lazy rescale: P / (1 - p) would leave fp16
+              // for p near 1), and the epilogue applies 1 / (1 - p) in fp32
+              const int key = key0 + i * 16 + 4 * fk + r;  // even
+              const uint32_t u = drop_pair(drow[qb], key, p.drop_hi);
+              w[j] = pack_f16(drop_keep(u, key, p.drop_thr) ? p0 : 0.f, drop_keep(u, key + 1, p.drop_thr) ? p1 : 0.f);
+            }
           }
+          pf[g][qb] = __builtin_bit_cast(half8, make_uint4(w[0], w[1], w[2], w[3]));
         }
-      l_run += lsum;
-      // O^T += V^T P^T over four 16-key steps
-  #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const uint4 pw = make_uint4(pk[ks >> 1][4 * (ks & 1) + 0], pk[ks >> 1][4 * (ks & 1) + 1],
-                                    pk[ks >> 1][4 * (ks & 1) + 2], pk[ks >> 1][4 * (ks & 1) + 3]);
-        const half8 pf = __builtin_bit_cast(half8, pw);
-        if (ks == 3) {  // deferred past the barrier (operands stay in registers)
-          dpf = pf;
-  #pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            if constexpr (VPRE) dvf[db] = vf[3][db];
-            else dvf[db] = vread(3, db);
-          }
-        } else if constexpr (VPRE) {
-  #pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[ks][db], pf, acc_o[db], 0, 0, 0);
-            if (ks < 2) vf[ks + 2][db] = vread(ks + 2, db);
-          }
-        } else {
-  #pragma unroll
-          for (int db = 0; db < DB; ++db) acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vread(ks, db), pf, acc_o[db], 0, 0, 0);
-        }
+        l_run[qb] += lsum;
       }
+      // O^T += V^T P^T over two 32-key steps; the second step's last DQ d blocks are
+      // deferred past the barrier (operands stay in registers)
+      if constexpr (VPRE) {
+  #pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          pv(vf[db], pf[0], db);
+          vf[db] = vread(1, db);
+        }
+  #pragma unroll
+        for (int db = 0; db < DB - DQ; ++db) pv(vf[db], pf[1], db);
+  #pragma unroll
+        for (int i = 0; i < DQ; ++i) dvf[i] = vf[DB - DQ + i];
+  #pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * (DB - DQ), 0);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+  #pragma unroll
+        for (int db = 0; db < DB; ++db) pv(vread(0, db), pf[0], db);
+  #pragma unroll
+        for (int db = 0; db < DB - DQ; ++db) pv(vread(1, db), pf[1], db);
+  #pragma unroll
+        for (int i = 0; i < DQ; ++i) dvf[i] = vread(1, DB - DQ + i);
+      }
+      dpf[0] = pf[1][0];
+      dpf[1] = pf[1][1];
     };
 
     // Tile kb lives in stage kb % 2; tile kb + 1's loads go out when tile kb's
@@ -630,57 +709,70 @@ attn_fwd_kernel(FwdParams p) {
       // Group 1's partial O^T (lane-major, DB x 16 values per lane), running max
       // and row sums go through the idle stages; group 0 merges them into its own:
       // m = max(m0, m1), O = O0 2^(m0 - m) + O1 2^(m1 - m), l likewise.
-      float* xo = reinterpret_cast<float*>(rw < 2 ? smem0 : smem1) + (rw & 1) * (DB * 16 * 64);
-      float* xm = reinterpret_cast<float*>(smem2) + rw * 128;
+      float* xo = reinterpret_cast<float*>(rw < 2 ? smem0 : smem1) + (rw & 1) * (DB * 8 * 64);
+      float* xm = reinterpret_cast<float*>(smem2) + rw * 256;
       if (grp) {
   #pragma unroll
         for (int db = 0; db < DB; ++db)
   #pragma unroll
-          for (int r = 0; r < 16; ++r) xo[(db * 16 + r) * 64 + lane] = acc_o[db][r];
-        xm[lane] = m_run;
-        xm[64 + lane] = l_run;
+          for (int qb = 0; qb < 2; ++qb)
+  #pragma unroll
+            for (int r = 0; r < 4; ++r) xo[(db * 8 + qb * 4 + r) * 64 + lane] = acc_o[qb].at(db, r);
+  #pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+          xm[qb * 128 + lane] = m_run[qb];
+          xm[qb * 128 + 64 + lane] = l_run[qb];
+        }
       }
       __syncthreads();
       if (!grp) {
-        const float m1 = xm[lane], l1 = xm[64 + lane];
-        const float mm = fmaxf(m_run, m1);
-        const float a0 = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - mm);
-        const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mm);
-        m_run = mm;
-        l_run = l_run * a0 + l1 * a1;
   #pragma unroll
-        for (int db = 0; db < DB; ++db)
+        for (int qb = 0; qb < 2; ++qb) {
+          const float m1 = xm[qb * 128 + lane], l1 = xm[qb * 128 + 64 + lane];
+          const float mm = fmaxf(m_run[qb], m1);
+          const float a0 = m_run[qb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[qb] - mm);
+          const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mm);
+          m_run[qb] = mm;
+          l_run[qb] = l_run[qb] * a0 + l1 * a1;
   #pragma unroll
-          for (int r = 0; r < 16; ++r) acc_o[db][r] = acc_o[db][r] * a0 + xo[(db * 16 + r) * 64 + lane] * a1;
+          for (int db = 0; db < DB; ++db) {
+            floatx4 x = acc_o[qb].get(db);
+  #pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = x[r] * a0 + xo[(db * 8 + qb * 4 + r) * 64 + lane] * a1;
+            acc_o[qb].set(db, x);
+          }
+        }
       }
       __syncthreads();  // the next pass reloads the stages
     }
 
     // ---- epilogue ----
-    const float l_tot = sum_xor32(l_run);
-    if ((!SPLIT || grp == 0) && qrow < p.Sq) {
-    const float sev = ldexp1(ev);
-    const int64_t orow = ((int64_t)bh * p.Sq + qrow) * p.D;
+    if (!SPLIT || grp == 0) {
+      const float sev = ldexp1(ev);
   #pragma unroll
-    for (int db = 0; db < DB; ++db)
+      for (int qb = 0; qb < 2; ++qb) {
+        const float l_tot = sum_xor32(sum_xor16(l_run[qb]));
+        if (qrow[qb] >= p.Sq) continue;
+        const int64_t orow = ((int64_t)bh * p.Sq + qrow[qb]) * p.D;
   #pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int d = db * 32 + 8 * rq + 4 * fk;
-        if (d >= p.D) continue;
-        float y[4];
+        for (int db = 0; db < DB; ++db) {
+          const int d = db * 16 + 4 * fk;
+          if (d >= p.D) continue;
+          float y[4];
   #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          y[e] = l_tot > 0.f ? acc_o[db][4 * rq + e] / l_tot : 0.f;
-          if constexpr (DROP) y[e] *= p.drop_scale;
+          for (int e = 0; e < 4; ++e) {
+            y[e] = l_tot > 0.f ? acc_o[qb].at(db, e) / l_tot : 0.f;
+            if constexpr (DROP) y[e] *= p.drop_scale;
+          }
+          *reinterpret_cast<uint2*>(p.o + orow + d) =
+              make_uint2(pack_bf16(y[0] * sev, y[1] * sev), pack_bf16(y[2] * sev, y[3] * sev));
+          if (p.o16) *reinterpret_cast<uint2*>(p.o16 + orow + d) = make_uint2(pack_f16(y[0], y[1]), pack_f16(y[2], y[3]));
         }
-        *reinterpret_cast<uint2*>(p.o + orow + d) =
-            make_uint2(pack_bf16(y[0] * sev, y[1] * sev), pack_bf16(y[2] * sev, y[3] * sev));
-        if (p.o16) *reinterpret_cast<uint2*>(p.o16 + orow + d) = make_uint2(pack_f16(y[0], y[1]), pack_f16(y[2], y[3]));
+        // lse in log2 units (v_log_f32); rows that see no key get +inf so the
+        // backward's exp2(logit - lse) is 0 there
+        if (p.lse && fk == 0)
+          p.lse[(int64_t)bh * p.Sq + qrow[qb]] = (l_tot > 0.f) ? m_run[qb] + __builtin_amdgcn_logf(l_tot) : INFINITY;
       }
-    // lse in log2 units (v_log_f32); rows that see no key get +inf so the
-    // backward's exp2(logit - lse) is 0 there
-    if (p.lse && fk == 0)
-      p.lse[(int64_t)bh * p.Sq + qrow] = (l_tot > 0.f) ? m_run + __builtin_amdgcn_logf(l_tot) : INFINITY;
     }
   }
 }
@@ -710,6 +802,19 @@ WsLayout fwd_ws(int64_t B, int64_t H, int64_t Hkv, int64_t Sq, int64_t Sk, int64
   return w;
 }
 
+// Compute units of the current device.
+int64_t num_cus() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 template <int DP, int NW>
 int launch_fwd_nw(const FwdParams& p, bool causal, bool has_bias, bool split, dim3 grid, hipStream_t st) {
   // dropout kernels exist for 4-wave blocks only (the launcher picks those)
@@ -725,13 +830,25 @@ int launch_fwd_nw(const FwdParams& p, bool causal, bool has_bias, bool split, di
     }
   } else if (split) {
     if constexpr (NW == 8 && DP <= 128) {
-      if (!p.conv_k) attn_fwd_kernel<DP, 8, true, false, false, true, true><<<grid, 512, 0, st>>>(p);
-      else attn_fwd_kernel<DP, 8, true, false, false, true><<<grid, 512, 0, st>>>(p);
+#define SPLIT_FORM(C, HB)                                                                    \
+  if (!p.conv_k) attn_fwd_kernel<DP, 8, C, HB, false, true, true><<<grid, 512, 0, st>>>(p); \
+  else attn_fwd_kernel<DP, 8, C, HB, false, true><<<grid, 512, 0, st>>>(p)
+      if (causal) {
+        if (has_bias) { SPLIT_FORM(true, true); } else { SPLIT_FORM(true, false); }
+      } else {
+        if (has_bias) { SPLIT_FORM(false, true); } else { SPLIT_FORM(false, false); }
+      }
+#undef SPLIT_FORM
     }
-  } else if (!p.conv_k) {  // bf16 K rows (no bias rows, no dropout, head dim <= 128)
+  } else if (!p.conv_k) {  // bf16 K rows (no dropout, head dim <= 128)
     if constexpr (DP <= 128) {
-      if (causal) attn_fwd_kernel<DP, NW, true, false, false, false, true><<<grid, NW * 64, 0, st>>>(p);
-      else attn_fwd_kernel<DP, NW, false, false, false, false, true><<<grid, NW * 64, 0, st>>>(p);
+      if (causal) {
+        if (has_bias) attn_fwd_kernel<DP, NW, true, true, false, false, true><<<grid, NW * 64, 0, st>>>(p);
+        else attn_fwd_kernel<DP, NW, true, false, false, false, true><<<grid, NW * 64, 0, st>>>(p);
+      } else {
+        if (has_bias) attn_fwd_kernel<DP, NW, false, true, false, false, true><<<grid, NW * 64, 0, st>>>(p);
+        else attn_fwd_kernel<DP, NW, false, false, false, false, true><<<grid, NW * 64, 0, st>>>(p);
+      }
     }
   } else if (causal) {
     if (has_bias) attn_fwd_kernel<DP, NW, true, true, false><<<grid, NW * 64, 0, st>>>(p);
@@ -748,7 +865,7 @@ int launch_fwd_nw(const FwdParams& p, bool causal, bool has_bias, bool split, di
 // more queries and win once there are enough of them: measured on MI355X
 // (causal, D = 128) at S = 16384, B = 1, H = 16 (1024 blocks of 8 waves, 962 vs
 // 925 TFLOPS) and at S = 4096, B = 2, H = 16 (512 blocks, 632 vs 611). With at
-// most ~1.5 rounds of 8-wave blocks a causal grid is better served by 4-wave
+// most ~1.5 rounds of 8-wave blocks a causal grid is better served by 128-row
 // blocks that pair a heavy and a light query tile (S = 4096, B = 1: 563 vs 476).
 // Head dim 256 always uses 4-wave blocks (one wave per SIMD, 512 registers).
 template <int DP>
@@ -759,12 +876,13 @@ int launch_fwd_dp(FwdParams p, bool causal, bool has_bias, hipStream_t st, int n
   // balances many rounds); otherwise as measured above
   const bool pair = causal && tiles4 >= 2 * p.B * p.H && tiles8 < 384 && nw_override <= 0 &&
                     getenv("TBF16_ATTN_NOPAIR") == nullptr;
-  // the paired grid runs as split-key 8-wave blocks where those exist (no bias
-  // rows, no dropout, head dim <= 128); TBF16_ATTN_SPLIT=0 / 1 turns that off / on
-  // for any causal grid (benchmarking)
+  // the paired grid, and any grid whose 128-row tiles are no more than the CUs, run as
+  // split-key 8-wave blocks where those exist (no dropout, head dim <= 128): two waves
+  // per SIMD instead of one (key-padding mask, 24 heads, S = 1111, D = 64: kernel 36.6 ->
+  // 29.2 us); TBF16_ATTN_SPLIT=0 / 1 turns that off / on for any grid (benchmarking)
   const char* sv = getenv("TBF16_ATTN_SPLIT");
-  const bool split_ok = causal && DP <= 128 && !has_bias && !p.drop_thr && nw_override <= 0;
-  const bool split = split_ok && (sv ? atoi(sv) != 0 : pair);
+  const bool split_ok = DP <= 128 && !p.drop_thr && nw_override <= 0;
+  const bool split = split_ok && (sv ? atoi(sv) != 0 : pair || tiles4 <= num_cus());
   int nw = nw_override > 0 ? nw_override : pair ? 4 : (tiles8 >= 128 ? 8 : 4);
   if (DP > 128 || p.drop_thr) nw = 4;
   if (split) nw = 8;
@@ -815,10 +933,10 @@ extern "C" int tbf16_attn_fwd(const void* q, const void* k, const void* v, int64
   float* pk = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + w.off_k);
   float* pv = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + w.off_v);
   // S^T = K Q^T on k's and q's own bf16 rows where the head dim is a whole
-  // staging width and there are no bias rows or dropout (TBF16_ATTN_KF16 forces
+  // staging width and there is no dropout (TBF16_ATTN_KF16 forces
   // the fp16 k16 copy, for benchmarking); then q's and k's maxima are needed
   // only for the exponents the caller asks for
-  const bool kbf = D == w.DP && w.DP <= 128 && !bias && dropout_p == 0.f && k_strides[2] < ((int64_t)1 << 23) &&
+  const bool kbf = D == w.DP && w.DP <= 128 && dropout_p == 0.f && k_strides[2] < ((int64_t)1 << 23) &&
                    getenv("TBF16_ATTN_KF16") == nullptr;
   const bool derive_a = !kbf || exps != nullptr;
   {
