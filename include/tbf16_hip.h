@@ -94,6 +94,17 @@ int tbf16_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w
                  const float* ws, const void* bias, void* y, int64_t ldy, int t, int l1, int cfg, void* workspace,
                  void* stream);
 
+/* tbf16_linear for any N (a vocabulary with an added token): w16, ws and bias have N rows,
+ * y's rows ldy >= N rounded up to 8 elements (a multiple of 8), of which those past N
+ * are written with values to leave out. workspace: tbf16_linear_ws_bytes(M, K, N rounded
+ * up to 8, -1). The same for tbf16_gemm_f16. No counterpart in the reference, whose
+ * callers pad (tbf16/ops.py:145-178). */
+int tbf16_linear_any_n(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N, int64_t ldw,
+                       const float* ws, const void* bias, void* y, int64_t ldy, int t, int l1, void* workspace,
+                       void* stream);
+int tbf16_gemm_f16_any_n(const void* a16, int64_t M, int64_t K, int64_t lda, const float* sa, const void* b16, int64_t N,
+                         int64_t ldb, const float* sb, const void* bias, void* y, int64_t ldy, void* stream);
+
 /* tbf16_linear without a workspace argument and without allocating anything: the
  * workspace lives in a static device array of TBF16_NOALLOC_SCRATCH_BYTES per GPU
  * (12 MiB, held until the process ends). No counterpart in the reference: it is

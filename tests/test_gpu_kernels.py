@@ -191,6 +191,25 @@ def test_linear_dispatch_splits_bit_exact(dev, M, N, K):
         assert torch.equal(y.cpu(), want), name
 
 
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K", [(2, 1, 64), (17, 9, 4096), (100, 515, 200), (300, 2049, 520), (64, 32001, 64), (2, 257, 16392)])
+def test_linear_any_n(dev, M, N, K, bias):
+    """N that is no multiple of 8 without padding the weight, scale and bias views that
+    start at any element, split and unsplit: exact products, and the same from
+    already-quantised rows."""
+    g = torch.Generator().manual_seed(N)
+    a, b = torch.randint(-1, 2, (M, K), generator=g), torch.randint(-1, 2, (N, K), generator=g)
+    sw = torch.ldexp(torch.ones(N + 1), torch.randint(-3, 4, (N + 1,), generator=g).float())[1:]
+    bb = torch.randint(-8, 9, (N + 1,), generator=g).bfloat16()[1:] if bias else None
+    want = (a @ b.t()).double() * sw.double() + (bb.double() if bias else 0.0)
+    wide = lambda t: torch.cat([t[:1], t]).to(dev)[1:]  # noqa: E731  (a view one element into its storage)
+    args = (b.half().to(dev), wide(sw), wide(bb) if bias else None)
+    y = tbf16.scaled_linear(a.bfloat16().to(dev), *args)
+    assert y.shape == (M, N) and torch.equal(y.cpu(), want.bfloat16())
+    y = ops.linear_q(a.half().to(dev), torch.ones(M, device=dev), *args)
+    assert y.shape == (M, N) and torch.equal(y.cpu(), want.bfloat16())
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (200, 768, 2560), (300, 264, 3040)])
 def test_linear_split_k(dev, M, N, K):
     """K split over two blocks per tile (what tbf16_linear picks where the tiles leave

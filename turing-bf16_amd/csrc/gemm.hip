@@ -663,12 +663,13 @@ __device__ __forceinline__ void store_tile16(const floatx4 (&acc)[TN / 16][TM / 
 // Loads of tiles past the last go to a resource of length 0 (no memory traffic, zeros
 // nobody reads). The fp32 additions run over k in ascending order.
 // HA, FB: 16-row and 16-column blocks per wave and half (BM = 64 HA, BN = 128 FB).
-// part / kt_per: split K, as gemm_kernel.
+// part / kt_per: split K, as gemm_kernel. NB <= N: rows of b, N rounded up to 8 (the
+// columns past NB are zeros plus the last bias, for the caller to leave out).
 template <int HA, int FB, int S, bool KEVEN>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void pingpong_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const float* __restrict__ a_sinv, const uint16_t* __restrict__ B,
     int64_t ldb, const float* __restrict__ b_sinv, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C,
-    int64_t ldc, int M, int N, int K_all, float* __restrict__ part, int kt_per) {
+    int64_t ldc, int M, int N, int K_all, float* __restrict__ part, int kt_per, int NB) {
   constexpr int BM = 64 * HA, BN = 128 * FB, RA = 16 * HA, CB = 16 * FB;
   constexpr int AB = 4 * HA, BB = 8 * FB;  // 1 KB blocks (8 rows of 128 bytes) of a half tile
   constexpr int AL = (AB + 7) / 8, BL = BB / 8;
@@ -706,8 +707,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // the epilogue's factors, one a thread, loaded ahead of the direct loads (rows past M
   // and columns past N take the last one's and are not stored)
   const int fc = tid - 256;
-  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, N - 1)];
-  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), N - 1)] : (uint16_t)0;
+  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, NB - 1)];
+  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), NB - 1)] : (uint16_t)0;
 
   // direct loads: lane l of the load of 1 KB block b lands at row 8 b + l / 8 of the
   // half tile, physical chunk l % 8, so it fetches the logical chunk `chunk` (the XOR
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const BufRes ares =
       make_res(A + (int64_t)m0 * lda + kbase, min<int64_t>((int64_t)(M - m0) * lda * 2 - kbase * 2, 0x7fffffff));
   const BufRes bres =
-      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(N - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
+      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(NB - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
   const int KT = (K + 63) / 64;
   auto aload = [&](int h, uint8_t* half, int kt) {
     const BufRes rt{ares.lo, ares.hi, kt < KT ? ares.bytes : 0};
@@ -865,12 +866,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // The two groups' fp32 sums are added even + odd: another order than k ascending,
 // the same for every launch. part / kt_per: split K, as gemm_kernel. R <= BN: columns
 // per block (a multiple of 8); below BN the weights of a single row of tiles are
-// spread over every CU, the rest of the tile is zeros.
+// spread over every CU, the rest of the tile is zeros. NB: as pingpong_kernel.
 template <int RM, int RN, int S, bool KEVEN>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void ksplit_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const float* __restrict__ a_sinv, const uint16_t* __restrict__ B,
     int64_t ldb, const float* __restrict__ b_sinv, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C,
-    int64_t ldc, int M, int N_all, int K_all, float* __restrict__ part, int kt_per, int R) {
+    int64_t ldc, int M, int N_all, int K_all, float* __restrict__ part, int kt_per, int R, int NB) {
   constexpr int BM = 32 * RM, BN = 32 * RN, TM = 16 * RM, TN = 16 * RN;
   constexpr int STG = (BM + BN) * 128, NL = (BM + BN) / 64, AL = BM / 64;  // loads per wave and tile; the first AL are A's
   constexpr int XB = RM / 2 * RN * 16 * 64;  // bytes of the half sub-tile a wave hands over
@@ -901,8 +902,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // the epilogue's factors (see pingpong_kernel)
   const int fc = tid - 256;
-  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, N - 1)];
-  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), N - 1)] : (uint16_t)0;
+  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, NB - 1)];
+  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), NB - 1)] : (uint16_t)0;
 
   // direct loads: 1 KB block wave + 8 i of the stage (rows of A, then of B)
   const int chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
@@ -915,7 +916,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const BufRes ares =
       make_res(A + (int64_t)m0 * lda + kbase, min<int64_t>((int64_t)(M - m0) * lda * 2 - kbase * 2, 0x7fffffff));
   const BufRes bres =
-      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(N - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
+      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(min(N, NB) - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
   const int KT = (K + 63) / 64;
   auto load = [&](uint8_t* stage, int kt) {
     const BufRes ra{ares.lo, ares.hi, kt < KT ? ares.bytes : 0}, rb{bres.lo, bres.hi, kt < KT ? bres.bytes : 0};
@@ -1041,7 +1042,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
                                                             const float* __restrict__ a_sinv,
                                                             const float* __restrict__ b_sinv,
                                                             const uint16_t* __restrict__ bias,
-                                                            uint16_t* __restrict__ C, int64_t ldc, int M, int N) {
+                                                            uint16_t* __restrict__ C, int64_t ldc, int M, int N, int NB) {
   const int ng = N >> 3;
   const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (g >= (int64_t)M * ng) return;
@@ -1062,10 +1063,23 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   float sa;
   if constexpr (A_BF16) sa = ldexp1(-a_exp[m]);
   else sa = a_sinv[m];
-  const float4 s0 = *reinterpret_cast<const float4*>(b_sinv + n), s1 = *reinterpret_cast<const float4*>(b_sinv + n + 4);
+  float4 s0, s1;
   uint4 bw = make_uint4(0, 0, 0, 0);
-  if (bias) bw = make_uint4(*reinterpret_cast<const uint32_t*>(bias + n), *reinterpret_cast<const uint32_t*>(bias + n + 2),
-                            *reinterpret_cast<const uint32_t*>(bias + n + 4), *reinterpret_cast<const uint32_t*>(bias + n + 6));
+  if (n + 8 <= NB) {
+    __builtin_memcpy(&s0, b_sinv + n, 16);
+    __builtin_memcpy(&s1, b_sinv + n + 4, 16);
+    if (bias) __builtin_memcpy(&bw, bias + n, 16);
+  } else {  // the last columns of an N that is no multiple of 8
+    float sv[8];
+    uint16_t bv[8];
+    for (int e = 0; e < 8; ++e) {
+      sv[e] = b_sinv[min(n + e, NB - 1)];
+      bv[e] = bias ? bias[min(n + e, NB - 1)] : (uint16_t)0;
+    }
+    s0 = make_float4(sv[0], sv[1], sv[2], sv[3]);
+    s1 = make_float4(sv[4], sv[5], sv[6], sv[7]);
+    __builtin_memcpy(&bw, bv, 16);
+  }
   const uint4 out = make_uint4(pack_bf16(fmaf(lo.x * sa, s0.x, bf16_lo(bw.x)), fmaf(lo.y * sa, s0.y, bf16_hi(bw.x))),
                                pack_bf16(fmaf(lo.z * sa, s0.z, bf16_lo(bw.y)), fmaf(lo.w * sa, s0.w, bf16_hi(bw.y))),
                                pack_bf16(fmaf(hi.x * sa, s1.x, bf16_lo(bw.z)), fmaf(hi.y * sa, s1.y, bf16_hi(bw.z))),
@@ -1632,12 +1646,15 @@ void launch_cfg(bool even, unsigned blocks, const uint16_t* a, int64_t lda, cons
 }
 
 // part / splits: split K over `splits` blocks per tile (tile configurations only),
-// the fp32 partial sums in part (splits x M x N), then splitk_reduce_kernel.
+// the fp32 partial sums in part (splits x M x N), then splitk_reduce_kernel. NB: rows
+// of b where N is their number rounded up to 8 (the ping-pong configurations).
 template <bool A_BF16>
 int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const float* a_sinv, const void* B,
                 int64_t ldb, const float* b_sinv, const void* bias, void* C, int64_t ldc, int64_t M, int64_t N,
-                int64_t K, hipStream_t st, float* part = nullptr, int splits = 1) {
+                int64_t K, hipStream_t st, float* part = nullptr, int splits = 1, int64_t NB = 0) {
   const int bm = kCfgs[cfg].bm, bn = kCfgs[cfg].bn;
+  if (NB == 0) NB = N;
+  TB_CHECK(NB == N || kCfgs[cfg].pingpong, "gemm: configuration %d takes N %% 8 == 0", cfg);
   TB_CHECK(splits == 1 || (part != nullptr && splits > 1 && !kCfgs[cfg].skinny && !kCfgs[cfg].stream &&
                            (splits - 1) * cdiv(cdiv(K, kCfgs[cfg].bk), splits) * kCfgs[cfg].bk < K),
            "gemm: split K needs a tile configuration, a partial-sum buffer and k tiles for every split");
@@ -1700,10 +1717,10 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
     const dim3 grid(g, part ? (unsigned)splits : 1u);                                                  \
     if (even)                                                                                          \
       pingpong_kernel<HA_, FB_, S_, true><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, \
-                                                            M, N, K, part, kt_per);                    \
+                                                            M, N, K, part, kt_per, NB);                \
     else                                                                                               \
       pingpong_kernel<HA_, FB_, S_, false><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, \
-                                                             M, N, K, part, kt_per);                   \
+                                                             M, N, K, part, kt_per, NB);               \
   }
     case 20: PINGPONG(4, 2, 2); break;
     case 21: PINGPONG(3, 2, 2); break;
@@ -1716,10 +1733,10 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
     const dim3 grid(g, part ? (unsigned)splits : 1u);                                                       \
     if (even)                                                                                               \
       ksplit_kernel<RM_, RN_, S_, true><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, M, \
-                                                              N, K, part, kt_per, rows);                    \
+                                                              N, K, part, kt_per, rows, NB);                \
     else                                                                                                    \
       ksplit_kernel<RM_, RN_, S_, false><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, M, \
-                                                               N, K, part, kt_per, rows);                   \
+                                                               N, K, part, kt_per, rows, NB);               \
   }
     case 25: KSPLIT(8, 4, 3); break;
     case 26: KSPLIT(6, 4, 3); break;
@@ -1738,7 +1755,7 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
   if (part) {
     const int64_t groups = M * (N / 8);
     splitk_reduce_kernel<A_BF16><<<(unsigned)cdiv(groups, 256), 256, 0, st>>>(part, splits, a_exp, a_sinv, b_sinv, bi, c,
-                                                                             ldc, (int)M, (int)N);
+                                                                             ldc, (int)M, (int)N, (int)NB);
     TB_LAUNCH_CHECK("gemm split-K reduction");
   }
   return 0;
@@ -1825,7 +1842,7 @@ LinearWs fused_ws(int64_t M, int64_t K, int64_t N, int cfg) {
 
 int linear_into(const LinearWs& w, const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N,
                 int64_t ldw, const float* ws, const void* bias, void* y, int64_t ldy, int t, int l1, uint8_t* wsp,
-                hipStream_t st) {
+                hipStream_t st, int64_t NB = 0) {
   int32_t* exps = reinterpret_cast<int32_t*>(wsp + w.exps);
   float* part = w.splits > 1 ? reinterpret_cast<float*>(wsp + w.part) : nullptr;
   if (!w.q16) {
@@ -1837,7 +1854,7 @@ int linear_into(const LinearWs& w, const void* x, int64_t M, int64_t K, int64_t 
   float* sinv = reinterpret_cast<float*>(wsp + w.sinv);
   void* x16 = wsp + w.x16;
   if (int rc = launch_quantize_rows(x, M, K, ldx, t, l1, x16, K, sinv, exps, st)) return rc;
-  return launch_gemm<false>(w.cfg, x16, K, nullptr, sinv, w16, ldw, ws, bias, y, ldy, M, N, K, st, part, w.splits);
+  return launch_gemm<false>(w.cfg, x16, K, nullptr, sinv, w16, ldw, ws, bias, y, ldy, M, N, K, st, part, w.splits, NB);
 }
 }  // namespace
 
@@ -1857,6 +1874,18 @@ extern "C" int tbf16_linear(const void* x, int64_t M, int64_t K, int64_t ldx, co
   if (M == 0 || N == 0) return 0;
   return linear_into(linear_ws(M, K, N, cfg), x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1,
                      static_cast<uint8_t*>(workspace), as_stream(stream));
+}
+
+extern "C" int tbf16_linear_any_n(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N,
+                                  int64_t ldw, const float* ws, const void* bias, void* y, int64_t ldy, int t, int l1,
+                                  void* workspace, void* stream) {
+  const int64_t Np = cdiv(N, 8) * 8;
+  if (int rc = check_gemm("linear_any_n", M, Np, K, x, ldx, w16, ldw, nullptr, nullptr, y, ldy)) return rc;
+  TB_CHECK(ws != nullptr && aligned4(ws), "linear_any_n: bad scales");
+  TB_CHECK((workspace != nullptr && aligned16(workspace)) || M == 0, "linear_any_n: workspace missing or misaligned");
+  if (M == 0 || N == 0) return 0;
+  return linear_into(linear_ws(M, K, Np, -1), x, M, K, ldx, w16, Np, ldw, ws, bias, y, ldy, t, l1,
+                     static_cast<uint8_t*>(workspace), as_stream(stream), N);
 }
 
 // ---- tbf16_linear_noalloc: the workspace in a static device array ---------------
@@ -1941,4 +1970,16 @@ extern "C" int tbf16_gemm_f16(const void* a16, int64_t M, int64_t K, int64_t lda
   if (M == 0 || N == 0) return 0;
   return launch_gemm<false>(cfg < 0 ? pick_f16(M, N, K).cfg : cfg, a16, lda, nullptr, sa, b16, ldb, sb, bias, y, ldy, M, N,
                             K, as_stream(stream));
+}
+
+extern "C" int tbf16_gemm_f16_any_n(const void* a16, int64_t M, int64_t K, int64_t lda, const float* sa, const void* b16,
+                                    int64_t N, int64_t ldb, const float* sb, const void* bias, void* y, int64_t ldy,
+                                    void* stream) {
+  const int64_t Np = cdiv(N, 8) * 8;
+  if (int rc = check_gemm("gemm_f16_any_n", M, Np, K, a16, lda, b16, ldb, nullptr, nullptr, y, ldy)) return rc;
+  TB_CHECK(sb != nullptr && aligned4(sb), "gemm_f16_any_n: bad scales");
+  TB_CHECK(sa != nullptr || M == 0, "gemm_f16_any_n: sa missing");
+  if (M == 0 || N == 0) return 0;
+  return launch_gemm<false>(pick_f16(M, Np, K).cfg, a16, lda, nullptr, sa, b16, ldb, sb, bias, y, ldy, M, Np, K,
+                            as_stream(stream), nullptr, 1, N);
 }

@@ -41,6 +41,8 @@ _SIGS = {
     "tbf16_quantize_cols_t": (I, [P, I64, I64, I64, I, P, P, I64, P, P, I64, P]),
     "tbf16_linear_ws_bytes": (SZ, [I64, I64, I64, I]),
     "tbf16_linear": (I, [P, I64, I64, I64, P, I64, I64, P, P, P, I64, I, I, I, P, P]),
+    "tbf16_linear_any_n": (I, [P, I64, I64, I64, P, I64, I64, P, P, P, I64, I, I, P, P]),
+    "tbf16_gemm_f16_any_n": (I, [P, I64, I64, I64, P, P, I64, I64, P, P, P, I64, P]),
     "tbf16_linear_noalloc": (I, [P, I64, I64, I64, P, I64, I64, P, P, P, I64, I, I, I, P]),
     "tbf16_linear_exps": (I, [P, I64, I64, I64, P, P, I64, I64, P, P, P, I64, I, P]),
     "tbf16_gemm_f16": (I, [P, I64, I64, I64, P, P, I64, I64, P, P, P, I64, I, P]),

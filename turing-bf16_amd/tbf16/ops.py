@@ -113,7 +113,9 @@ def _bias_bf16(bias, N, device):
 
 
 def _prep_gemm_operands(x2, w16, w_sinv, bias):
-    """Pads K and N to multiples of 8 where needed (copies only then)."""
+    """Pads K to a multiple of 8 where needed (copies only then), and N where a tile
+    configuration is pinned: the dispatcher's kernels take any N and rows of y padded to
+    Np, N rounded up to 8."""
     M, K = x2.shape
     N = w16.shape[0]
     if w16.shape[1] != K:
@@ -125,7 +127,7 @@ def _prep_gemm_operands(x2, w16, w_sinv, bias):
     ws = w_sinv.float().contiguous()
     b = _bias_bf16(bias, N, x2.device)
     Np = N + (-N) % 8
-    if Np != N:
+    if Np != N and _GEMM_CFG >= 0:
         w16 = F.pad(w16, (0, 0, 0, Np - N))
         ws = F.pad(ws, (0, Np - N), value=1.0)
         if b is not None:
@@ -154,8 +156,12 @@ def _linear(x2, w16, w_sinv, bias, t, l1):
     M, Kp = x2.shape
     y = torch.empty((M, Np), device=x2.device, dtype=torch.bfloat16)
     work = torch.empty((_linear_ws_bytes(x2.device, M, Kp, Np),), device=x2.device, dtype=torch.uint8)
-    launch("tbf16_linear", x2, ptr(x2), M, Kp, x2.stride(0), ptr(w16), Np, w16.stride(0), ptr(ws), ptr(b), ptr(y),
-           y.stride(0), int(t), int(l1), _GEMM_CFG, ptr(work))
+    if w16.shape[0] != Np:
+        launch("tbf16_linear_any_n", x2, ptr(x2), M, Kp, x2.stride(0), ptr(w16), N, w16.stride(0), ptr(ws), ptr(b), ptr(y),
+               Np, int(t), int(l1), ptr(work))
+    else:
+        launch("tbf16_linear", x2, ptr(x2), M, Kp, x2.stride(0), ptr(w16), Np, w16.stride(0), ptr(ws), ptr(b), ptr(y),
+               Np, int(t), int(l1), _GEMM_CFG, ptr(work))
     return y if Np == N else y[:, :N]
 
 
@@ -187,7 +193,10 @@ def linear_q(x16, x_sinv, w16, w_sinv, bias=None):
     x16, w16, ws, b, N, Np = _prep_gemm_operands(x16, w16, w_sinv, bias)
     sa = x_sinv.float().contiguous()
     y = torch.empty((M, Np), device=x16.device, dtype=torch.bfloat16)
-    if M:
+    if M and w16.shape[0] != Np:
+        launch("tbf16_gemm_f16_any_n", x16, ptr(x16), M, x16.shape[1], x16.stride(0), ptr(sa), ptr(w16), N,
+               w16.stride(0), ptr(ws), ptr(b), ptr(y), Np)
+    elif M:
         launch("tbf16_gemm_f16", x16, ptr(x16), M, x16.shape[1], x16.stride(0), ptr(sa), ptr(w16), Np, w16.stride(0),
                ptr(ws), ptr(b), ptr(y), y.stride(0), _GEMM_CFG)
     return y if Np == N else y[:, :N]
