@@ -60,12 +60,6 @@ int tbf16_quantize_rows(const void* x, int64_t R, int64_t K, int64_t ldx, int t,
 int tbf16_quantize_rows_t(const void* x, int64_t R, int64_t K, int64_t ldx, int t, void* yT, int64_t ldyT,
                           float* s_inv, int32_t* exps_ws, void* stream);
 
-/* tbf16_quantize_rows (max scales) and tbf16_quantize_rows_t in one call: y16 (R, K),
- * row stride ldy, and yT (K, R), row stride ldyT. For the training forward, whose own
- * product reads y16 and whose dW reads yT (tbf16/autograd.py:60-68). */
-int tbf16_quantize_rows_both(const void* x, int64_t R, int64_t K, int64_t ldx, int t, void* y16, int64_t ldy, void* yT,
-                             int64_t ldyT, float* s_inv, int32_t* exps_ws, void* stream);
-
 /* Column quantisation: amax[c] = max_r |x[r,c] * row_mul[r]|, y = fp16((x * row_mul)
  * * 2^p[c]), s_inv[c] = 2^-p[c]; row_mul (R,) fp32 powers of two or NULL. The fp16
  * result is written transposed: yT (K, R), row stride ldyT >= R.
@@ -136,6 +130,23 @@ int tbf16_linear_exps(const void* x, int64_t M, int64_t K, int64_t ldx, const in
  * small_kernels.cu:289-302) and _scaled_mm (tbf16/autograd.py:49-55). */
 int tbf16_gemm_f16(const void* a16, int64_t M, int64_t K, int64_t lda, const float* sa, const void* b16, int64_t N,
                    int64_t ldb, const float* sb, const void* bias, void* y, int64_t ldy, int cfg, void* stream);
+
+/* The training linear (tbf16/autograd.py:58-90), its scaling passes and products in one
+ * call each way; same values as the single entry points above.
+ * Forward: x16 (M, K), xT (K, ldT), sx (M,) as tbf16_quantize_rows / _t of x at t, the
+ * weight w bf16 (N, K) by rows at t, y = bf16(x w^T + bias); K and N multiples of 8.
+ * x NULL: x16 and sx are given (an activation that several layers read).
+ * Backward: dx = dY W from dY rows by L1 norm at t_rows and W columns at t_w; dw = dY^T X
+ * from dY's columns (with sx folded in) at t_dy and xT; db = the columns' fp32 sums, bf16.
+ * Each of dx (M, K), dw (N, K), db (N,) may be NULL. */
+size_t tbf16_train_linear_fwd_ws_bytes(int64_t N, int64_t K);
+int tbf16_train_linear_fwd(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w, int64_t N, int64_t ldw,
+                           const void* bias, int t, void* x16, void* xT, int64_t ldT, float* sx, int32_t* exps_ws,
+                           void* y, int64_t ldy, void* ws, int64_t ws_bytes, void* stream);
+size_t tbf16_train_linear_bwd_ws_bytes(int64_t M, int64_t N, int64_t K);
+int tbf16_train_linear_bwd(const void* dy, int64_t M, int64_t N, int64_t lddy, const void* w, int64_t K, int64_t ldw,
+                           const void* xT, int64_t ldT, const float* sx, int t_w, int t_rows, int t_dy, void* dx,
+                           void* dw, void* db, void* ws, int64_t ws_bytes, void* stream);
 
 /* M = 1: y[n] = bf16((sum_k x[k] * w16[n,k]) * ws[n] + bias[n]) in fp32.
  * Replaces gemv (tbf16/csrc/small_kernels.cu:304-315, kernel :107-132). */

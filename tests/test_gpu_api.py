@@ -430,3 +430,44 @@ def _to_double(m):
     import copy
     d = copy.deepcopy(m).double()
     return d
+
+
+@pytest.mark.parametrize("layout", ["whole", "view"])
+@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (37, 264, 72), (130, 520, 1032), (1000, 768, 256)])
+@pytest.mark.parametrize("grads", ["xwb", "x", "w", "b", "xb"])
+def test_autograd_linear_one_call_matches_passes(dev, monkeypatch, M, K, N, grads, layout):
+    """The training linear in one native call each way against the pass-by-pass route:
+    the same bits (db: fp32 sums in another order, so within one bf16 rounding and the
+    sum's own error), for every set of wanted gradients, row strides wider than the
+    matrix, and an activation that two layers read."""
+    import tbf16.autograd as ag
+    from tbf16 import routing
+    g = torch.Generator().manual_seed(M + N)
+
+    def mat(r, c):
+        t = (torch.randn(r, c, generator=g) * torch.exp2(torch.randint(-9, 9, (r, 1), generator=g).float())).bfloat16().to(dev)
+        return torch.cat([t, t], 1)[:, :c] if layout == "view" else t
+
+    x, w1, w2, dy = mat(M, K), mat(N, K), mat(N, K), mat(M, N)
+    b = torch.randn(N, generator=g).bfloat16().to(dev)
+
+    def run():
+        routing.activations.clear()
+        xs, ws1, ws2, bs = (t.detach().requires_grad_(c in grads) for t, c in ((x, "x"), (w1, "w"), (w2, "w"), (b, "b")))
+        y1, y2 = ag.linear(xs, ws1, bs), ag.linear(xs, ws2, bs)
+        leaves = [t for t in (xs, ws1, ws2, bs) if t.requires_grad]
+        out = [y1.detach(), y2.detach()]
+        for y in (y1, y2):
+            out += [t for t in torch.autograd.grad(y, leaves, dy, allow_unused=True) if t is not None]
+        return out
+
+    got = run()
+    monkeypatch.setattr(ag, "_one_call", lambda *a: False)
+    want = run()
+    assert len(got) == len(want)
+    for a, e in zip(got, want):
+        if a.dim() == 1:
+            bound = dy.float().abs().sum(0) * (M * 2.0 ** -24) + e.float().abs() * 2.0 ** -7
+            assert ((a.float() - e.float()).abs() <= bound).all()
+        else:
+            assert torch.equal(a, e)

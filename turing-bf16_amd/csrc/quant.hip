@@ -61,11 +61,10 @@ __global__ __launch_bounds__(256) void row_exps_kernel(const uint16_t* __restric
 
 // quantize_rows: amax pass, then y = fp16(x * 2^p) (small_kernels.cu:35-74).
 // Rows of up to kRegChunks x 512 elements are read once, into registers.
-__global__ __launch_bounds__(256) void quantize_rows_kernel(const uint16_t* __restrict__ x, int64_t R, int K,
-                                                            int64_t ldx, int t, int l1, uint16_t* __restrict__ y,
-                                                            int64_t ldy, float* __restrict__ s_inv,
-                                                            int32_t* __restrict__ exps) {
-  const int64_t row = (int64_t)blockIdx.x * kRowWaves + (threadIdx.x >> 6);
+__device__ __forceinline__ void quantize_rows_block(int64_t block, const uint16_t* __restrict__ x, int64_t R, int K,
+                                                    int64_t ldx, int t, int l1, uint16_t* __restrict__ y, int64_t ldy,
+                                                    float* __restrict__ s_inv, int32_t* __restrict__ exps) {
+  const int64_t row = block * kRowWaves + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= R) return;
   const uint16_t* xr = x + row * ldx;
@@ -94,6 +93,13 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint16_t* __re
   }
 }
 
+__global__ __launch_bounds__(256) void quantize_rows_kernel(const uint16_t* __restrict__ x, int64_t R, int K,
+                                                            int64_t ldx, int t, int l1, uint16_t* __restrict__ y,
+                                                            int64_t ldy, float* __restrict__ s_inv,
+                                                            int32_t* __restrict__ exps) {
+  quantize_rows_block(blockIdx.x, x, R, K, ldx, t, l1, y, ldy, s_inv, exps);
+}
+
 // Transposing convert: yT[c][r] = fp16((x[r][c] * rowmul[r]) * colmul[c]). Each
 // thread converts an 8 x 8 block (eight 16-byte row loads) and transposes it in
 // registers with v_perm_b32 into eight 16-byte column stores; lane l of a wave
@@ -102,14 +108,13 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint16_t* __re
 // LDS is involved. A block of four waves covers 64 rows x 256 columns. Rows in
 // [R, ldyT) are written as zeros, so that the transposed operand can be consumed with a padded contraction length.
 // rowmul = 2^rexp[r] or rm[r] (fp32) or 1; colmul = 2^cexp[c] or 1.
-__global__ __launch_bounds__(256) void transpose_convert_kernel(const uint16_t* __restrict__ x, int64_t R, int64_t K,
-                                                                int64_t ldx, const int32_t* __restrict__ rexp,
-                                                                const float* __restrict__ rm,
-                                                                const int32_t* __restrict__ cexp,
-                                                                uint16_t* __restrict__ yT, int64_t ldyT) {
+__device__ __forceinline__ void transpose_convert_block(int64_t bx, int64_t by, const uint16_t* __restrict__ x, int64_t R,
+                                                        int64_t K, int64_t ldx, const int32_t* __restrict__ rexp,
+                                                        const float* __restrict__ rm, const int32_t* __restrict__ cexp,
+                                                        uint16_t* __restrict__ yT, int64_t ldyT) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t r0 = (int64_t)blockIdx.y * 64 + 8 * (lane & 7);
-  const int64_t c0 = (int64_t)blockIdx.x * 256 + 64 * wave + 8 * (lane >> 3);
+  const int64_t r0 = by * 64 + 8 * (lane & 7);
+  const int64_t c0 = bx * 256 + 64 * wave + 8 * (lane >> 3);
   if (c0 >= K || r0 >= ldyT) return;
   // all eight loads go out before any is used; rows >= R read row R - 1 and are
   // written as zeros
@@ -141,20 +146,36 @@ __global__ __launch_bounds__(256) void transpose_convert_kernel(const uint16_t* 
   }
 }
 
+__global__ __launch_bounds__(256) void transpose_convert_kernel(const uint16_t* __restrict__ x, int64_t R, int64_t K,
+                                                                int64_t ldx, const int32_t* __restrict__ rexp,
+                                                                const float* __restrict__ rm,
+                                                                const int32_t* __restrict__ cexp,
+                                                                uint16_t* __restrict__ yT, int64_t ldyT) {
+  transpose_convert_block(blockIdx.x, blockIdx.y, x, R, K, ldx, rexp, rm, cexp, yT, ldyT);
+}
+
 // Column amax partials: each thread covers 8 adjacent columns over a chunk of
 // rows; partial[chunk][col] (small_kernels.cu:136-155 merges with atomicMax; the
-// partials keep this pass free of a zero-fill and of atomics).
-__global__ __launch_bounds__(256) void col_amax_partial_kernel(const uint16_t* __restrict__ x, const float* __restrict__ rm,
-                                                               int64_t R, int64_t K, int64_t ldx, int64_t rows_per_chunk,
-                                                               float* __restrict__ partial) {
-  const int64_t c8 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// partials keep this pass free of a zero-fill and of atomics). SUM: the fp32 column
+// sums of x itself (no row_mul) go to psum the same way.
+template <bool SUM>
+__device__ __forceinline__ void col_amax_block(int64_t bx, int64_t by, const uint16_t* __restrict__ x,
+                                               const float* __restrict__ rm, int64_t R, int64_t K, int64_t ldx,
+                                               int64_t rows_per_chunk, float* __restrict__ partial,
+                                               float* __restrict__ psum) {
+  const int64_t c8 = bx * 256 + threadIdx.x;
   if (c8 * 8 >= K) return;
-  const int64_t r0 = (int64_t)blockIdx.y * rows_per_chunk;
+  const int64_t r0 = by * rows_per_chunk;
   const int64_t r1 = min(R, r0 + rows_per_chunk);
   float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  float sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 4
   for (int64_t r = r0; r < r1; ++r) {
     const uint4 v = ldg16(x + r * ldx + c8 * 8);
+    if constexpr (SUM) {
+      sum[0] += bf16_lo(v.x); sum[1] += bf16_hi(v.x); sum[2] += bf16_lo(v.y); sum[3] += bf16_hi(v.y);
+      sum[4] += bf16_lo(v.z); sum[5] += bf16_hi(v.z); sum[6] += bf16_lo(v.w); sum[7] += bf16_hi(v.w);
+    }
     const float f = rm ? fabsf(rm[r]) : 1.f;
     m[0] = fmaxf(m[0], fabsf(bf16_lo(v.x)) * f);
     m[1] = fmaxf(m[1], fabsf(bf16_hi(v.x)) * f);
@@ -165,19 +186,31 @@ __global__ __launch_bounds__(256) void col_amax_partial_kernel(const uint16_t* _
     m[6] = fmaxf(m[6], fabsf(bf16_lo(v.w)) * f);
     m[7] = fmaxf(m[7], fabsf(bf16_hi(v.w)) * f);
   }
-  float* out = partial + (int64_t)blockIdx.y * K + c8 * 8;
+  float* out = partial + by * K + c8 * 8;
   reinterpret_cast<float4*>(out)[0] = make_float4(m[0], m[1], m[2], m[3]);
   reinterpret_cast<float4*>(out)[1] = make_float4(m[4], m[5], m[6], m[7]);
+  if constexpr (SUM) {
+    out = psum + by * K + c8 * 8;
+    reinterpret_cast<float4*>(out)[0] = make_float4(sum[0], sum[1], sum[2], sum[3]);
+    reinterpret_cast<float4*>(out)[1] = make_float4(sum[4], sum[5], sum[6], sum[7]);
+  }
+}
+__global__ __launch_bounds__(256) void col_amax_partial_kernel(const uint16_t* __restrict__ x, const float* __restrict__ rm,
+                                                               int64_t R, int64_t K, int64_t ldx, int64_t rows_per_chunk,
+                                                               float* __restrict__ partial) {
+  col_amax_block<false>(blockIdx.x, blockIdx.y, x, rm, R, K, ldx, rows_per_chunk, partial, nullptr);
 }
 
 // Reduce the partials of each column, then p[c] and s_inv[c] (small_kernels.cu:172,181).
 // Block = 64 columns x 4 chunk groups (thread g = tid / 64 takes chunks g, g + 4,
 // ... with several loads in flight); the 4 group maxima meet in LDS.
-__global__ __launch_bounds__(256) void col_exps_kernel(const float* __restrict__ partial, int64_t nchunks, int64_t K,
-                                                       int t, int32_t* __restrict__ cexp, float* __restrict__ s_inv) {
+// psum / sum: also the columns' sums of psum's chunks, rounded once to bf16.
+__device__ __forceinline__ void col_exps_block(int64_t block, const float* __restrict__ partial, int64_t nchunks, int64_t K,
+                                               int t, int32_t* __restrict__ cexp, float* __restrict__ s_inv,
+                                               const float* __restrict__ psum, uint16_t* __restrict__ sum) {
   __shared__ float red[4][64];
   const int cl = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int64_t c = (int64_t)blockIdx.x * 64 + cl;
+  const int64_t c = block * 64 + cl;
   float m = 0.f;
   if (c < K) {
 #pragma unroll 8
@@ -191,6 +224,90 @@ __global__ __launch_bounds__(256) void col_exps_kernel(const float* __restrict__
     cexp[c] = p;
     s_inv[c] = ldexp1(-p);
   }
+  if (sum) {
+    float a = 0.f;
+    if (c < K) {
+#pragma unroll 8
+      for (int64_t i = g; i < nchunks; i += 4) a += psum[i * K + c];
+    }
+    __syncthreads();
+    red[g][cl] = a;
+    __syncthreads();
+    if (g == 0 && c < K)
+      sum[c] = (uint16_t)(pack_bf16((red[0][cl] + red[1][cl]) + (red[2][cl] + red[3][cl]), 0.f) & 0xffffu);
+  }
+}
+__global__ __launch_bounds__(256) void col_exps_kernel(const float* __restrict__ partial, int64_t nchunks, int64_t K,
+                                                       int t, int32_t* __restrict__ cexp, float* __restrict__ s_inv) {
+  col_exps_block(blockIdx.x, partial, nchunks, K, t, cexp, s_inv, nullptr, nullptr);
+}
+
+// ---- training linear: passes that do not depend on each other in one launch ------
+// A small layer's step is bound by its launches (1000 x 768 -> 3072 with a bias: 17
+// launches, 246 us of host time). Each kernel gives a range of its blocks to each pass.
+
+// forward: x's rows and w's rows
+struct TrainFwd {
+  const uint16_t *x, *w;
+  uint16_t *x16, *w16;
+  float *sx, *sw;
+  int32_t* xexp;
+  int64_t M, N, ldx, ldw, xblocks;
+  int K, t;
+};
+__global__ __launch_bounds__(256) void train_rows_kernel(TrainFwd p) {
+  const int64_t b = blockIdx.x;
+  if (b < p.xblocks) quantize_rows_block(b, p.x, p.M, p.K, p.ldx, p.t, 0, p.x16, p.K, p.sx, p.xexp);
+  else quantize_rows_block(b - p.xblocks, p.w, p.N, p.K, p.ldw, p.t, 0, p.w16, p.K, p.sw, nullptr);
+}
+
+// backward: dY's column maxima (and sums) and W's, dY's rows; then the exponents; then
+// the two transposed copies
+struct TrainBwd {
+  const uint16_t *dy, *w;
+  const float* sx;
+  int64_t M, N, K, lddy, ldw, ldT;        // ldT: row stride of dycT, M rounded up to 8
+  int t_dy, t_w, t_rows;
+  int64_t wch, dch;                       // row chunks of W's and dY's column passes
+  float *wpart, *dpart, *dsum;
+  int32_t *wexp, *dexp;
+  float *swc, *sdyc, *sdy, *ones;
+  uint16_t *wcT, *dycT, *dy16, *db;       // null: not wanted
+  int64_t wx, wblocks, dx, dblocks;       // blocks of a pass: x per row chunk, and in all
+};
+__global__ __launch_bounds__(256) void train_scan_kernel(TrainBwd p) {
+  int64_t b = blockIdx.x;
+  if (b < p.dblocks) {
+    const int64_t rows = (p.M + p.dch - 1) / p.dch;
+    if (p.db) col_amax_block<true>(b % p.dx, b / p.dx, p.dy, p.sx, p.M, p.N, p.lddy, rows, p.dpart, p.dsum);
+    else col_amax_block<false>(b % p.dx, b / p.dx, p.dy, p.sx, p.M, p.N, p.lddy, rows, p.dpart, nullptr);
+    return;
+  }
+  b -= p.dblocks;
+  if (b < p.wblocks) {
+    col_amax_block<false>(b % p.wx, b / p.wx, p.w, nullptr, p.N, p.K, p.ldw, (p.N + p.wch - 1) / p.wch, p.wpart, nullptr);
+    return;
+  }
+  quantize_rows_block(b - p.wblocks, p.dy, p.M, (int)p.N, p.lddy, p.t_rows, 1, p.dy16, p.N, p.sdy, nullptr);
+}
+__global__ __launch_bounds__(256) void train_exps_kernel(TrainBwd p, int64_t dblocks, int64_t wblocks) {
+  const int64_t b = blockIdx.x;
+  if (b < dblocks) {
+    col_exps_block(b, p.dpart, p.dch, p.N, p.t_dy, p.dexp, p.sdyc, p.dsum, p.db);
+  } else if (b < dblocks + wblocks) {
+    col_exps_block(b - dblocks, p.wpart, p.wch, p.K, p.t_w, p.wexp, p.swc, nullptr, nullptr);
+  } else {
+    const int64_t i = (b - dblocks - wblocks) * 256 + threadIdx.x;
+    if (i < p.K) p.ones[i] = 1.f;
+  }
+}
+__global__ __launch_bounds__(256) void train_transpose_kernel(TrainBwd p, int64_t dx, int64_t dblocks, int64_t wx) {
+  const int64_t b = blockIdx.x;
+  if (b < dblocks)
+    transpose_convert_block(b % dx, b / dx, p.dy, p.M, p.N, p.lddy, nullptr, p.sx, p.dexp, p.dycT, p.ldT);
+  else
+    transpose_convert_block((b - dblocks) % wx, (b - dblocks) / wx, p.w, p.N, p.K, p.ldw, nullptr, nullptr, p.wexp, p.wcT,
+                            p.N);
 }
 
 __global__ void fill_kernel(float* __restrict__ p, int64_t n, float v) {
@@ -462,21 +579,6 @@ extern "C" int tbf16_quantize_rows_t(const void* x, int64_t R, int64_t K, int64_
   return 0;
 }
 
-extern "C" int tbf16_quantize_rows_both(const void* x, int64_t R, int64_t K, int64_t ldx, int t, void* y16, int64_t ldy,
-                                        void* yT, int64_t ldyT, float* s_inv, int32_t* exps_ws, void* stream) {
-  if (int rc = check_rows("quantize_rows_both", x, R, K, ldx)) return rc;
-  TB_CHECK(ldy % 8 == 0 && ldy >= K && aligned16(y16), "quantize_rows_both: bad output");
-  TB_CHECK(ldyT % 8 == 0 && ldyT >= R && aligned16(yT) && s_inv && exps_ws, "quantize_rows_both: bad output");
-  hipStream_t st = as_stream(stream);
-  if (int rc = launch_quantize_rows(x, R, K, ldx, t, 0, y16, ldy, s_inv, exps_ws, st)) return rc;
-  if (K == 0 || ldyT == 0) return 0;
-  dim3 grid((unsigned)cdiv(K, 256), (unsigned)cdiv(ldyT, 64));
-  transpose_convert_kernel<<<grid, 256, 0, st>>>((const uint16_t*)x, R, K, ldx, exps_ws, nullptr, nullptr,
-                                                 (uint16_t*)yT, ldyT);
-  TB_LAUNCH_CHECK("quantize_rows_both");
-  return 0;
-}
-
 extern "C" size_t tbf16_quantize_cols_ws_bytes(int64_t R, int64_t K) {
   const int64_t ch = col_chunks(R, K);
   return align_up((size_t)(ch * K) * sizeof(float), 256) + align_up((size_t)K * sizeof(int32_t), 256);
@@ -507,6 +609,128 @@ extern "C" int tbf16_quantize_cols_t(const void* x, int64_t R, int64_t K, int64_
   transpose_convert_kernel<<<grid, 256, 0, st>>>((const uint16_t*)x, R, K, ldx, nullptr, row_mul, cexp, (uint16_t*)yT,
                                                  ldyT);
   TB_LAUNCH_CHECK("quantize_cols/convert");
+  return 0;
+}
+
+// ---- the training linear's two halves --------------------------------------------
+extern "C" size_t tbf16_train_linear_fwd_ws_bytes(int64_t N, int64_t K) {
+  return N <= 0 || K < 0 ? 0 : align_up((size_t)N * (size_t)K * 2, 256) + align_up((size_t)N * 4, 256);
+}
+extern "C" int tbf16_train_linear_fwd(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w, int64_t N,
+                                      int64_t ldw, const void* bias, int t, void* x16, void* xT, int64_t ldT, float* sx,
+                                      int32_t* exps_ws, void* y, int64_t ldy, void* ws, int64_t ws_bytes, void* stream) {
+  if (int rc = check_rows("train_linear_fwd: w", w, N, K, ldw)) return rc;
+  TB_CHECK(M > 0 && N > 0 && K > 0 && N % 8 == 0, "train_linear_fwd: empty, or N no multiple of 8");
+  TB_CHECK(x16 && aligned16(x16) && sx, "train_linear_fwd: x16 or its scales missing");
+  TB_CHECK(ws && aligned16(ws) && ws_bytes >= (int64_t)tbf16_train_linear_fwd_ws_bytes(N, K),
+           "train_linear_fwd: workspace too small");
+  hipStream_t st = as_stream(stream);
+  TrainFwd p{};
+  p.w = (const uint16_t*)w;
+  p.w16 = static_cast<uint16_t*>(ws);
+  p.sw = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + align_up((size_t)N * (size_t)K * 2, 256));
+  p.N = N; p.ldw = ldw; p.K = (int)K; p.t = t;
+  if (x) {
+    if (int rc = check_rows("train_linear_fwd: x", x, M, K, ldx)) return rc;
+    TB_CHECK(xT && aligned16(xT) && ldT % 8 == 0 && ldT >= M && exps_ws, "train_linear_fwd: bad output");
+    p.x = (const uint16_t*)x;
+    p.x16 = (uint16_t*)x16;
+    p.sx = sx;
+    p.xexp = exps_ws;
+    p.M = M; p.ldx = ldx;
+    p.xblocks = cdiv(M, kRowWaves);
+  }
+  train_rows_kernel<<<(unsigned)(p.xblocks + cdiv(N, kRowWaves)), 256, 0, st>>>(p);
+  TB_LAUNCH_CHECK("train_linear_fwd/rows");
+  if (x) {
+    dim3 grid((unsigned)cdiv(K, 256), (unsigned)cdiv(ldT, 64));
+    transpose_convert_kernel<<<grid, 256, 0, st>>>(p.x, M, K, ldx, exps_ws, nullptr, nullptr, (uint16_t*)xT, ldT);
+    TB_LAUNCH_CHECK("train_linear_fwd/transpose");
+  }
+  return tbf16_gemm_f16(x16, M, K, K, sx, p.w16, N, K, p.sw, bias, y, ldy, -1, stream);
+}
+
+namespace {
+struct TrainBwdWs {
+  size_t wpart, dpart, dsum, wexp, dexp, swc, sdyc, sdy, ones, wcT, dycT, dy16, total;
+};
+TrainBwdWs train_bwd_ws(int64_t M, int64_t N, int64_t K) {
+  TrainBwdWs w{};
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += align_up(bytes, 256);
+    return o;
+  };
+  const int64_t M8 = cdiv(M, 8) * 8, wch = col_chunks(N, K), dch = col_chunks(M, N);
+  w.wpart = take((size_t)(wch * K) * 4);
+  w.dpart = take((size_t)(dch * N) * 4);
+  w.dsum = take((size_t)(dch * N) * 4);
+  w.wexp = take((size_t)K * 4);
+  w.dexp = take((size_t)N * 4);
+  w.swc = take((size_t)K * 4);
+  w.sdyc = take((size_t)N * 4);
+  w.sdy = take((size_t)M * 4);
+  w.ones = take((size_t)K * 4);
+  w.wcT = take((size_t)K * (size_t)N * 2);
+  w.dycT = take((size_t)N * (size_t)M8 * 2);
+  w.dy16 = take((size_t)M * (size_t)N * 2);
+  w.total = at;
+  return w;
+}
+}  // namespace
+
+extern "C" size_t tbf16_train_linear_bwd_ws_bytes(int64_t M, int64_t N, int64_t K) {
+  return M <= 0 || N <= 0 || K <= 0 ? 0 : train_bwd_ws(M, N, K).total;
+}
+extern "C" int tbf16_train_linear_bwd(const void* dy, int64_t M, int64_t N, int64_t lddy, const void* w, int64_t K,
+                                      int64_t ldw, const void* xT, int64_t ldT, const float* sx, int t_w, int t_rows,
+                                      int t_dy, void* dx, void* dw, void* db, void* ws, int64_t ws_bytes, void* stream) {
+  if (int rc = check_rows("train_linear_bwd: dy", dy, M, N, lddy)) return rc;
+  if (int rc = check_rows("train_linear_bwd: w", w, N, K, ldw)) return rc;
+  TB_CHECK(M > 0 && N > 0 && K > 0, "train_linear_bwd: empty");
+  TB_CHECK(dx == nullptr || aligned16(dx), "train_linear_bwd: misaligned dx");
+  TB_CHECK(dw == nullptr || (aligned16(dw) && xT && aligned16(xT) && ldT == cdiv(M, 8) * 8 && sx),
+           "train_linear_bwd: dw needs the transposed x16, its row stride and scales");
+  TB_CHECK(ws && aligned16(ws) && ws_bytes >= (int64_t)tbf16_train_linear_bwd_ws_bytes(M, N, K),
+           "train_linear_bwd: workspace too small");
+  hipStream_t st = as_stream(stream);
+  const TrainBwdWs o = train_bwd_ws(M, N, K);
+  uint8_t* const b = static_cast<uint8_t*>(ws);
+  TrainBwd p{};
+  p.dy = (const uint16_t*)dy;
+  p.w = (const uint16_t*)w;
+  p.sx = dw ? sx : nullptr;
+  p.M = M; p.N = N; p.K = K; p.lddy = lddy; p.ldw = ldw; p.ldT = ldT;
+  p.t_dy = t_dy; p.t_w = t_w; p.t_rows = t_rows;
+  p.wch = col_chunks(N, K);
+  p.dch = col_chunks(M, N);
+  p.wpart = (float*)(b + o.wpart); p.dpart = (float*)(b + o.dpart); p.dsum = (float*)(b + o.dsum);
+  p.wexp = (int32_t*)(b + o.wexp); p.dexp = (int32_t*)(b + o.dexp);
+  p.swc = (float*)(b + o.swc); p.sdyc = (float*)(b + o.sdyc); p.sdy = (float*)(b + o.sdy); p.ones = (float*)(b + o.ones);
+  p.wcT = (uint16_t*)(b + o.wcT); p.dycT = (uint16_t*)(b + o.dycT); p.dy16 = (uint16_t*)(b + o.dy16);
+  p.db = (uint16_t*)db;
+  const bool cols = dw || db;  // dY's column pass
+  p.dx = cdiv(cdiv(N, 8), 256);
+  p.dblocks = cols ? p.dx * p.dch : 0;
+  p.wx = cdiv(cdiv(K, 8), 256);
+  p.wblocks = dx ? p.wx * p.wch : 0;
+  const int64_t rblocks = dx ? cdiv(M, kRowWaves) : 0;
+  if (p.dblocks + p.wblocks + rblocks == 0) return 0;
+  train_scan_kernel<<<(unsigned)(p.dblocks + p.wblocks + rblocks), 256, 0, st>>>(p);
+  TB_LAUNCH_CHECK("train_linear_bwd/scan");
+  const int64_t de = cols ? cdiv(N, 64) : 0, we = dx ? cdiv(K, 64) : 0;
+  train_exps_kernel<<<(unsigned)(de + we + (dw ? cdiv(K, 256) : 0)), 256, 0, st>>>(p, de, we);
+  TB_LAUNCH_CHECK("train_linear_bwd/exps");
+  const int64_t tdx = cdiv(N, 256), td = dw ? tdx * cdiv(ldT, 64) : 0, twx = cdiv(K, 256), tw = dx ? twx * cdiv(N, 64) : 0;
+  if (td + tw > 0) {
+    train_transpose_kernel<<<(unsigned)(td + tw), 256, 0, st>>>(p, tdx, td, twx);
+    TB_LAUNCH_CHECK("train_linear_bwd/transpose");
+  }
+  if (dx)
+    if (int rc = tbf16_gemm_f16(p.dy16, M, N, N, p.sdy, p.wcT, K, N, p.swc, nullptr, dx, K, -1, stream)) return rc;
+  if (dw)
+    if (int rc = tbf16_gemm_f16(p.dycT, N, ldT, ldT, p.sdyc, xT, K, ldT, p.ones, nullptr, dw, K, -1, stream)) return rc;
   return 0;
 }
 

@@ -36,7 +36,6 @@ _SIGS = {
     "tbf16_row_exps": (I, [P, I64, I64, I64, I, I, P, P, P]),
     "tbf16_quantize_rows": (I, [P, I64, I64, I64, I, I, P, I64, P, P]),
     "tbf16_quantize_rows_t": (I, [P, I64, I64, I64, I, P, I64, P, P, P]),
-    "tbf16_quantize_rows_both": (I, [P, I64, I64, I64, I, P, I64, P, I64, P, P, P]),
     "tbf16_quantize_cols_ws_bytes": (SZ, [I64, I64]),
     "tbf16_quantize_cols_t": (I, [P, I64, I64, I64, I, P, P, I64, P, P, I64, P]),
     "tbf16_linear_ws_bytes": (SZ, [I64, I64, I64, I]),
@@ -46,6 +45,10 @@ _SIGS = {
     "tbf16_linear_noalloc": (I, [P, I64, I64, I64, P, I64, I64, P, P, P, I64, I, I, I, P]),
     "tbf16_linear_exps": (I, [P, I64, I64, I64, P, P, I64, I64, P, P, P, I64, I, P]),
     "tbf16_gemm_f16": (I, [P, I64, I64, I64, P, P, I64, I64, P, P, P, I64, I, P]),
+    "tbf16_train_linear_fwd_ws_bytes": (SZ, [I64, I64]),
+    "tbf16_train_linear_fwd": (I, [P, I64, I64, I64, P, I64, I64, P, I, P, P, I64, P, P, P, I64, P, I64, P]),
+    "tbf16_train_linear_bwd_ws_bytes": (SZ, [I64, I64, I64]),
+    "tbf16_train_linear_bwd": (I, [P, I64, I64, I64, P, I64, I64, P, I64, P, I, I, I, P, P, P, P, I64, P]),
     "tbf16_gemv": (I, [P, P, I64, I64, I64, P, P, P, P]),
     "tbf16_head_amax": (I, [P, I, I64, I64, I64, I64, I64, I64, I64, P, P]),
     "tbf16_head_scale_cast": (I, [P, I, I64, I64, I64, I64, I64, I64, I64, P, I64, I64, P, I, P]),
