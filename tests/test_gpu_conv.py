@@ -261,3 +261,39 @@ def test_conv_native_paths_and_unbatched(dev):
     assert e.tolist() == [3, 3, 3] and x16.shape == (3, 0, 4, 4)
     with pytest.raises(TypeError):
         tconv.unscale_output(x, e, tc.weight_scale)
+
+
+@pytest.mark.parametrize("cl", [False, True])
+@pytest.mark.parametrize("B,C,O,H,W,k,stride,pad,dil,bias", [
+    (1, 8, 16, 5, 7, (3, 3), (1, 1), (1, 1), (1, 1), True),        # less than one tile, rows of 35 pixels
+    (2, 72, 40, 33, 21, (3, 3), (2, 2), (1, 1), (1, 1), True),     # channels past a multiple of 64
+    (3, 136, 264, 18, 18, (5, 5), (1, 3), (2, 2), (1, 1), False),
+    (1, 64, 8, 9, 70, (3, 5), (1, 1), (0, 2), (2, 1), True),       # padding on one side pair, dilation
+    (1, 128, 512, 64, 64, (3, 3), (1, 1), (1, 1), (1, 1), True),   # larger tiles
+    (2, 64, 1, 16, 64, (1, 3), (2, 1), (0, 1), (1, 1), True),
+])
+def test_conv2d_native_forms(dev, B, C, O, H, W, k, stride, pad, dil, bias, cl):
+    """The implicit convolution over the geometries it takes: exact small-integer products
+    (fp32 sums of at most 5 x 5 x 136 terms of magnitude 1, one rounding to bf16), so
+    every tap, edge and remainder must agree bit for bit; samples of different scales."""
+    from tbf16 import conv as TC
+    g = torch.Generator().manual_seed(C + O)
+    m = torch.nn.Conv2d(C, O, k, stride, pad, dil, bias=bias).to(dev).bfloat16()
+    x = torch.randint(-1, 2, (B, C, H, W), generator=g).float() * 2.0 ** (7 * torch.arange(B).view(B, 1, 1, 1))
+    w = torch.randint(-1, 2, (O, C, *k), generator=g).float()
+    b = torch.randint(-4, 5, (O,), generator=g).float() if bias else None
+    with torch.no_grad():
+        m.weight.copy_(w)
+        if bias:
+            m.bias.copy_(b)
+    want = torch.nn.functional.conv2d(x.double(), w.double(), b.double() if bias else None, stride, pad, dil).bfloat16()
+    xd = x.bfloat16().to(dev)
+    xd = xd.to(memory_format=torch.channels_last) if cl else xd
+    c = TC.convert_conv(m)
+    macs = want.numel() * w[0].numel()
+    if macs >= 4 * TC._NATIVE_MIN_MACS or macs <= TC._NATIVE_MIN_MACS // 4:
+        assert TC._native_layout(c, xd, c.padding, c.bias) == (int(cl) if macs >= TC._NATIVE_MIN_MACS else None)
+    with torch.no_grad():
+        y = TC._conv2d_native(c, xd, c.padding, c.bias, int(cl))
+    assert torch.equal(y.cpu(), want)
+    assert y.is_contiguous(memory_format=torch.channels_last if cl else torch.contiguous_format)

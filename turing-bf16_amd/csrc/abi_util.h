@@ -43,6 +43,12 @@ struct AmaxSegs {
 };
 int launch_head_amax3(const AmaxSegs& segs, int64_t D, hipStream_t st);
 
+// A 2-D convolution's sizes: the zero-padded channels-last input Hp x Wp x Cp (channels
+// padded to a multiple of 64), KH x KW taps, output row length Wo, strides, dilations.
+struct ConvShape {
+  int64_t Hp, Wp, Cp, KH, KW, Wo, sh, sw, dh, dw;
+};
+
 }  // namespace tbf16
 
 #define TB_CHECK(cond, ...)           \

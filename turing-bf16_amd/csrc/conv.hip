@@ -2,8 +2,10 @@
 // as an fp16 one on inputs scaled by exact powers of two -- one exponent per
 // sample for the input (a convolution mixes positions, so rows cannot be scaled
 // separately) and one per output channel for the weight -- and the scales are
-// undone in an epilogue that writes bf16. The fp16 convolution itself is
-// MIOpen's (called by the Python layer); these kernels are the passes around it.
+// undone in an epilogue that writes bf16. tbf16_conv2d runs 2-D convolutions whole
+// (an implicit GEMM, gemm.hip's ksplit_kernel); for the others (1-D, 3-D, groups, small
+// ones) the fp16 convolution is MIOpen's, called by the Python layer between the
+// input and epilogue passes here.
 //
 // Memory layout: a sample is n = C * prod(spatial) elements stored back to back
 // (contiguous NC... or channels-last, both keep the batch outermost), so the
@@ -13,6 +15,12 @@
 
 #include "abi_util.h"
 #include "common.h"
+
+namespace tbf16 {
+int launch_conv_gemm(bool channels_last, const uint16_t* x16, const uint16_t* wp, int64_t B, int64_t O, int64_t P, int64_t K,
+                     const float* w_sinv, const uint16_t* bias, const ConvShape& c, const int32_t* exps, uint16_t* y,
+                     hipStream_t st);
+}  // namespace tbf16
 
 namespace {
 using namespace tbf16;
@@ -72,8 +80,8 @@ __device__ __forceinline__ void for_run(int64_t lo, int64_t hi, FV f, FS g) {
 
 // Block b * nch + c reduces elements [c * kChunk, (c + 1) * kChunk) of sample b
 // into partial[b * nch + c].
-__global__ __launch_bounds__(kThreads) void sample_amax_kernel(const uint16_t* __restrict__ x, int64_t n, int nch,
-                                                               uint32_t* __restrict__ partial) {
+__device__ __forceinline__ void sample_amax_block(const uint16_t* __restrict__ x, int64_t n, int nch,
+                                                  uint32_t* __restrict__ partial) {
   const int64_t b = blockIdx.x / nch;
   const int64_t c = blockIdx.x - b * nch;
   const int64_t lo = b * n + c * kChunk;
@@ -93,6 +101,108 @@ __global__ __launch_bounds__(kThreads) void sample_amax_kernel(const uint16_t* _
       [&](int64_t i) { m = max(m, x[i] & 0x7FFFu); });
   m = block_max_u32(m);
   if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+
+__global__ __launch_bounds__(kThreads) void sample_amax_kernel(const uint16_t* __restrict__ x, int64_t n, int nch,
+                                                               uint32_t* __restrict__ partial) {
+  sample_amax_block(x, n, nch, partial);
+}
+
+// ---- implicit convolution: its two operands -------------------------------------------
+// MIOpen's fp16 convolution of 512 channels at 128 x 128 wrote the input out nine times
+// (57 us) for a GEMM of 72 us, between a cast pass (7 us), an epilogue (6 us) and a copy
+// of the bias. Here the cast pass writes the input once, channels last with its zero
+// padding and channels padded to 64, and the GEMM reads each tap straight from it: 151 ->
+// 86 us a call (contiguous), 175 -> 88 (channels last).
+// The first launch also takes the samples' maxima and lays the weight out as
+// [channel][tap][Cp] (its (O, C, KH, KW) rows have the taps innermost).
+__global__ __launch_bounds__(kThreads) void conv_scan_kernel(const uint16_t* __restrict__ x, int64_t n, int nch,
+                                                             uint32_t* __restrict__ partial, unsigned amax_blocks,
+                                                             const uint16_t* __restrict__ w, int64_t O, int C, int T,
+                                                             int Cp, uint16_t* __restrict__ wp) {
+  if (blockIdx.x < amax_blocks) {
+    sample_amax_block(x, n, nch, partial);
+    return;
+  }
+  // one thread per 8 channels of one tap, taps varying fastest: a wave's reads of one
+  // channel cover neighbouring taps and channels
+  const int64_t i = (int64_t)(blockIdx.x - amax_blocks) * kThreads + threadIdx.x;
+  const int c8 = Cp >> 3;
+  if (i >= O * c8 * T) return;
+  const int tap = (int)(i % T), c = (int)(i / T % c8) * 8;
+  const int64_t o = i / T / c8;
+  uint16_t v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = c + e < C ? w[(o * C + c + e) * T + tap] : (uint16_t)0;
+  __builtin_memcpy(wp + (o * T + tap) * Cp + c, v, 16);
+}
+
+// Block (64 padded columns, padded row, image x 64-channel chunk): x16 = fp16(x 2^-e) of its
+// pixels and channels, zeros in the padding. CL: x is channels last (C % 8 == 0); else its
+// 64 x 64 (channel, pixel) square is turned over in LDS.
+template <bool CL>
+__global__ __launch_bounds__(kThreads) void conv_pack_kernel(const uint16_t* __restrict__ x, int C, int H, int W, int ph,
+                                                             int pw, int Hp, int Wp, int Cp, int nch,
+                                                             const uint32_t* __restrict__ partial, int t,
+                                                             int32_t* __restrict__ exps, uint16_t* __restrict__ y) {
+  __shared__ __align__(16) uint16_t tile[CL ? 1 : 64][72];  // [pixel][channel], padded against bank conflicts
+  const int chunks = Cp >> 6;
+  const int64_t b = blockIdx.z / chunks;
+  const int c0 = (int)(blockIdx.z % chunks) * 64, w0 = (int)blockIdx.x * 64, hp = (int)blockIdx.y;
+  const int h = hp - ph;
+  const bool row_in = h >= 0 && h < H;
+  uint16_t* const yrow = y + ((b * Hp + hp) * Wp) * (int64_t)Cp + c0;
+  // the raw values first: they are in flight while the sample's exponent is derived
+  uint4 vec[2];       // CL: pixel i / 8, channels 8 (i % 8) .. + 7 for i = thread + 256 j
+  uint32_t pair[8];   // else pixels 2 (thread % 32), + 1 of channel thread / 32 + 8 j
+  if constexpr (CL) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = threadIdx.x + j * kThreads, w = w0 + (i >> 3) - pw, c = (i & 7) * 8;
+      vec[j] = make_uint4(0, 0, 0, 0);
+      if (row_in && w >= 0 && w < W && c0 + c < C) vec[j] = ldg16(x + ((b * H + h) * (int64_t)W + w) * C + c0 + c);
+    }
+  } else {
+    const int w = w0 + 2 * (threadIdx.x & 31) - pw;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int c = c0 + (threadIdx.x >> 5) + 8 * j;
+      pair[j] = 0u;
+      if (row_in && c < C) {
+        const uint16_t* const src = x + ((b * C + c) * (int64_t)H + h) * W + w;
+        if (w >= 0 && w + 1 < W) __builtin_memcpy(&pair[j], src, 4);
+        else if (w >= 0 && w < W) pair[j] = src[0];
+        else if (w + 1 >= 0 && w + 1 < W) pair[j] = (uint32_t)src[1] << 16;
+      }
+    }
+  }
+  uint32_t m = 0u;
+  for (int i = threadIdx.x; i < nch; i += kThreads) m = max(m, partial[b * nch + i]);
+  const int e = sample_exp(block_max_u32(m), t);
+  if (blockIdx.x == 0 && blockIdx.y == 0 && c0 == 0 && threadIdx.x == 0) exps[b] = e;
+  const float s = ldexp1(-e);
+  if constexpr (CL) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = threadIdx.x + j * kThreads, px = w0 + (i >> 3);
+      if (px < Wp) stg16(yrow + (int64_t)px * Cp + (i & 7) * 8, cvt_bf16x8_f16x8(vec[j], s));
+    }
+  } else {
+    const int px = 2 * (threadIdx.x & 31);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int c = (threadIdx.x >> 5) + 8 * j;
+      const uint32_t v = cvt_bf16x2_f16x2(pair[j], s);
+      tile[px][c] = (uint16_t)v;
+      tile[px + 1][c] = (uint16_t)(v >> 16);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = threadIdx.x + j * kThreads, p = i >> 3, c = (i & 7) * 8;
+      if (w0 + p < Wp) stg16(yrow + (int64_t)(w0 + p) * Cp + c, *reinterpret_cast<const uint4*>(&tile[p][c]));
+    }
+  }
 }
 
 // Block b * nch + c: the exponent of sample b from its nch partial maxima, then
@@ -280,4 +390,83 @@ extern "C" int tbf16_conv_epilogue(const void* y16, int64_t B, int64_t O, int64_
 #undef LAUNCH
   TB_LAUNCH_CHECK("conv_epilogue");
   return 0;
+}
+
+namespace {
+struct Conv2dPlan {
+  ConvShape c;
+  int64_t B, O, P, K, nch;
+  size_t exps, wp, x16, total;
+};
+// 0, or an error with its reason set: sizes the kernels' 32-bit offsets do not reach
+int conv2d_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, const int64_t* stride,
+                const int64_t* pad, const int64_t* dilation, Conv2dPlan& p) {
+  TB_CHECK(B > 0 && C > 0 && H > 0 && W > 0 && O > 0 && KH > 0 && KW > 0, "conv2d: empty");
+  TB_CHECK(stride && pad && dilation && stride[0] > 0 && stride[1] > 0 && pad[0] >= 0 && pad[1] >= 0 && dilation[0] > 0 &&
+               dilation[1] > 0,
+           "conv2d: bad stride, padding or dilation");
+  ConvShape& c = p.c;
+  c.Hp = H + 2 * pad[0];
+  c.Wp = W + 2 * pad[1];
+  c.Cp = cdiv(C, 64) * 64;
+  c.KH = KH; c.KW = KW;
+  c.sh = stride[0]; c.sw = stride[1];
+  c.dh = dilation[0]; c.dw = dilation[1];
+  const int64_t eh = (KH - 1) * c.dh + 1, ew = (KW - 1) * c.dw + 1;
+  TB_CHECK(c.Hp >= eh && c.Wp >= ew, "conv2d: the kernel is larger than the padded input");
+  const int64_t Ho = (c.Hp - eh) / c.sh + 1;
+  c.Wo = (c.Wp - ew) / c.sw + 1;
+  p.B = B; p.O = O;
+  p.P = Ho * c.Wo;
+  p.K = KH * KW * c.Cp;
+  p.nch = amax_chunks(C * H * W);
+  TB_CHECK(c.Hp * c.Wp * c.Cp < (int64_t)1 << 30 && p.K < (int64_t)1 << 22 && O < (int64_t)1 << 31 && B < 65536 &&
+               c.Hp < 65536 && B * (c.Cp / 64) < 65536 && B * p.nch < (int64_t)1 << 30 && O * p.K < (int64_t)1 << 33,
+           "conv2d: tensor too large");
+  p.exps = align_up((size_t)(B * p.nch) * 4, 256);
+  p.wp = p.exps + align_up((size_t)B * 4, 256);
+  p.x16 = p.wp + align_up((size_t)O * (size_t)p.K * 2, 256);
+  p.total = p.x16 + align_up((size_t)B * (size_t)(c.Hp * c.Wp * c.Cp) * 2, 256);
+  return 0;
+}
+}  // namespace
+
+extern "C" size_t tbf16_conv2d_ws_bytes(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW,
+                                        const int64_t* stride, const int64_t* pad, const int64_t* dilation) {
+  Conv2dPlan p;
+  return conv2d_plan(B, C, H, W, O, KH, KW, stride, pad, dilation, p) ? 0 : p.total;
+}
+
+extern "C" int tbf16_conv2d(const void* x, int64_t B, int64_t C, int64_t H, int64_t W, int channels_last, int t,
+                            const void* w16, int64_t O, int64_t KH, int64_t KW, const int64_t* stride, const int64_t* pad,
+                            const int64_t* dilation, const float* w_sinv, const void* bias, void* y, void* ws,
+                            int64_t ws_bytes, void* stream) {
+  Conv2dPlan p;
+  if (int rc = conv2d_plan(B, C, H, W, O, KH, KW, stride, pad, dilation, p)) return rc;
+  TB_CHECK(x && w16 && w_sinv && y && aligned16(x) && aligned16(y), "conv2d: null or misaligned pointer");
+  TB_CHECK(!channels_last || C % 8 == 0, "conv2d: channels-last input needs channels in multiples of 8");
+  TB_CHECK(ws && aligned16(ws) && ws_bytes >= (int64_t)p.total, "conv2d: workspace too small");
+  hipStream_t st = as_stream(stream);
+  uint8_t* const base = static_cast<uint8_t*>(ws);
+  uint32_t* const partial = reinterpret_cast<uint32_t*>(base);
+  int32_t* const exps = reinterpret_cast<int32_t*>(base + p.exps);
+  uint16_t* const wp = reinterpret_cast<uint16_t*>(base + p.wp);
+  uint16_t* const x16 = reinterpret_cast<uint16_t*>(base + p.x16);
+  const ConvShape& c = p.c;
+  const unsigned amax_blocks = (unsigned)(B * p.nch);
+  const int64_t wblocks = cdiv(O * (c.Cp / 8) * KH * KW, kThreads);
+  conv_scan_kernel<<<(unsigned)(amax_blocks + wblocks), kThreads, 0, st>>>((const uint16_t*)x, C * H * W, (int)p.nch, partial,
+                                                                            amax_blocks, (const uint16_t*)w16, O, (int)C,
+                                                                            (int)(KH * KW), (int)c.Cp, wp);
+  TB_LAUNCH_CHECK("conv2d/scan");
+  const dim3 grid((unsigned)cdiv(c.Wp, 64), (unsigned)c.Hp, (unsigned)(B * (c.Cp / 64)));
+#define PACK(CL)                                                                                                       \
+  conv_pack_kernel<CL><<<grid, kThreads, 0, st>>>((const uint16_t*)x, (int)C, (int)H, (int)W, (int)pad[0], (int)pad[1], \
+                                                  (int)c.Hp, (int)c.Wp, (int)c.Cp, (int)p.nch, partial, t, exps, x16)
+  if (channels_last) PACK(true);
+  else PACK(false);
+#undef PACK
+  TB_LAUNCH_CHECK("conv2d/pack");
+  return launch_conv_gemm(channels_last != 0, x16, wp, B, O, p.P, p.K, w_sinv, (const uint16_t*)bias, c, exps,
+                          (uint16_t*)y, st);
 }

@@ -851,6 +851,83 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                part ? part + (int64_t)ks * M * N : nullptr, N);
 }
 
+// Where an implicit convolution's output pixels lie in its zero-padded channels-last
+// input, in elements: `image` one image, row_step / col_step from one output row / column
+// to the next; in bytes: next_col / next_row from the end of one tap's `chunks` 64-channel
+// chunks (of one row's KW taps) to the start of the next.
+struct ConvGeom {
+  int64_t image = 0, out_image = 0;
+  int Wo = 1, row_step = 0, col_step = 0, KW = 1, chunks = 1, next_col = 0, next_row = 0;
+  const int32_t* exps = nullptr;
+};
+
+// store_tile16 for an implicit convolution: bf16(acc * sc[channel] + bias[channel]), channels
+// along columns (CONV 1) or rows (CONV 2); rows of y at any alignment, the last columns
+// one by one.
+template <int TM, int TN, int CONV>
+__device__ __forceinline__ void store_conv(const floatx4 (&acc)[TN / 16][TM / 16], const float* sc_l, const float* cb_l,
+                                           int wm, int wn, int lane, int m0, int n0, uint16_t* __restrict__ C, int64_t ldc,
+                                           int M, int N) {
+  constexpr int FM = TM / 16, FN = TN / 16, NP = FN / 2;
+  const int fr = lane & 15, fk = lane >> 4;
+  const int cl = ((fk & 1) << 4) | ((fk >> 1) << 3);
+  const bool hi8 = (lane & 8) != 0;
+  auto put = [&](int m, int n, const uint32_t (&v)[4]) {
+    if (m >= M || n >= N) return;
+    uint16_t* const dst = C + (int64_t)m * ldc + n;
+    if (n + 8 <= N) {
+      __builtin_memcpy(dst, v, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < N) dst[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int ml = wm * TM + j * 16 + fr;
+    uint32_t v[NP][4];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      uint32_t w[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const floatx4 c = acc[2 * p + i][j];
+        float4 sc, cb;
+        if constexpr (CONV == 1) {
+          const int nl = wn * TN + (2 * p + i) * 16 + 4 * fk;
+          sc = *reinterpret_cast<const float4*>(sc_l + nl);
+          cb = *reinterpret_cast<const float4*>(cb_l + nl);
+        } else {
+          sc.x = sc.y = sc.z = sc.w = sc_l[ml];
+          cb.x = cb.y = cb.z = cb.w = cb_l[ml];
+        }
+        w[i][0] = pack_bf16(fmaf(c[0], sc.x, cb.x), fmaf(c[1], sc.y, cb.y));
+        w[i][1] = pack_bf16(fmaf(c[2], sc.z, cb.z), fmaf(c[3], sc.w, cb.w));
+      }
+      const auto d0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+      const auto d1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+      v[p][0] = d0[0]; v[p][1] = d1[0]; v[p][2] = d0[1]; v[p][3] = d1[1];
+    }
+    const int row0 = m0 + wm * TM + j * 16, col0 = n0 + wn * TN + cl;
+    if constexpr (NP == 2) {
+      uint32_t f[4], g[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t t0 = __builtin_amdgcn_mov_dpp((int)v[0][d], 0x128, 0xF, 0xF, false);
+        const uint32_t t1 = __builtin_amdgcn_mov_dpp((int)v[1][d], 0x128, 0xF, 0xF, false);
+        f[d] = hi8 ? t1 : v[0][d];
+        g[d] = hi8 ? v[1][d] : t0;
+      }
+      const int n = col0 + (hi8 ? 32 : 0);
+      put(row0 + (lane & 7), n, f);
+      put(row0 + (lane & 7) + 8, n, g);
+    } else {
+      put(row0 + fr, col0, v[0]);
+    }
+  }
+}
+
 // Ping-pong GEMM on fp16 operands for tiles too small for pingpong_kernel's phases:
 // both groups of four waves (2 x 2 sub-tiles of 16 RM x 16 RN) cover the whole BM x BN
 // tile, group 0 with the even k tiles, group 1 with the odd ones, and their sums meet
@@ -867,11 +944,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // the same for every launch. part / kt_per: split K, as gemm_kernel. R <= BN: columns
 // per block (a multiple of 8); below BN the weights of a single row of tiles are
 // spread over every CU, the rest of the tile is zeros. NB: as pingpong_kernel.
-template <int RM, int RN, int S, bool KEVEN>
+// CONV: an implicit convolution. 1: a's rows are output pixels (y is pixels x channels), 2:
+// b's are (y is channels x pixels), one image per blockIdx.y; the other operand is the
+// weight [channel][tap][Cp]. A pixel's k tile is 64 channels of one tap of the zero-
+// padded channels-last input, so a row's loads start at its own top left element and
+// every k tile adds the same offset to all of them (ConvGeom). The factors are 2^e[image]
+// ws[channel] and the bias fp32.
+template <int RM, int RN, int S, bool KEVEN, int CONV = 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void ksplit_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const float* __restrict__ a_sinv, const uint16_t* __restrict__ B,
     int64_t ldb, const float* __restrict__ b_sinv, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C,
-    int64_t ldc, int M, int N_all, int K_all, float* __restrict__ part, int kt_per, int R, int NB) {
+    int64_t ldc, int M, int N_all, int K_all, float* __restrict__ part, int kt_per, int R, int NB, ConvGeom cg) {
   constexpr int BM = 32 * RM, BN = 32 * RN, TM = 16 * RM, TN = 16 * RN;
   constexpr int STG = (BM + BN) * 128, NL = (BM + BN) / 64, AL = BM / 64;  // loads per wave and tile; the first AL are A's
   constexpr int XB = RM / 2 * RN * 16 * 64;  // bytes of the half sub-tile a wave hands over
@@ -880,7 +963,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __shared__ __align__(1024) uint8_t st3[S > 3 ? STG : 16], st4[S > 4 ? STG : 16], st5[S > 5 ? STG : 16];
   __shared__ __align__(1024) uint8_t st6[S > 6 ? STG : 16], st7[S > 7 ? STG : 16], st8[S > 8 ? STG : 16];
   __shared__ __align__(16) float sa_l[BM], sb_l[BN];
-  __shared__ __align__(16) uint16_t bias_l[BN];
+  __shared__ __align__(16) uint16_t bias_l[CONV ? 8 : BN];
+  __shared__ __align__(16) float cbias_l[CONV == 1 ? BN : CONV == 2 ? BM : 4];
   uint8_t* const stages[9] = {st0, st1, st2, st3, st4, st5, st6, st7, st8};
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -896,14 +980,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int within = bid % (GM * tiles_n);
   const int m0 = (first + within % gsize) * BM;
   const int n0 = (within / gsize) * R, N = min(N_all, n0 + R);
-  const int ks = part ? (int)blockIdx.y : 0;
+  const int ks = !CONV && part ? (int)blockIdx.y : 0;
+  if constexpr (CONV == 1) A += (int64_t)blockIdx.y * cg.image;
+  if constexpr (CONV == 2) B += (int64_t)blockIdx.y * cg.image;
+  if constexpr (CONV != 0) C += (int64_t)blockIdx.y * cg.out_image;
   const int kbase = ks * kt_per * 64;
   const int K = part ? min(K_all - kbase, kt_per * 64) : K_all;
 
   // the epilogue's factors (see pingpong_kernel)
   const int fc = tid - 256;
-  const float fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, NB - 1)];
-  const uint16_t fbias = bias ? bias[min(n0 + max(fc, 0), NB - 1)] : (uint16_t)0;
+  float fsc, fcb = 0.f;
+  uint16_t fbias = 0;
+  if constexpr (CONV != 0) {
+    const int o = CONV == 1 ? min(n0 + (tid & 255), N_all - 1) : min(m0 + (tid & 255), M - 1);
+    fsc = ldexp1(cg.exps[blockIdx.y]) * (CONV == 1 ? b_sinv : a_sinv)[o];
+    if (bias) fcb = bf16_lo(bias[o]);
+  } else {
+    fsc = fc < 0 ? a_sinv[min(m0 + tid, M - 1)] : b_sinv[min(n0 + fc, NB - 1)];
+    if (bias) fbias = bias[min(n0 + max(fc, 0), NB - 1)];
+  }
 
   // direct loads: 1 KB block wave + 8 i of the stage (rows of A, then of B)
   const int chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
@@ -911,12 +1006,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int r = 8 * (wave + 8 * (i < AL ? i : i - AL)) + (lane >> 3);
-    off[i] = (r * (int)(i < AL ? lda : ldb) + chunk * 8) * 2;
+    if ((CONV == 1 && i < AL) || (CONV == 2 && i >= AL)) {  // pixels past the last take the last's
+      const int px = CONV == 1 ? min(m0 + r, M - 1) : min(n0 + r, N_all - 1);
+      off[i] = (px / cg.Wo * cg.row_step + px % cg.Wo * cg.col_step + chunk * 8) * 2;
+    } else {
+      off[i] = (r * (int)(i < AL ? lda : ldb) + chunk * 8) * 2;
+    }
   }
   const BufRes ares =
-      make_res(A + (int64_t)m0 * lda + kbase, min<int64_t>((int64_t)(M - m0) * lda * 2 - kbase * 2, 0x7fffffff));
+      CONV == 1 ? make_res(A, cg.image * 2)
+                : make_res(A + (int64_t)m0 * lda + kbase, min<int64_t>((int64_t)(M - m0) * lda * 2 - kbase * 2, 0x7fffffff));
   const BufRes bres =
-      make_res(B + (int64_t)n0 * ldb + kbase, min<int64_t>((int64_t)(min(N, NB) - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
+      CONV == 2 ? make_res(B, cg.image * 2)
+                : make_res(B + (int64_t)n0 * ldb + kbase,
+                           min<int64_t>((int64_t)(min(N, NB) - n0) * ldb * 2 - kbase * 2, 0x7fffffff));
+  // byte offset of a pixel's k tile from its top left element; load() is called for the
+  // k tiles in order by every wave
+  int p_off = 0, p_chunk = 0, p_col = 0;
   const int KT = (K + 63) / 64;
   auto load = [&](uint8_t* stage, int kt) {
     const BufRes ra{ares.lo, ares.hi, kt < KT ? ares.bytes : 0}, rb{bres.lo, bres.hi, kt < KT ? bres.bytes : 0};
@@ -924,7 +1030,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const bool kok = KEVEN || kt * 64 + chunk * 8 < K;  // a k tail reads zeros
 #pragma unroll
     for (int i = 0; i < NL; ++i)
-      buf_load16_lds(i < AL ? ra : rb, base + i * 8192, kok ? off[i] : (int)0x80000000, kt * 128);
+      buf_load16_lds(i < AL ? ra : rb, base + i * 8192, kok ? off[i] : (int)0x80000000,
+                     (CONV == 1 && i < AL) || (CONV == 2 && i >= AL) ? p_off : kt * 128);
+    if constexpr (CONV != 0) {
+      p_off += 128;
+      if (++p_chunk == cg.chunks) {
+        p_chunk = 0;
+        p_off += cg.next_col;
+        if (++p_col == cg.KW) {
+          p_col = 0;
+          p_off += cg.next_row;
+        }
+      }
+    }
   };
 
   floatx4 acc[RN][RM];  // [16 columns][16 rows]
@@ -946,7 +1064,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 #pragma unroll
   for (int t = 0; t < S - 1; ++t) load(stages[t], t);
-  if (fc < 0) {
+  if constexpr (CONV != 0) {
+    if (tid < (CONV == 1 ? BN : BM)) {
+      (CONV == 1 ? sb_l : sa_l)[tid] = fsc;
+      cbias_l[tid] = fcb;
+    }
+  } else if (fc < 0) {
     if (tid < BM) sa_l[tid] = fsc;
   } else if (fc < BN) {
     sb_l[fc] = fsc;
@@ -1025,8 +1148,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         sum[i][j][3] = o[3] + v.w;
       }
     // rows wm TM + g TM / 2 of the tile: sub-tile row 2 wm + g of height TM / 2
-    store_tile16<TM / 2, TN>(sum, sa_l, sb_l, bias_l, 2 * wm + g, wn, lane, m0, n0, C, ldc, M, N,
-                             part ? part + (int64_t)ks * M * N_all : nullptr, N_all);
+    if constexpr (CONV != 0)
+      store_conv<TM / 2, TN, CONV>(sum, CONV == 1 ? sb_l : sa_l, cbias_l, 2 * wm + g, wn, lane, m0, n0, C, ldc, M, N);
+    else
+      store_tile16<TM / 2, TN>(sum, sa_l, sb_l, bias_l, 2 * wm + g, wn, lane, m0, n0, C, ldc, M, N,
+                               part ? part + (int64_t)ks * M * N_all : nullptr, N_all);
   };
   if (wave < 4) run(std::integral_constant<int, 0>{});
   else run(std::integral_constant<int, 1>{});
@@ -1733,10 +1859,10 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
     const dim3 grid(g, part ? (unsigned)splits : 1u);                                                       \
     if (even)                                                                                               \
       ksplit_kernel<RM_, RN_, S_, true><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, M, \
-                                                              N, K, part, kt_per, rows, NB);                \
+                                                              N, K, part, kt_per, rows, NB, ConvGeom{});    \
     else                                                                                                    \
       ksplit_kernel<RM_, RN_, S_, false><<<grid, 512, 0, st>>>(a, lda, a_sinv, b, ldb, b_sinv, bi, c, ldc, M, \
-                                                               N, K, part, kt_per, rows, NB);               \
+                                                               N, K, part, kt_per, rows, NB, ConvGeom{});   \
   }
     case 25: KSPLIT(8, 4, 3); break;
     case 26: KSPLIT(6, 4, 3); break;
@@ -1949,6 +2075,57 @@ extern "C" int tbf16_linear_noalloc(const void* x, int64_t M, int64_t K, int64_t
   if (int rc = scratch_ptr(&wsp)) return rc;
   return linear_into(w, x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1, wsp, st);
 }
+
+// ---- implicit convolution ---------------------------------------------------------
+namespace tbf16 {
+int launch_conv_gemm(bool channels_last, const uint16_t* x16, const uint16_t* wp, int64_t B, int64_t O, int64_t P, int64_t K,
+                     const float* w_sinv, const uint16_t* bias, const ConvShape& c, const int32_t* exps, uint16_t* y,
+                     hipStream_t st) {
+  ConvGeom g;
+  g.image = c.Hp * c.Wp * c.Cp;
+  g.out_image = O * P;
+  g.Wo = (int)c.Wo;
+  g.row_step = (int)(c.sh * c.Wp * c.Cp);
+  g.col_step = (int)(c.sw * c.Cp);
+  g.KW = (int)c.KW;
+  g.chunks = (int)(c.Cp / 64);
+  g.next_col = (int)((c.dw * c.Cp - c.Cp) * 2);
+  g.next_row = (int)((c.dh * c.Wp * c.Cp - c.KW * c.dw * c.Cp) * 2);
+  g.exps = exps;
+  const int64_t M = channels_last ? P : O, N = channels_last ? O : P, KT = K / 64, cus = num_cus();
+  int cfg = 27;
+  float best = INFINITY;
+  for (const F16Cand& f : kF16Cands) {
+    const TileCfg& t = kCfgs[f.cfg];
+    if (!t.ksplit || f.cfg == 26) continue;
+    const int64_t tiles = B * cdiv(M, t.bm) * cdiv(N, t.bn);
+    const float us = (float)cdiv(tiles, cus) *
+                     (f.c1 + (float)KT * (f.light + (f.full - f.light) * std::min(1.f, (float)tiles / (float)cus)));
+    if (us < best) {
+      best = us;
+      cfg = f.cfg;
+    }
+  }
+  const dim3 grid((unsigned)(cdiv(M, kCfgs[cfg].bm) * cdiv(N, kCfgs[cfg].bn)), (unsigned)B);
+#define CONV_GEMM(RM_, RN_, S_)                                                                                     \
+  if (channels_last)                                                                                                \
+    ksplit_kernel<RM_, RN_, S_, true, 1><<<grid, 512, 0, st>>>(x16, 0, nullptr, wp, K, w_sinv, bias, y, O, (int)M, (int)N, \
+                                                               (int)K, nullptr, 0, 32 * RN_, (int)N, g);             \
+  else                                                                                                              \
+    ksplit_kernel<RM_, RN_, S_, true, 2><<<grid, 512, 0, st>>>(wp, K, w_sinv, x16, 0, nullptr, bias, y, P, (int)M, (int)N, \
+                                                               (int)K, nullptr, 0, 32 * RN_, (int)N, g)
+  switch (cfg) {
+    case 25: CONV_GEMM(8, 4, 3); break;
+    case 28: CONV_GEMM(4, 2, 6); break;
+    case 29: CONV_GEMM(2, 4, 6); break;
+    case 30: CONV_GEMM(2, 2, 6); break;
+    default: CONV_GEMM(4, 4, 4); break;
+  }
+#undef CONV_GEMM
+  TB_LAUNCH_CHECK("conv2d/gemm");
+  return 0;
+}
+}  // namespace tbf16
 
 extern "C" int tbf16_linear_exps(const void* x, int64_t M, int64_t K, int64_t ldx, const int32_t* exps,
                                  const void* w16, int64_t N, int64_t ldw, const float* ws, const void* bias, void* y,

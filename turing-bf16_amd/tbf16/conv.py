@@ -7,16 +7,19 @@ one pass that writes bf16. The weight conversion is lossless; the input's is
 lossless for every element within 2^14 of its sample's max (smaller ones become
 fp16 subnormals, far below the output's bf16 rounding).
 
-On MI355X the passes around the convolution are HIP kernels behind the C ABI
-(tbf16_conv_input: per-sample max, exponent and scaled fp16 copy;
-tbf16_conv_epilogue: both scales and the bias in one bf16-writing pass); the fp16
-convolution is MIOpen's, through torch. 1x1 convolutions (stride 1, no padding,
+On MI355X a 2-D convolution of some size runs whole on the library's kernels
+(tbf16_conv2d: per-sample maxima, one scaled channels-last copy of the input, an
+implicit GEMM that writes bf16 from its fp32 sums). For the others the passes around the
+convolution are HIP kernels (tbf16_conv_input: per-sample max, exponent and scaled fp16
+copy; tbf16_conv_epilogue: both scales and the bias in one bf16-writing pass) and the
+fp16 convolution is MIOpen's, through torch. 1x1 convolutions (stride 1, no padding,
 one group) are per-pixel linear layers and go through scaled_linear, which scales
 each pixel separately. Inference only: inputs that need gradients, or are not
 bf16, run the native convolution on the dequantized weight (conv.py:34-38).
 Converted modules get the class TBF16<their class>, the buffers weight16 and
 weight_scale and the method dequantized_weight(), as in the reference.
 """
+import ctypes
 import functools
 from typing import NamedTuple
 
@@ -93,6 +96,63 @@ def _pointwise(conv: nn.Module) -> bool:
     return unpadded and conv.groups == 1 and set(conv.kernel_size) == {1} and set(conv.stride) == {1}
 
 
+def _pair(v) -> ctypes.Array:
+    return (ctypes.c_int64 * 2)(*v)
+
+
+# Multiply-adds below which the fp16 convolution stays the library's.
+_NATIVE_MIN_MACS = 1 << 29
+
+
+def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
+    """0 (contiguous) or 1 (channels last) when the native 2-D convolution takes this
+    call, else None: one group, zero padding given in numbers, a bf16 bias, an input
+    dense in exactly one of the two layouts.
+    Small convolutions (_NATIVE_MIN_MACS) keep the library's fp16 convolution and its
+    fp16 rounding: their results are pinned bit for bit to the reference's formula on
+    that call. The native kernel is the faster one there too (64 -> 64 at 16 x 16: 22 us
+    against 51)."""
+    if (x.dim() != 4 or conv.groups != 1 or isinstance(padding, str) or x.numel() == 0 or x.data_ptr() % 16
+            or not conv.weight16.is_contiguous() or (bias is not None and bias.dtype != torch.bfloat16)):
+        return None
+    nchw, nhwc = x.is_contiguous(), x.is_contiguous(memory_format=torch.channels_last)
+    if nchw == nhwc or (nhwc and x.shape[1] % 8):
+        return None
+    # the kernels pad channels to 64: with three of them on a large image the padded copy
+    # costs more than MIOpen's passes (3 -> 128 at 512 x 512: 93 us against 89; every
+    # other shape measured is 1.07 to 3.8 times as fast, 3 -> 64 at 2 x 224 x 224 1.6)
+    if x.shape[1] < 4 and x.numel() > x.shape[1] << 17:
+        return None
+    # (input pixels over strides: the output's, up to its edges)
+    macs = x.numel() // (conv.stride[0] * conv.stride[1]) * (conv.weight16.numel() // x.shape[1])
+    return int(nhwc) if macs >= _NATIVE_MIN_MACS else None
+
+
+def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int):
+    """The whole scaled convolution on the library's own kernels, or None for sizes they
+    do not take."""
+    B, C, H, W = x.shape
+    w16 = conv.weight16
+    O, _, KH, KW = w16.shape
+    pad = (padding, padding) if isinstance(padding, int) else padding
+    stride, dilation = conv.stride, conv.dilation
+    geom = (_pair(stride), _pair(pad), _pair(dilation))
+    wsb = lib().tbf16_conv2d_ws_bytes(B, C, H, W, O, KH, KW, *geom)
+    if wsb == 0:
+        return None
+    _dev_check(x, w16, conv.weight_scale)
+    Ho = (H + 2 * pad[0] - dilation[0] * (KH - 1) - 1) // stride[0] + 1
+    Wo = (W + 2 * pad[1] - dilation[1] * (KW - 1) - 1) // stride[1] + 1
+    y = torch.empty((B, O, Ho, Wo), device=x.device, dtype=torch.bfloat16,
+                    memory_format=torch.channels_last if layout else torch.contiguous_format)
+    ws = torch.empty(wsb, device=x.device, dtype=torch.uint8)
+    b = None if bias is None else bias.detach().contiguous()
+    s = conv.weight_scale.float().contiguous()
+    launch("tbf16_conv2d", x, ptr(x), B, C, H, W, layout, int(conv._tbf16_plan.target_exp), ptr(w16), O, KH, KW, *geom,
+           ptr(s), ptr(b), ptr(y), ptr(ws), wsb)
+    return y
+
+
 def _run_scaled(conv: nn.Module, x: torch.Tensor, bias) -> torch.Tensor:
     """The scaled fp16 convolution of a batched bf16 input (tbf16/conv.py:39-60)."""
     plan = conv._tbf16_plan
@@ -103,6 +163,11 @@ def _run_scaled(conv: nn.Module, x: torch.Tensor, bias) -> torch.Tensor:
     if conv.padding_mode != "zeros":  # reflect / replicate / circular: pad first, convolve unpadded
         x = F.pad(x, conv._reversed_padding_repeated_twice, mode=conv.padding_mode)
         padding = 0
+    layout = _native_layout(conv, x, padding, bias)
+    if layout is not None:
+        y = _conv2d_native(conv, x, padding, bias, layout)
+        if y is not None:
+            return y
     exps, x16 = scale_input(x, plan.target_exp)
     y16 = _CONV[x.dim() - 2](x16, conv.weight16, None, conv.stride, padding, conv.dilation, conv.groups)
     return unscale_output(y16, exps, conv.weight_scale, bias)
