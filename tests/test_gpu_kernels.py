@@ -191,6 +191,29 @@ def test_linear_dispatch_splits_bit_exact(dev, M, N, K):
         assert torch.equal(y.cpu(), want), name
 
 
+@pytest.mark.parametrize("M,K,N", [(17, 6528, 832), (32, 4104, 264), (33, 6528, 832), (2048, 3200, 640), (1999, 3400, 520),
+                                   (640, 16384, 512)])
+def test_linear_dispatch_few_rows_and_row_chunks(dev, M, K, N):
+    """At most 32 rows whose tiles would split K (converted in the skinny kernel) and 33;
+    x16 beyond the no-allocation array, which that entry point then takes in chunks of
+    rows (the last one short): exact products, and the same bits from both entry points."""
+    g = torch.Generator().manual_seed(M)
+    a, b = torch.randint(-1, 2, (M, K), generator=g), torch.randint(-1, 2, (N, K), generator=g)
+    ones = torch.ones(N, device=dev)
+    b16 = b.half().to(dev)
+    work, _ = linear_ws(M, K, N, -1, dev)
+    for x, exact in ((a.bfloat16().to(dev), True), (torch.randn(M, K, generator=g).bfloat16().to(dev), False)):
+        ys = []
+        for name, tail in (("tbf16_linear", (work.data_ptr(), _ext.stream())), ("tbf16_linear_noalloc", (_ext.stream(),))):
+            y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+            _ext.call(name, x.data_ptr(), M, K, K, b16.data_ptr(), N, K, ones.data_ptr(), None, y.data_ptr(), N, 15, 0, -1,
+                      *tail)
+            ys.append(y.cpu())
+        assert torch.equal(ys[0], ys[1])
+        if exact:
+            assert torch.equal(ys[0], (a.double() @ b.double().t()).bfloat16())
+
+
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("M,N,K", [(2, 1, 64), (17, 9, 4096), (100, 515, 200), (300, 2049, 520), (64, 32001, 64), (2, 257, 16392)])
 def test_linear_any_n(dev, M, N, K, bias):

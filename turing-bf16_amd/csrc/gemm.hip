@@ -1,12 +1,24 @@
 // Scaled GEMM on CDNA4 fp16 MFMA: y = bf16(acc * sa[m] * sb[n] + bias[n]) with
 // acc[m, n] = sum_k a16[m, k] * b16[n, k] in fp32.
 //
-// a is either already fp16 (a16 with fp32 inverse row scales sa) or bf16 that is
-// converted to fp16 with an exact per-row power of two 2^p[m] on its way from
-// registers into LDS, sa = 2^-p[m] (the fused path, tbf16/csrc/gemm_sm75.cu:78-226).
-// b is fp16 (prepare_weight's w16) with fp32 inverse row scales sb.
+// b is fp16 (prepare_weight's w16) with fp32 inverse row scales sb. a is fp16 too (a16
+// with fp32 inverse row scales sa: tbf16_linear's own scaled copy of x, one row pass), or
+// bf16 converted to fp16 with an exact per-row power of two 2^p[m], sa = 2^-p[m], on its
+// way from registers into LDS (the fused path, tbf16/csrc/gemm_sm75.cu:78-226).
 //
-// Tiling (gfx950, 64-wide waves, 160 KB LDS):
+// Kernels, all for 64-wide waves and 160 KB LDS; the dispatch (pick_f16, pick_fused) says
+// where each runs, and its configuration number pins it:
+//  - pingpong_kernel, fp16 a: large tiles, two wave groups alternating MFMAs and loads.
+//  - ksplit_kernel, fp16 a: small tiles (decode to mid-size M), the groups on alternate k
+//    tiles; also the implicit convolutions.
+//  - gemm_kernel: the form that converts bf16 a in its staging (tbf16_linear_exps, and
+//    the no-allocation entry point where x16 does not fit its array).
+//  - skinny_kernel: the same at M <= 32, K split across waves.
+//  - stream_kernel: decode on fp16 a with plain waves, by configuration number only:
+//    ksplit_kernel's 64-row tiles replaced it in the dispatch (16 x 2560 -> 10240: 17.3
+//    -> 15.5 us a call).
+//
+// gemm_kernel's tiling:
 //  - block tile BM (rows of a) x BN (rows of b), k tile BK (32 or 64); WM x WN
 //    waves, each owning a (BM/WM) x (BN/WN) sub-tile made of 32x32 MFMA blocks
 //    (v_mfma_f32_32x32x16_f16: 16 fp32 accumulators per lane per block).
@@ -15,7 +27,7 @@
 //    fragment reads (ds_read_b128) and the row stores are bank-conflict free.
 //  - PF register sets are in flight: each k tile's global loads are issued PF
 //    compute phases before they are stored to LDS.
-//  - the headline shape (config 9) uses BK = 64, so that every global load
+//  - the largest tile (config 9) uses BK = 64, so that every global load
 //    instruction covers whole 128-byte row segments: half the L2 requests of
 //    BK = 32, which measurably raises the clock the chip holds under this
 //    kernel. Two LDS stages of 64 KB; fragments are read one 16-wide k step
@@ -26,18 +38,16 @@
 //  - config 0 (BK = 32, three LDS stages in a ring, the next tile's first
 //    fragments read before the barrier) and the plain two-stage loop of the
 //    smaller tiles remain selectable.
+// Common to the tile kernels:
 //  - the MFMA's first operand is the b fragment, the second the a fragment, so a
-//    lane's 16 accumulators are four runs of 4 consecutive n for one m. The
-//    epilogue applies the scales and bias in fp32 straight from the
-//    accumulators, rounds once to bf16 and regroups lanes with three register
-//    exchanges (v_permlane32_swap, v_permlane16_swap, a DPP row_ror:8), so each
-//    store instruction writes whole 128-byte rows with no LDS round trip or
-//    barrier (plain 8-byte stores from the accumulators were written back in
-//    partial sectors).
+//    lane's accumulators are runs of 4 consecutive n for one m. The epilogues
+//    apply the scales and bias in fp32 straight from the accumulators, round
+//    once to bf16 and regroup lanes with register exchanges, so each store
+//    instruction writes whole 128-byte rows with no LDS round trip or barrier
+//    (plain 8-byte stores from the accumulators were written back in partial
+//    sectors).
 //  - block ids are remapped so that each XCD (8 per chip, round-robin dispatch)
 //    gets a contiguous range of tiles, grouped 8 a-tiles deep for L2 reuse.
-// M <= 64 (decode) uses a separate skinny kernel that splits K across waves
-// (see skinny_kernel below).
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -566,8 +576,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(const uint16_t* __res
 
 // Epilogue of a wave's TM x TN sub-tile made of 16x16 MFMA blocks: acc[i][j] holds
 // columns 16 i and rows 16 j, lane l columns 4 (l / 16) .. + 3 of row l % 16. The same
-// fp32 arithmetic as store_tile; part: the raw fp32 sums, row stride ldp. v_permlane16_swap pairs column blocks 2 p and 2 p + 1
-// between 16-lane rows, so a lane holds 16 bytes of its row (columns 0 / 16 / 8 / 24 of
+// fp32 arithmetic as store_tile; part: the raw fp32 sums, row stride ldp.
+// v_permlane16_swap pairs column blocks 2 p and 2 p + 1 between 16-lane rows, so a lane holds 16 bytes of its row (columns 0 / 16 / 8 / 24 of
 // the 32-column pair for l / 16 = 0 / 1 / 2 / 3); with two pairs, a DPP row_ror:8
 // exchange between lanes l and l ^ 8 makes each store write whole 128-byte rows.
 template <int TM, int TN>
@@ -1944,18 +1954,28 @@ LinearWs layout_ws(int64_t M, int64_t K, int64_t N, int cfg, int splits, bool q1
   }
   return w;
 }
+// Rows a call of the no-allocation entry point's array takes at once: their scales, x16
+// and partial sums, a multiple of 64 (0: not even 64 rows).
+int64_t scratch_rows(int64_t K, int64_t N, int splits) {
+  const int64_t per_row = 2 * K + 12 + (splits > 1 ? (int64_t)splits * N * 4 : 0);
+  return (TBF16_NOALLOC_SCRATCH_BYTES - 1024) / per_row / 64 * 64;
+}
 // The dispatcher's choice (cfg < 0): x quantised once and a kernel on fp16 operands,
 // also for wide tiles (4096^3: 101 us + 9 us of row pass against 118 + 5 with the
-// conversion in the GEMM). Where that workspace would not fit the no-allocation entry
-// point's array, only kernels whose output the converting tiles reproduce bit for bit,
-// which that entry point then runs.
-LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg) {
+// conversion in the GEMM). For at most 32 rows a kernel that would split K is not worth
+// its third launch: the skinny kernel converting x itself takes two (6x3712x2640: 17.2 us
+// a call against 18.9); ragged: N is not the caller's, which that kernel cannot take.
+// Where that workspace would not fit the no-allocation entry point's array, a kernel
+// whose output that entry point reproduces bit for bit: the converting tiles do k
+// ascending, row chunks of the same configuration anything that takes 64 rows.
+LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg, bool ragged = false) {
   if (cfg >= 0) return layout_ws(M, K, N, cfg, pick_split(cfg, M, N, K), quantize_once(cfg, K));
   const size_t base = layout_ws(M, K, N, 20, 1, true).bytes;
-  const bool bounded = base > TBF16_NOALLOC_SCRATCH_BYTES;
-  const F16Pick p = pick_f16(M, N, K, true,
-                             bounded ? kSplitPartBytes : std::min<size_t>(kSplitPartBytes, TBF16_NOALLOC_SCRATCH_BYTES - base),
+  const bool over = base > TBF16_NOALLOC_SCRATCH_BYTES, bounded = over && scratch_rows(K, N, 1) == 0;
+  const F16Pick p = pick_f16(M, N, K, !over || bounded || scratch_rows(K, N, 8) > 0,
+                             over ? kSplitPartBytes : std::min<size_t>(kSplitPartBytes, TBF16_NOALLOC_SCRATCH_BYTES - base),
                              bounded);
+  if (M <= 32 && p.splits > 1 && !ragged) return layout_ws(M, K, N, pick_fused(M, N, false), 1, false);
   return layout_ws(M, K, N, p.cfg, p.splits, true);
 }
 // The form that converts x inside the GEMM, the same output bits: the pinned
@@ -1987,7 +2007,8 @@ int linear_into(const LinearWs& w, const void* x, int64_t M, int64_t K, int64_t 
 extern "C" size_t tbf16_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int cfg) {
   if (M <= 0 || K < 0 || N <= 0 || cfg >= kNumCfgs) return M > 0 ? (size_t)M * 4 : 0;
   // enough for either form of the call
-  return std::max(linear_ws(M, K, N, cfg).bytes, layout_ws(M, K, N, 0, cfg < 0 ? pick_split(12, M, N, K) : 1, false).bytes);
+  return std::max(std::max(linear_ws(M, K, N, cfg).bytes, linear_ws(M, K, N, cfg, true).bytes),
+                  layout_ws(M, K, N, 0, cfg < 0 ? pick_split(12, M, N, K) : 1, false).bytes);
 }
 
 extern "C" int tbf16_linear(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w16, int64_t N,
@@ -2010,7 +2031,7 @@ extern "C" int tbf16_linear_any_n(const void* x, int64_t M, int64_t K, int64_t l
   TB_CHECK(ws != nullptr && aligned4(ws), "linear_any_n: bad scales");
   TB_CHECK((workspace != nullptr && aligned16(workspace)) || M == 0, "linear_any_n: workspace missing or misaligned");
   if (M == 0 || N == 0) return 0;
-  return linear_into(linear_ws(M, K, Np, -1), x, M, K, ldx, w16, Np, ldw, ws, bias, y, ldy, t, l1,
+  return linear_into(linear_ws(M, K, Np, -1, true), x, M, K, ldx, w16, Np, ldw, ws, bias, y, ldy, t, l1,
                      static_cast<uint8_t*>(workspace), as_stream(stream), N);
 }
 
@@ -2062,18 +2083,31 @@ extern "C" int tbf16_linear_noalloc(const void* x, int64_t M, int64_t K, int64_t
              "linear_noalloc: cannot query the stream's device");
     TB_CHECK(sd == cur, "linear_noalloc: the stream belongs to device %d, the current device is %d", (int)sd, cur);
   }
-  // where the fp16 copy of x does not fit, a tile configuration converts x inside
-  // the GEMM instead (the same output), except at decode sizes and in the kernels that
+  // where the fp16 copy of x does not fit, the dispatcher's choice runs over chunks of
+  // rows if it adds over alternate k tiles or more than two splits, else a tile configuration converts x inside
+  // the GEMM instead (the same output); except at decode sizes and in the kernels that
   // take fp16 a only, whose calls are rejected
   LinearWs w = linear_ws(M, K, N, cfg);
   const bool f16_only = cfg >= 0 ? kCfgs[cfg].stream || kCfgs[cfg].pingpong : M <= 128 && N >= 32 * num_cus();
-  if (w.bytes > TBF16_NOALLOC_SCRATCH_BYTES && !f16_only) w = fused_ws(M, K, N, cfg);
+  int64_t rows = M;
+  if (w.bytes > TBF16_NOALLOC_SCRATCH_BYTES && !f16_only) {
+    if (cfg < 0 && w.q16 && (kCfgs[w.cfg].ksplit || w.splits > 2)) {
+      rows = cdiv(cdiv(M, cdiv(M, scratch_rows(K, N, w.splits))), 64) * 64;
+      w = layout_ws(rows, K, N, w.cfg, w.splits, true);
+    } else {
+      w = fused_ws(M, K, N, cfg);
+    }
+  }
   TB_CHECK(w.bytes <= TBF16_NOALLOC_SCRATCH_BYTES,
            "linear_noalloc: %lld x %lld needs %zu workspace bytes, beyond the scratch limit of %d bytes", (long long)M,
            (long long)K, w.bytes, TBF16_NOALLOC_SCRATCH_BYTES);
   uint8_t* wsp = nullptr;
   if (int rc = scratch_ptr(&wsp)) return rc;
-  return linear_into(w, x, M, K, ldx, w16, N, ldw, ws, bias, y, ldy, t, l1, wsp, st);
+  for (int64_t m = 0; m < M; m += rows)
+    if (int rc = linear_into(w, static_cast<const uint16_t*>(x) + m * ldx, std::min(rows, M - m), K, ldx, w16, N, ldw, ws,
+                             bias, static_cast<uint16_t*>(y) + m * ldy, ldy, t, l1, wsp, st))
+      return rc;
+  return 0;
 }
 
 // ---- implicit convolution ---------------------------------------------------------
