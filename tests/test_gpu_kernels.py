@@ -405,6 +405,15 @@ def test_attention_causal_block_forms(dev, monkeypatch, B, H, S, D, layout, spli
     _attn_checks(q, k, v, dev, label=f"split={split} k={kform} {layout} B={B} H={H} S={S} D={D}")
 
 
+@pytest.mark.parametrize("H,S,D", [(1, 129, 128), (150, 200, 64), (170, 200, 64), (170, 300, 128), (280, 200, 64), (390, 200, 64)])
+def test_attention_causal_grids(dev, H, S, D):
+    """The causal grids on both sides of each line: single split-key tiles, pairs in one
+    round, single tiles where the pairs are just more than a round, 256-row blocks."""
+    g = torch.Generator().manual_seed(H)
+    q, k, v = (torch.randn(1, H, S, D, generator=g).bfloat16() for _ in range(3))
+    _attn_checks(q, k, v, dev, label=f"H={H} S={S} D={D}")
+
+
 @pytest.mark.parametrize("split", ["0", "1"])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("Sq,Sk,D", [(33, 65, 64), (130, 257, 128), (200, 127, 96), (257, 64, 64), (16, 3, 128)])

@@ -443,7 +443,7 @@ attn_fwd_kernel(FwdParams p) {
     acc_o[1].clear();
     // running max in log2 units; stays stale until a row's max grows by more than
     // 2^8, so exp2 arguments are <= 8 and P <= 256 (fp16-safe)
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+    float m_run[2] = {-INFINITY, -INFINITY}, mneg[2] = {0.f, 0.f}, l_run[2] = {0.f, 0.f};
     const float c = HAS_BIAS ? 1.f : p.scale_log2;
 
     const int nkb_all = (p.Sk + BKV - 1) / BKV;
@@ -573,14 +573,17 @@ attn_fwd_kernel(FwdParams p) {
         for (int i = 0; i < 4; ++i)
   #pragma unroll
           for (int r = 0; r < 4; ++r) mx[qb] = fmaxf(mx[qb], sacc[i][qb][r]);
-        mx[qb] = max_xor32(max_xor16(mx[qb])) * c;
       }
-      if (__any(mx[0] > m_run[0] + 8.f || mx[1] > m_run[1] + 8.f)) {  // wave-uniform: rescale only when some row needs it
+      // wave-uniform: rescale only when some row needs it. Some lane's own maximum says
+      // so exactly when a row's does, so the row maxima (exchanges between the four
+      // lanes of a row, a serial chain each tile) are only taken here.
+      if (__any(mx[0] * c > m_run[0] + 8.f || mx[1] * c > m_run[1] + 8.f)) {
   #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-          const float m_new = fmaxf(m_run[qb], mx[qb]);
+          const float m_new = fmaxf(m_run[qb], max_xor32(max_xor16(mx[qb])) * c);
           const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run[qb] - m_new);
           m_run[qb] = m_new;
+          mneg[qb] = (m_new == -INFINITY) ? 0.f : -m_new;
           l_run[qb] *= alpha;
           acc_o[qb].scale(alpha);
         }
@@ -591,7 +594,6 @@ attn_fwd_kernel(FwdParams p) {
       half8 pf[2][2];
   #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
-        const float mneg = (m_run[qb] == -INFINITY) ? 0.f : -m_run[qb];
         float lsum = 0.f;
   #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -599,8 +601,8 @@ attn_fwd_kernel(FwdParams p) {
   #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int i = 2 * g + (j >> 1), r = 2 * (j & 1);
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[i][qb][r], c, mneg));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[i][qb][r + 1], c, mneg));
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[i][qb][r], c, mneg[qb]));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[i][qb][r + 1], c, mneg[qb]));
             w[j] = pack_f16(p0, p1);
             lsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, w[j]), ones, lsum, false);
             if constexpr (DROP) {  // l keeps the undropped weights; the PV product gets the kept ones,
@@ -871,18 +873,27 @@ int launch_fwd_nw(const FwdParams& p, bool causal, bool has_bias, bool split, di
 template <int DP>
 int launch_fwd_dp(FwdParams p, bool causal, bool has_bias, hipStream_t st, int nw_override) {
   const int64_t tiles8 = cdiv(p.Sq, 256) * p.B * p.H, tiles4 = cdiv(p.Sq, 128) * p.B * p.H;
-  // causal with few blocks: 4-wave blocks that pair a heavy and a light query
-  // tile, so every block has the same work (heaviest-first ordering only
-  // balances many rounds); otherwise as measured above
-  const bool pair = causal && tiles4 >= 2 * p.B * p.H && tiles8 < 384 && nw_override <= 0 &&
-                    getenv("TBF16_ATTN_NOPAIR") == nullptr;
-  // the paired grid, and any grid whose 128-row tiles are no more than the CUs, run as
   // split-key 8-wave blocks where those exist (no dropout, head dim <= 128): two waves
-  // per SIMD instead of one (key-padding mask, 24 heads, S = 1111, D = 64: kernel 36.6 ->
-  // 29.2 us); TBF16_ATTN_SPLIT=0 / 1 turns that off / on for any grid (benchmarking)
+  // per SIMD instead of one
   const char* sv = getenv("TBF16_ATTN_SPLIT");
-  const bool split_ok = DP <= 128 && !p.drop_thr && nw_override <= 0;
-  const bool split = split_ok && (sv ? atoi(sv) != 0 : pair || tiles4 <= num_cus());
+  const bool split_ok = DP <= 128 && !p.drop_thr && nw_override <= 0 && (!sv || atoi(sv) != 0);
+  // causal with few blocks: blocks that pair a heavy and a light 128-row query tile, so
+  // that every block has the same work (heaviest-first ordering only balances many
+  // rounds). A pair pays for two prologues, merges and epilogues (about 9 key tiles'
+  // time), so single split-key tiles, the heaviest first, are better while the heaviest
+  // one bounds the grid anyway: heads x (tiles + 1) well below two CU counts (D = 128, per
+  // call, paired -> single: 8 heads, S = 900 37.7 -> 28.2 us, 16 heads, S = 2399 60.5 ->
+  // 53.9, S = 3500 78.2 -> 76.6, S = 4096 88.0 -> 90.6), and where the pairs would be a
+  // little more than one round (24 heads, S = 3000 127.4 -> 94.3; 1.5 rounds of pairs, 64
+  // heads, S = 1500: 69.5 -> 80.3).
+  const int64_t heads = (int64_t)p.B * p.H, n4 = cdiv(p.Sq, 128), pairs = heads * cdiv(n4, 2), cus = num_cus();
+  const bool single = split_ok && (10 * heads * (n4 + 1) <= 18 * cus || (pairs > cus && 10 * pairs <= 13 * cus));
+  const bool few = causal && n4 >= 2 && tiles8 < 384 && nw_override <= 0;
+  const bool pair = few && !single && getenv("TBF16_ATTN_NOPAIR") == nullptr;
+  // the paired and single causal grids, and any grid whose 128-row tiles are no more than
+  // the CUs, run as split-key blocks (key-padding mask, 24 heads, S = 1111, D = 64: kernel
+  // 36.6 -> 29.2 us); TBF16_ATTN_SPLIT=0 / 1 turns that off / on for any grid (benchmarking)
+  const bool split = split_ok && (sv || pair || (few && single) || tiles4 <= cus);
   int nw = nw_override > 0 ? nw_override : pair ? 4 : (tiles8 >= 128 ? 8 : 4);
   if (DP > 128 || p.drop_thr) nw = 4;
   if (split) nw = 8;
