@@ -104,7 +104,7 @@ int tbf16_gemm_f16_any_n(const void* a16, int64_t M, int64_t K, int64_t lda, con
  * (12 MiB, held until the process ends). No counterpart in the reference: it is
  * for callers that cannot allocate (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc). Where x's fp16 copy does not fit in the array,
- * a tile configuration converts x inside the GEMM instead (the same output); M
+ * it is made in chunks of rows or x is converted inside the GEMM (the same output); M
  * above TBF16_NOALLOC_MAX_ROWS, or a decode-sized call (M <= 128) whose copy does
  * not fit (K beyond ~48k at M = 128), is rejected (TBF16_EINVAL). The array used is
  * the current device's, so the stream must belong to the current device (a stream

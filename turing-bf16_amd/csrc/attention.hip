@@ -17,10 +17,10 @@
 // Block = 4 or 8 waves, 32 query rows per wave; key tiles of 64.
 //  - a wave keeps its 32 q rows as MFMA fragments in registers for the whole
 //    kernel and computes S^T = K Q^T with 16x16x32 MFMAs (K from LDS), so each lane
-//    owns two query rows, 16 apart: row max / sum need exchanges with lanes ^ 16 and
-//    ^ 32. Long sequences run at the clock that the chip's power allows, and this MFMA
+//    owns two query rows, 16 apart; row maxima and sums need exchanges with lanes ^ 16
+//    and ^ 32, outside the key loop but for the rare rescale. Long sequences run at the clock that the chip's power allows, and this MFMA
 //    shape costs less of it than 32x32x16: 16k causal, 16 heads, D = 128, 1.85 -> 1.90
-//    GHz and 1035 -> 984 us a call.
+//    GHz and 1035 -> 984 us a call (955 with the maxima out of the loop).
 //  - online softmax in fp32, base 2 (logit * scale * log2 e), P rounded to fp16.
 //  - O^T = V^T P^T: V is stored transposed in LDS (d-major, keys permuted within
 //    each 32-key group, vt_run) so that the A fragment of a lane is one 16-byte read
@@ -29,8 +29,8 @@
 //  - row sums l come from the fp16 P that enters the PV product (v_dot2 with
 //    ones), so the normalisation matches the weights actually applied.
 //  - output bf16(O / l * 2^ev) written from registers: one rounding.
-// Causal blocks are launched heaviest first, or (few blocks per CU) each takes a
-// heavy and a light query tile; key tiles past the diagonal are skipped, and
+// Causal blocks are launched heaviest first, or (about one round of them) each takes
+// a heavy and a light query tile; key tiles past the diagonal are skipped, and
 // only tiles crossing the diagonal or the end of the keys run the masked copy of
 // the tile loop.
 #include <stdlib.h>

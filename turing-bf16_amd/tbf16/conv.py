@@ -7,7 +7,7 @@ one pass that writes bf16. The weight conversion is lossless; the input's is
 lossless for every element within 2^14 of its sample's max (smaller ones become
 fp16 subnormals, far below the output's bf16 rounding).
 
-On MI355X a 2-D convolution of some size runs whole on the library's kernels
+On MI355X a 2-D convolution of some size runs whole on this library's kernels
 (tbf16_conv2d: per-sample maxima, one scaled channels-last copy of the input, an
 implicit GEMM that writes bf16 from its fp32 sums). For the others the passes around the
 convolution are HIP kernels (tbf16_conv_input: per-sample max, exponent and scaled fp16
