@@ -190,15 +190,16 @@ int tbf16_conv_epilogue(const void* y16, int64_t B, int64_t O, int64_t P, int ch
 
 /* The whole scaled 2-D convolution (tbf16/conv.py:39-60; one group, zero padding): x bf16
  * (B, C, H, W), contiguous or (channels_last, C % 8 == 0) channels last, each sample scaled
- * as tbf16_conv_input does at t; w16 fp16 (O, C, KH, KW) contiguous with its inverse scales
- * per channel; bias bf16 (O,) or NULL; y bf16 in x's layout, rounded once from fp32. stride,
+ * as tbf16_conv_input does at t; w16 fp16 (O, Cw, KH, KW) contiguous, Cw = C (anything else is
+ * rejected), with its inverse scales per channel; bias bf16 (O,) or NULL; y bf16 in x's layout, rounded once from fp32. stride,
  * pad and dilation: two each. Replaces the reference's cuDNN call and the passes
  * around it. A size query returns 0 for sizes the kernels do not take. */
 size_t tbf16_conv2d_ws_bytes(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW,
                              const int64_t* stride, const int64_t* pad, const int64_t* dilation);
 int tbf16_conv2d(const void* x, int64_t B, int64_t C, int64_t H, int64_t W, int channels_last, int t, const void* w16,
-                 int64_t O, int64_t KH, int64_t KW, const int64_t* stride, const int64_t* pad, const int64_t* dilation,
-                 const float* w_sinv, const void* bias, void* y, void* ws, int64_t ws_bytes, void* stream);
+                 int64_t O, int64_t Cw, int64_t KH, int64_t KW, const int64_t* stride, const int64_t* pad,
+                 const int64_t* dilation, const float* w_sinv, const void* bias, void* y, void* ws, int64_t ws_bytes,
+                 void* stream);
 
 /* Scaled attention forward (flash-style, no S x S buffer).
  * Exponents (tbf16/attention.py:38-48): eq/ek = max over heads of frexp(amax),

@@ -1,0 +1,53 @@
+"""Which native call a public entry point makes, and what it refuses, with the launches
+replaced: no GPU needed."""
+import ctypes
+
+import pytest
+import torch
+import torch.nn as nn
+
+from tbf16 import _ext
+from tbf16 import conv as tconv
+
+
+def _converted(C, O, k=3, **kw):
+    """A converted Conv2d on the CPU (convert_conv without its quantisation kernel)."""
+    m = nn.Conv2d(C, O, k, **kw).bfloat16()
+    w16 = m.weight.detach().half()
+    m.weight = None
+    m.register_buffer("weight16", w16)
+    m.register_buffer("weight_scale", torch.ones(O))
+    m._tbf16_plan = tconv.ConvPlan(0, tconv._pointwise(m))
+    m.__class__ = tconv._scaled_class(type(m))
+    return m
+
+
+@pytest.fixture
+def conv_calls(monkeypatch):
+    """The native calls that a converted convolution on CPU tensors would launch."""
+    calls = []
+    monkeypatch.setattr(tconv, "_dev_check", lambda *ts: None)
+    monkeypatch.setattr(tconv, "launch", lambda name, *args: calls.append(name))
+    monkeypatch.setattr(tconv, "scale_input", lambda x, t: (torch.zeros(x.shape[0], dtype=torch.int32), x.half()))
+    monkeypatch.setattr(tconv, "unscale_output", lambda y16, *args: y16.bfloat16())
+    return calls
+
+
+@pytest.mark.parametrize("C", [256, 1024, 4])
+@pytest.mark.parametrize("cl", [False, True])
+def test_conv2d_of_other_channel_counts_is_refused(conv_calls, C, cl):
+    m = _converted(512, 512, padding=1)
+    fmt = torch.channels_last if cl else torch.contiguous_format
+    with torch.no_grad():
+        m(torch.zeros(1, 512, 64, 64, dtype=torch.bfloat16).to(memory_format=fmt))
+        assert conv_calls == ["tbf16_conv2d"]
+        with pytest.raises(RuntimeError, match="channels"):  # torch's own error
+            m(torch.zeros(1, C, 64, 64, dtype=torch.bfloat16).to(memory_format=fmt))
+    assert conv_calls == ["tbf16_conv2d"]
+
+
+def test_conv2d_entry_point_refuses_other_channel_counts():
+    two = (ctypes.c_int64 * 2)(1, 1)
+    for C in (256, 1024):
+        rc = _ext.lib().tbf16_conv2d(16, 1, C, 64, 64, 0, 0, 16, 512, 512, 3, 3, two, two, two, 16, None, 16, 16, 1 << 40, None)
+        assert rc == -1 and "channels" in _ext.lib().tbf16_last_error().decode()

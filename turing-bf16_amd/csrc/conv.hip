@@ -438,9 +438,10 @@ extern "C" size_t tbf16_conv2d_ws_bytes(int64_t B, int64_t C, int64_t H, int64_t
 }
 
 extern "C" int tbf16_conv2d(const void* x, int64_t B, int64_t C, int64_t H, int64_t W, int channels_last, int t,
-                            const void* w16, int64_t O, int64_t KH, int64_t KW, const int64_t* stride, const int64_t* pad,
-                            const int64_t* dilation, const float* w_sinv, const void* bias, void* y, void* ws,
-                            int64_t ws_bytes, void* stream) {
+                            const void* w16, int64_t O, int64_t Cw, int64_t KH, int64_t KW, const int64_t* stride,
+                            const int64_t* pad, const int64_t* dilation, const float* w_sinv, const void* bias, void* y,
+                            void* ws, int64_t ws_bytes, void* stream) {
+  TB_CHECK(Cw == C, "conv2d: the input has %lld channels, the weight %lld", (long long)C, (long long)Cw);
   Conv2dPlan p;
   if (int rc = conv2d_plan(B, C, H, W, O, KH, KW, stride, pad, dilation, p)) return rc;
   TB_CHECK(x && w16 && w_sinv && y && aligned16(x) && aligned16(y), "conv2d: null or misaligned pointer");

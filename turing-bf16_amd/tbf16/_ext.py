@@ -56,7 +56,7 @@ _SIGS = {
     "tbf16_conv_input": (I, [P, I64, I64, I, P, P, P, I64, P]),
     "tbf16_conv_epilogue": (I, [P, I64, I64, I64, I, P, P, P, P, P]),
     "tbf16_conv2d_ws_bytes": (SZ, [I64] * 7 + [PI64] * 3),
-    "tbf16_conv2d": (I, [P, I64, I64, I64, I64, I, I, P, I64, I64, I64, PI64, PI64, PI64, P, P, P, P, I64, P]),
+    "tbf16_conv2d": (I, [P, I64, I64, I64, I64, I, I, P, I64, I64, I64, I64, PI64, PI64, PI64, P, P, P, P, I64, P]),
     "tbf16_attn_fwd_ws_bytes": (SZ, [I64, I64, I64, I64, I64, I64]),
     "tbf16_attn_fwd": (I, [P, P, P, I64, I64, I64, I64, I64, I64, PI64, PI64, PI64, P, PI64, F, I, I, F, U64, P, P, P, P,
                            P, I64, P]),

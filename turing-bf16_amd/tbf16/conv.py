@@ -107,12 +107,14 @@ _NATIVE_MIN_MACS = 1 << 29
 def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
     """0 (contiguous) or 1 (channels last) when the native 2-D convolution takes this
     call, else None: one group, zero padding given in numbers, a bf16 bias, an input
-    dense in exactly one of the two layouts.
+    dense in exactly one of the two layouts, as many channels as the weight has (the
+    library's convolution refuses any other input).
     Small convolutions (_NATIVE_MIN_MACS) keep the library's fp16 convolution and its
     fp16 rounding: their results are pinned bit for bit to the reference's formula on
     that call. The native kernel is the faster one there too (64 -> 64 at 16 x 16: 22 us
     against 51)."""
-    if (x.dim() != 4 or conv.groups != 1 or isinstance(padding, str) or x.numel() == 0 or x.data_ptr() % 16
+    if (x.dim() != 4 or conv.weight16.dim() != 4 or x.shape[1] != conv.weight16.shape[1] or conv.groups != 1
+            or isinstance(padding, str) or x.numel() == 0 or x.data_ptr() % 16
             or not conv.weight16.is_contiguous() or (bias is not None and bias.dtype != torch.bfloat16)):
         return None
     nchw, nhwc = x.is_contiguous(), x.is_contiguous(memory_format=torch.channels_last)
@@ -133,7 +135,7 @@ def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int)
     do not take."""
     B, C, H, W = x.shape
     w16 = conv.weight16
-    O, _, KH, KW = w16.shape
+    O, Cw, KH, KW = w16.shape
     pad = (padding, padding) if isinstance(padding, int) else padding
     stride, dilation = conv.stride, conv.dilation
     geom = (_pair(stride), _pair(pad), _pair(dilation))
@@ -148,8 +150,8 @@ def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int)
     ws = torch.empty(wsb, device=x.device, dtype=torch.uint8)
     b = None if bias is None else bias.detach().contiguous()
     s = conv.weight_scale.float().contiguous()
-    launch("tbf16_conv2d", x, ptr(x), B, C, H, W, layout, int(conv._tbf16_plan.target_exp), ptr(w16), O, KH, KW, *geom,
-           ptr(s), ptr(b), ptr(y), ptr(ws), wsb)
+    launch("tbf16_conv2d", x, ptr(x), B, C, H, W, layout, int(conv._tbf16_plan.target_exp), ptr(w16), O, Cw, KH, KW,
+           *geom, ptr(s), ptr(b), ptr(y), ptr(ws), wsb)
     return y
 
 
