@@ -471,3 +471,20 @@ def test_autograd_linear_one_call_matches_passes(dev, monkeypatch, M, K, N, grad
             assert ((a.float() - e.float()).abs() <= bound).all()
         else:
             assert torch.equal(a, e)
+
+
+@pytest.mark.parametrize("grads", ["x"])
+@pytest.mark.parametrize("M,K,N", [(10, 16, 12), (100, 264, 75), (37, 1024, 32001)])
+def test_autograd_linear_any_n(dev, M, K, N, grads):
+    """The training linear whose N is no multiple of 8 (an odd vocabulary head), with a bias,
+    for sets of wanted gradients, against fp64: bf16 results of fp32 sums (1.7e-3 from
+    their rounding)."""
+    import tbf16.autograd as ag
+    x, w, b, dy = (randn(*s, seed=40 + i).bfloat16().to(dev) for i, s in enumerate(((M, K), (N, K), (N,), (M, N))))
+    leaves = [t.requires_grad_(c in grads) for t, c in zip((x, w, b), "xwb")]
+    y = ag.linear(*leaves)
+    assert rel(y, x.double() @ w.double().t() + b.double()) < 3e-3
+    got = torch.autograd.grad(y, [t for t in leaves if t.requires_grad], dy)
+    ref = {"x": dy.double() @ w.double(), "w": dy.double().t() @ x.double(), "b": dy.double().sum(0)}
+    for c, t in zip(grads, got):
+        assert t.shape == ref[c].shape and rel(t, ref[c]) < 3e-3, c

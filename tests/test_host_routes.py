@@ -51,3 +51,30 @@ def test_conv2d_entry_point_refuses_other_channel_counts():
     for C in (256, 1024):
         rc = _ext.lib().tbf16_conv2d(16, 1, C, 64, 64, 0, 0, 16, 512, 512, 3, 3, two, two, two, 16, None, 16, 16, 1 << 40, None)
         assert rc == -1 and "channels" in _ext.lib().tbf16_last_error().decode()
+
+
+@pytest.fixture
+def linear_calls(monkeypatch):
+    """The native calls of the training linear on CPU tensors, as (name, arguments)."""
+    from tbf16 import autograd, ops, routing
+    calls = []
+    monkeypatch.setattr(ops, "_dev_check", lambda *ts: None)
+    for mod in (ops, autograd):
+        monkeypatch.setattr(mod, "launch", lambda name, where, *args: calls.append((name, args)))
+    routing.activations.clear()
+    yield calls
+    routing.activations.clear()
+
+
+@pytest.mark.parametrize("N", [12, 1025])
+def test_linear_input_gradient_of_any_n(linear_calls, N):
+    """dX = dY W of a frozen layer whose N is no multiple of 8: the product's two operands
+    have one (padded) contraction length."""
+    from tbf16 import autograd
+    x = torch.zeros(10, 16, dtype=torch.bfloat16, requires_grad=True)
+    y = autograd.linear(x, torch.zeros(N, 16, dtype=torch.bfloat16))
+    assert y.shape == (10, N)
+    (dx,) = torch.autograd.grad(y, [x], torch.zeros(10, N, dtype=torch.bfloat16))
+    assert dx.shape == (10, 16)
+    name, args = linear_calls[-1]
+    assert name == "tbf16_gemm_f16" and args[1:4] == (10, N + -N % 8, N + -N % 8)
