@@ -473,11 +473,11 @@ def test_autograd_linear_one_call_matches_passes(dev, monkeypatch, M, K, N, grad
             assert torch.equal(a, e)
 
 
-@pytest.mark.parametrize("grads", ["x"])
-@pytest.mark.parametrize("M,K,N", [(10, 16, 12), (100, 264, 75), (37, 1024, 32001)])
+@pytest.mark.parametrize("grads", ["x", "xwb", "w"])
+@pytest.mark.parametrize("M,K,N", [(10, 16, 12), (100, 264, 75), (37, 1024, 32001), (33, 30, 40), (65, 77, 19)])
 def test_autograd_linear_any_n(dev, M, K, N, grads):
-    """The training linear whose N is no multiple of 8 (an odd vocabulary head), with a bias,
-    for sets of wanted gradients, against fp64: bf16 results of fp32 sums (1.7e-3 from
+    """The training linear whose N or K is no multiple of 8 (an odd vocabulary head), with a
+    bias, for sets of wanted gradients, against fp64: bf16 results of fp32 sums (1.7e-3 from
     their rounding)."""
     import tbf16.autograd as ag
     x, w, b, dy = (randn(*s, seed=40 + i).bfloat16().to(dev) for i, s in enumerate(((M, K), (N, K), (N,), (M, N))))

@@ -78,3 +78,12 @@ def test_linear_input_gradient_of_any_n(linear_calls, N):
     assert dx.shape == (10, 16)
     name, args = linear_calls[-1]
     assert name == "tbf16_gemm_f16" and args[1:4] == (10, N + -N % 8, N + -N % 8)
+
+
+@pytest.mark.parametrize("K,N", [(16, 12), (30, 40), (13, 1025)])
+def test_linear_gradients_have_their_leaves_shapes(linear_calls, K, N):
+    from tbf16 import autograd
+    leaves = [torch.zeros(*s, dtype=torch.bfloat16, requires_grad=True) for s in ((10, K), (N, K), (N,))]
+    y = autograd.linear(*leaves)
+    grads = torch.autograd.grad(y, leaves, torch.zeros(10, N, dtype=torch.bfloat16))
+    assert [g.shape for g in grads] == [t.shape for t in leaves]
