@@ -87,3 +87,24 @@ def test_linear_gradients_have_their_leaves_shapes(linear_calls, K, N):
     y = autograd.linear(*leaves)
     grads = torch.autograd.grad(y, leaves, torch.zeros(10, N, dtype=torch.bfloat16))
     assert [g.shape for g in grads] == [t.shape for t in leaves]
+
+
+def test_linear_refuses_host_tensors(linear_calls, monkeypatch):
+    """A weight (or a saved tensor that a hook unpacked) in host memory raises before any
+    launch: its address must not reach a kernel."""
+    from tbf16 import autograd, ops
+    monkeypatch.undo()  # the real device check
+    calls = []
+    for mod in (ops, autograd):
+        monkeypatch.setattr(mod, "launch", lambda name, where, *args: calls.append(name))
+    x = torch.zeros(16, 16, dtype=torch.bfloat16, requires_grad=True)
+    w = torch.zeros(24, 16, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="device"):
+        autograd.linear(x, w)
+    assert calls == []
+    checked = []
+    monkeypatch.setattr(ops, "_dev_check", lambda *ts: checked.append(len(ts)))
+    y = autograd.linear(x, w)
+    checked.clear()
+    torch.autograd.grad(y, [x], torch.zeros_like(y))
+    assert checked and calls[-1] == "tbf16_train_linear_bwd"
