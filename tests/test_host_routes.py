@@ -108,3 +108,17 @@ def test_linear_refuses_host_tensors(linear_calls, monkeypatch):
     checked.clear()
     torch.autograd.grad(y, [x], torch.zeros_like(y))
     assert checked and calls[-1] == "tbf16_train_linear_bwd"
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.t().contiguous().t(), lambda t: torch.cat([t, t], 1)[:, :t.shape[1]]])
+def test_linear_backward_takes_saved_tensors_of_any_layout(linear_calls, unpack):
+    """Saved-tensor hooks may give x's transposed copy back with other strides: those go pass
+    by pass, where operands are made contiguous."""
+    from tbf16 import autograd
+    x = torch.zeros(16, 32, dtype=torch.bfloat16, requires_grad=True)
+    w = torch.zeros(24, 32, dtype=torch.bfloat16, requires_grad=True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: unpack(t) if t.dtype == torch.float16 else t):
+        y = autograd.linear(x, w)
+        grads = torch.autograd.grad(y, [x, w], torch.zeros_like(y))
+    assert [g.shape for g in grads] == [x.shape, w.shape]
+    assert "tbf16_train_linear_bwd" not in [name for name, _ in linear_calls]
