@@ -122,3 +122,14 @@ def test_linear_backward_takes_saved_tensors_of_any_layout(linear_calls, unpack)
         grads = torch.autograd.grad(y, [x, w], torch.zeros_like(y))
     assert [g.shape for g in grads] == [x.shape, w.shape]
     assert "tbf16_train_linear_bwd" not in [name for name, _ in linear_calls]
+
+
+@pytest.mark.parametrize("cast", [torch.bfloat16, torch.float32])
+def test_conv2d_cast_after_conversion_is_refused(conv_calls, cast):
+    """A model cast after its conversion has a weight that is no fp16 any more: torch's own
+    error, as its bits must not be read as fp16."""
+    m = _converted(128, 128, padding=1).to(cast)
+    m.bias = nn.Parameter(m.bias.detach().bfloat16())
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        m(torch.zeros(1, 128, 64, 64, dtype=torch.bfloat16))
+    assert conv_calls == []

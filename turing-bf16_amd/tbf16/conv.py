@@ -107,15 +107,16 @@ _NATIVE_MIN_MACS = 1 << 29
 def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
     """0 (contiguous) or 1 (channels last) when the native 2-D convolution takes this
     call, else None: one group, zero padding given in numbers, a bf16 bias, an input
-    dense in exactly one of the two layouts, as many channels as the weight has (the
-    library's convolution refuses any other input).
+    dense in exactly one of the two layouts, as many channels as the weight has, the weight
+    still fp16 (the library's convolution refuses any other).
     Small convolutions (_NATIVE_MIN_MACS) keep the library's fp16 convolution and its
     fp16 rounding: their results are pinned bit for bit to the reference's formula on
     that call. The native kernel is the faster one there too (64 -> 64 at 16 x 16: 22 us
     against 51)."""
     if (x.dim() != 4 or conv.weight16.dim() != 4 or x.shape[1] != conv.weight16.shape[1] or conv.groups != 1
             or isinstance(padding, str) or x.numel() == 0 or x.data_ptr() % 16
-            or not conv.weight16.is_contiguous() or (bias is not None and bias.dtype != torch.bfloat16)):
+            or conv.weight16.dtype != torch.float16 or not conv.weight16.is_contiguous()
+            or (bias is not None and bias.dtype != torch.bfloat16)):
         return None
     nchw, nhwc = x.is_contiguous(), x.is_contiguous(memory_format=torch.channels_last)
     if nchw == nhwc or (nhwc and x.shape[1] % 8):
