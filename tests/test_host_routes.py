@@ -133,3 +133,14 @@ def test_conv2d_cast_after_conversion_is_refused(conv_calls, cast):
     with torch.no_grad(), pytest.raises(RuntimeError):
         m(torch.zeros(1, 128, 64, 64, dtype=torch.bfloat16))
     assert conv_calls == []
+
+
+def test_conv2d_bias_in_host_memory_is_refused(conv_calls, monkeypatch):
+    """The native convolution checks every operand that it reads, the bias too."""
+    seen = []
+    monkeypatch.setattr(tconv, "_dev_check", lambda *ts: seen.extend(t.data_ptr() for t in ts if t is not None))
+    m = _converted(128, 128, padding=1)
+    x = torch.zeros(1, 128, 64, 64, dtype=torch.bfloat16)
+    with torch.no_grad():
+        m(x)
+    assert {t.data_ptr() for t in (x, m.weight16, m.weight_scale, m.bias)} <= set(seen)

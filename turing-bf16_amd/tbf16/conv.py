@@ -67,7 +67,7 @@ def scale_input(x: torch.Tensor, t: int):
 
 def unscale_output(y16: torch.Tensor, exps: torch.Tensor, w_sinv: torch.Tensor, bias=None) -> torch.Tensor:
     """fp16 (B, O, *spatial) -> bf16 y16 * 2^e[b] * w_sinv[o] + bias[o] (conv.py:56-60)."""
-    _dev_check(y16, exps, w_sinv)
+    _dev_check(y16, exps, w_sinv, bias)
     if y16.dtype != torch.float16 or exps.dtype != torch.int32 or exps.numel() != y16.shape[0]:
         raise TypeError("tbf16.conv.unscale_output: expected fp16 y16 and int32 exponents, one per sample")
     exps = exps.contiguous()
@@ -143,7 +143,7 @@ def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int)
     wsb = lib().tbf16_conv2d_ws_bytes(B, C, H, W, O, KH, KW, *geom)
     if wsb == 0:
         return None
-    _dev_check(x, w16, conv.weight_scale)
+    _dev_check(x, w16, conv.weight_scale, bias)
     Ho = (H + 2 * pad[0] - dilation[0] * (KH - 1) - 1) // stride[0] + 1
     Wo = (W + 2 * pad[1] - dilation[1] * (KW - 1) - 1) // stride[1] + 1
     y = torch.empty((B, O, Ho, Wo), device=x.device, dtype=torch.bfloat16,
