@@ -173,7 +173,8 @@ def test_gemm_pingpong_small_integers_bit_exact(dev, cfg, K):
         assert torch.equal(y.cpu(), want), (M, N)
 
 
-@pytest.mark.parametrize("M,N,K", [(2, 8, 1000), (64, 256, 8200), (130, 72, 4096), (260, 8, 30000), (2, 264, 130000)])
+@pytest.mark.parametrize("M,N,K", [(2, 8, 1000), (64, 256, 8200), (130, 72, 4096), (260, 8, 30000), (2, 264, 130000),
+                                   (72, 264, 98312)])
 def test_linear_dispatch_splits_bit_exact(dev, M, N, K):
     """The dispatcher's own choice where few tiles meet a long K (2, 4 or 8 splits, a K
     tail in the last one) and where x16 would not fit the no-allocation array (kernels

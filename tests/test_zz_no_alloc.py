@@ -64,3 +64,16 @@ def test_noalloc_rejects_rows_beyond_limit(dev):
     assert L.tbf16_linear_ws_bytes(255, K, 10240, 18) > (12 << 20)
     rc = L.tbf16_linear_noalloc(16, 255, K, K, 16, 10240, K, 16, None, 16, 10240, 15, 1, 18, None)
     assert rc == -1 and "scratch limit" in L.tbf16_last_error().decode()
+
+
+@pytest.mark.parametrize("M,K,N", [(4096, 4096, 4096), (4100, 4040, 4096), (6144, 2056, 2048), (2000, 4096, 4096),
+                                   (3000, 2304, 3072), (1500, 8192, 8192), (2048, 3200, 640), (130, 100008, 264),
+                                   (70, 130000, 4096)])
+def test_noalloc_same_bits_where_x16_does_not_fit(dev, M, K, N):
+    """x's fp16 copy beyond the scratch array: tiles that convert x inside the GEMM in place
+    of the ping-pong kernels (whole tiles and cut ones, a K tail), row chunks in place of
+    the alternate-k-tile kernels, and K so long that not 64 rows fit (k ascending, split in
+    two). Random data, so that another order of the sums would show in the bits."""
+    x, w16, ws, b = _inputs(dev, M, K, N, M)
+    assert 2 * M * K > 12 << 20
+    assert torch.equal(_no_alloc(x, w16, ws, b, 15, 0), _with_workspace(x, w16, ws, b, 15, 0))
