@@ -135,7 +135,7 @@ int tbf16_gemm_f16(const void* a16, int64_t M, int64_t K, int64_t lda, const flo
  * call each way; same values as the single entry points above.
  * Forward: x16 (M, K), xT (K, ldT), sx (M,) as tbf16_quantize_rows / _t of x at t, the
  * weight w bf16 (N, K) by rows at t, y = bf16(x w^T + bias); K and N multiples of 8.
- * x NULL: x16 and sx are given (an activation that several layers read).
+ * xT NULL (exps_ws too): no transposed copy, for the further layers that read one x.
  * Backward: dx = dY W from dY rows by L1 norm at t_rows and W columns at t_w; dw = dY^T X
  * from dY's columns (with sx folded in) at t_dy and xT; db = the columns' fp32 sums, bf16.
  * Each of dx (M, K), dw (N, K), db (N,) may be NULL. */

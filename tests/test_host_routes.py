@@ -144,3 +144,22 @@ def test_conv2d_bias_in_host_memory_is_refused(conv_calls, monkeypatch):
     with torch.no_grad():
         m(x)
     assert {t.data_ptr() for t in (x, m.weight16, m.weight_scale, m.bias)} <= set(seen)
+
+
+@pytest.mark.parametrize("N", [24, 12])
+def test_linear_keeps_one_copy_of_an_activation(linear_calls, N):
+    """What the memo keeps while x lives is the transposed fp16 copy and its scales, which the
+    backward saves anyway: a second copy for each of eight activations is memory that a
+    model may not have. A second layer on x makes no second transposed copy."""
+    from tbf16 import autograd, routing
+    M, K = 40, 64
+    x = torch.zeros(M, K, dtype=torch.bfloat16, requires_grad=True)
+    ws = [torch.zeros(N, K, dtype=torch.bfloat16, requires_grad=True) for _ in range(2)]
+    autograd.linear(x, ws[0])
+    (_, kept), = routing.activations._entries.values()
+    assert sum(t.numel() * t.element_size() for t in kept) <= 2 * K * M + 4 * M
+    first = len(linear_calls)
+    autograd.linear(x, ws[1])
+    (_, again), = routing.activations._entries.values()
+    assert all(a is b for a, b in zip(kept, again))
+    assert kept[0].data_ptr() not in [a for _, args in linear_calls[first:] for a in args]

@@ -619,30 +619,28 @@ extern "C" size_t tbf16_train_linear_fwd_ws_bytes(int64_t N, int64_t K) {
 extern "C" int tbf16_train_linear_fwd(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w, int64_t N,
                                       int64_t ldw, const void* bias, int t, void* x16, void* xT, int64_t ldT, float* sx,
                                       int32_t* exps_ws, void* y, int64_t ldy, void* ws, int64_t ws_bytes, void* stream) {
+  if (int rc = check_rows("train_linear_fwd: x", x, M, K, ldx)) return rc;
   if (int rc = check_rows("train_linear_fwd: w", w, N, K, ldw)) return rc;
   TB_CHECK(M > 0 && N > 0 && K > 0 && N % 8 == 0, "train_linear_fwd: empty, or N no multiple of 8");
   TB_CHECK(x16 && aligned16(x16) && sx, "train_linear_fwd: x16 or its scales missing");
+  TB_CHECK(xT == nullptr || (aligned16(xT) && ldT % 8 == 0 && ldT >= M && exps_ws), "train_linear_fwd: bad output");
   TB_CHECK(ws && aligned16(ws) && ws_bytes >= (int64_t)tbf16_train_linear_fwd_ws_bytes(N, K),
            "train_linear_fwd: workspace too small");
   hipStream_t st = as_stream(stream);
   TrainFwd p{};
+  p.x = (const uint16_t*)x;
+  p.x16 = (uint16_t*)x16;
+  p.sx = sx;
+  p.xexp = xT ? exps_ws : nullptr;
+  p.M = M; p.ldx = ldx;
+  p.xblocks = cdiv(M, kRowWaves);
   p.w = (const uint16_t*)w;
   p.w16 = static_cast<uint16_t*>(ws);
   p.sw = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + align_up((size_t)N * (size_t)K * 2, 256));
   p.N = N; p.ldw = ldw; p.K = (int)K; p.t = t;
-  if (x) {
-    if (int rc = check_rows("train_linear_fwd: x", x, M, K, ldx)) return rc;
-    TB_CHECK(xT && aligned16(xT) && ldT % 8 == 0 && ldT >= M && exps_ws, "train_linear_fwd: bad output");
-    p.x = (const uint16_t*)x;
-    p.x16 = (uint16_t*)x16;
-    p.sx = sx;
-    p.xexp = exps_ws;
-    p.M = M; p.ldx = ldx;
-    p.xblocks = cdiv(M, kRowWaves);
-  }
   train_rows_kernel<<<(unsigned)(p.xblocks + cdiv(N, kRowWaves)), 256, 0, st>>>(p);
   TB_LAUNCH_CHECK("train_linear_fwd/rows");
-  if (x) {
+  if (xT) {
     dim3 grid((unsigned)cdiv(K, 256), (unsigned)cdiv(ldT, 64));
     transpose_convert_kernel<<<grid, 256, 0, st>>>(p.x, M, K, ldx, exps_ws, nullptr, nullptr, (uint16_t*)xT, ldT);
     TB_LAUNCH_CHECK("train_linear_fwd/transpose");
