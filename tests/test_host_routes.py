@@ -163,3 +163,21 @@ def test_linear_keeps_one_copy_of_an_activation(linear_calls, N):
     (_, again), = routing.activations._entries.values()
     assert all(a is b for a, b in zip(kept, again))
     assert kept[0].data_ptr() not in [a for _, args in linear_calls[first:] for a in args]
+
+
+@pytest.mark.parametrize("B,C,O,side,k,native", [
+    (1, 8, 8, 1024, 3, False), (1, 16, 16, 512, 3, False),     # 8 and 4 times the input's memory
+    (1, 3, 64, 512, 5, False), (1, 4, 320, 512, 3, False),     # few channels, large images
+    (1, 96, 16, 1024, 3, False), (1, 96, 64, 1024, 3, True),   # 128 channels against 96 + O
+    (1, 16, 64, 256, 3, True), (2, 16, 64, 224, 7, True), (1, 512, 512, 128, 3, True), (1, 64, 64, 512, 3, True),
+])
+@pytest.mark.parametrize("cl", [False, True])
+def test_conv2d_route_by_the_padded_copy(B, C, O, side, k, native, cl):
+    """The native kernels pad the input's channels to a multiple of 64. They are used where
+    that copy is small, or no larger than the library path's own fp16 copies."""
+    if cl and C % 8:
+        pytest.skip("channels last takes channels in multiples of 8")
+    m = _converted(C, O, k, padding=k // 2)
+    x = torch.empty(B, C, side, side, dtype=torch.bfloat16, device="meta")
+    x = x.to(memory_format=torch.channels_last) if cl else x
+    assert tconv._native_layout(m, x, m.padding, m.bias) == (int(cl) if native else None)

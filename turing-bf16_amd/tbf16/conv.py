@@ -102,6 +102,12 @@ def _pair(v) -> ctypes.Array:
 
 # Multiply-adds below which the fp16 convolution stays the library's.
 _NATIVE_MIN_MACS = 1 << 29
+# Bytes of a padded input copy that are taken whatever the channels. Of 491 convolutions of
+# 3 to 96 channels (3x3, strided 3x3, 5x5, strided 7x7; 128 to 1024 pixels a side; both
+# layouts), native against library, 298 are taken, none more than 4% slower and the median
+# half the time (16 -> 64 at 256 x 256: 28 us against 55). At 32 MiB they begin to lose (16 -> 16
+# at 512 x 512: 70 us against 55; 8 -> 8 at 1024 x 1024: 222 against 98).
+_NATIVE_MAX_PADDED = 28 << 20
 
 
 def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
@@ -121,14 +127,18 @@ def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
     nchw, nhwc = x.is_contiguous(), x.is_contiguous(memory_format=torch.channels_last)
     if nchw == nhwc or (nhwc and x.shape[1] % 8):
         return None
-    # the kernels pad channels to 64: with three of them on a large image the padded copy
-    # costs more than MIOpen's passes (3 -> 128 at 512 x 512: 93 us against 89; every
-    # other shape measured is 1.07 to 3.8 times as fast, 3 -> 64 at 2 x 224 x 224 1.6)
-    if x.shape[1] < 4 and x.numel() > x.shape[1] << 17:
+    B, C, H, W = x.shape
+    O, _, KH, KW = conv.weight16.shape
+    ph, pw = (padding, padding) if isinstance(padding, int) else padding
+    pixels = B * H * W // (conv.stride[0] * conv.stride[1])  # the output's, up to its edges
+    if pixels * C * O * KH * KW < _NATIVE_MIN_MACS:
         return None
-    # (input pixels over strides: the output's, up to its edges)
-    macs = x.numel() // (conv.stride[0] * conv.stride[1]) * (conv.weight16.numel() // x.shape[1])
-    return int(nhwc) if macs >= _NATIVE_MIN_MACS else None
+    # The kernels' copy of the input has its channels padded to a multiple of 64: it is the
+    # memory of the call, and with few channels its time too. It is taken where it is small
+    # or no larger than the two fp16 tensors around the library's convolution.
+    padded = B * (H + 2 * ph) * (W + 2 * pw) * (C + -C % 64)
+    small = 2 * padded <= _NATIVE_MAX_PADDED
+    return int(nhwc) if small or (C >= 16 and padded <= B * C * H * W + pixels * O) else None
 
 
 def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int):
