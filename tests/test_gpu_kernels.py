@@ -438,6 +438,34 @@ def test_attention_bias_forms(dev, monkeypatch, Sq, Sk, D, causal, split):
         assert rel(got.cpu(), torch.softmax(s, -1) @ v.double()) < TOL
 
 
+@pytest.mark.parametrize("split", ["0", "1"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [64, 128, 192])
+def test_attention_running_maximum(dev, monkeypatch, D, causal, split):
+    """The running maximum of a row: key tiles in which it sees no key before the first one
+    that it sees (rows 0-15 and 16-31 of a wave's block at different tiles), rows that see
+    none, and maxima that grow tile by tile by more and by less than the lazy bound, in
+    only one of the two blocks or in both."""
+    monkeypatch.setenv("TBF16_ATTN_SPLIT", split)
+    g = torch.Generator().manual_seed(D)
+    S = 330
+    q, k, v = (torch.randn(1, 2, S, D, generator=g).bfloat16() for _ in range(3))
+    row, key = torch.arange(S).view(S, 1), torch.arange(S).view(1, S)
+    first = torch.where(row % 32 < 16, 70, 135) * (row // 32 % 2)  # every other wave block: keys from 70 / 135 on
+    mask = (key >= first).expand(1, 1, S, S).clone()
+    mask[..., 37, :] = False
+    mask[..., 300:, :] = False
+    grow = torch.where(row % 32 < 16, 4.0, 24.0) * (key // 64)     # in logits; the bound is 8 ln 2
+    for m in (mask, mask & (key < 200), grow.half().expand(1, 1, S, S)):
+        got = tbf16.sdpa(q.to(dev), k.to(dev), v.to(dev), attn_mask=m.to(dev), is_causal=causal)
+        s = q.double() @ k.double().transpose(-1, -2) * D ** -0.5
+        s = s + m.double() if m.dtype == torch.float16 else s.masked_fill(~m, -math.inf)
+        if causal:
+            s = s.masked_fill(key > row, -math.inf)
+        want = torch.nan_to_num(torch.softmax(s, -1)) @ v.double()  # rows that see no key: zeros
+        assert torch.isfinite(got).all() and rel(got.cpu(), want) < TOL
+
+
 @pytest.mark.parametrize("kform", ["bf16", "fp16"])
 @pytest.mark.parametrize("causal", [True, False])
 def test_sdpa_gqa_key_forms(dev, monkeypatch, causal, kform):

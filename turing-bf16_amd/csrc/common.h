@@ -222,22 +222,33 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 
 // Values of lanes l and l ^ 32 combined, through v_permlane32_swap (gfx950: a
 // VALU exchange of the wave's two 32-lane halves, no LDS round trip). Both
-// results of the swap hold one of the two lanes' values, so a symmetric op
-// (max, sum) needs no knowledge of which is which.
-__device__ __forceinline__ float max_xor32(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
+// results of the swap hold one of the two lanes' values, so a sum needs no
+// knowledge of which is which.
 __device__ __forceinline__ float sum_xor32(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// The same for lanes l and l ^ 16 (v_permlane16_swap).
-__device__ __forceinline__ float max_xor16(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+// max(a, b) as one instruction (fmaxf adds one per operand that may be a signalling NaN,
+// such as a value that came from a lane exchange).
+__device__ __forceinline__ float max_raw(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, INFINITY); }
+
+// The maxima of a and of b over the four lanes l % 16 + 16 i, packed: 16-lane rows 0 and 2
+// hold a's, rows 1 and 3 b's (v_permlane16_swap pairs the odd rows of its first operand with
+// the even rows of the second). unpack_pair16 gives such a pair to all lanes.
+__device__ __forceinline__ float max_pair16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const uint32_t m = __float_as_uint(max_raw(__uint_as_float(r[0]), __uint_as_float(r[1])));
+  const auto s = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+  return max_raw(__uint_as_float(s[0]), __uint_as_float(s[1]));
 }
+__device__ __forceinline__ void unpack_pair16(float v, float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+
+// As sum_xor32 for lanes l and l ^ 16 (v_permlane16_swap).
 __device__ __forceinline__ float sum_xor16(float v) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
