@@ -406,7 +406,8 @@ def test_attention_causal_block_forms(dev, monkeypatch, B, H, S, D, layout, spli
     _attn_checks(q, k, v, dev, label=f"split={split} k={kform} {layout} B={B} H={H} S={S} D={D}")
 
 
-@pytest.mark.parametrize("H,S,D", [(1, 129, 128), (150, 200, 64), (170, 200, 64), (170, 300, 128), (280, 200, 64), (390, 200, 64)])
+@pytest.mark.parametrize("H,S,D", [(1, 129, 128), (150, 200, 64), (170, 200, 64), (170, 300, 128), (280, 200, 64), (390, 200, 64),
+                                   (3, 130, 192), (5, 577, 256)])
 def test_attention_causal_grids(dev, H, S, D):
     """The causal grids on both sides of each line: single split-key tiles, pairs in one
     round, single tiles where the pairs are just more than a round, 256-row blocks."""

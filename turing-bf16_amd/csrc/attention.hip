@@ -115,10 +115,12 @@ __device__ __forceinline__ floatx4 mfma_qk(half8 k, half8 q, floatx4 c) {
 // vectors of up to 32 registers. As separate 4-register values the compiler gives each
 // MFMA a new destination and copies all of them around the rarely taken rescale (32
 // moves per tile, a sixth of the softmax's instructions); parts of one wide value stay
-// where they are.
+// where they are. Past 128 d the accumulators do not fit the VGPRs beside the rest, and
+// wide values are moved to the accumulation registers and back whole (270 moves a tile
+// against 150 as 4-register values: 2 x 8 x 2048 x 256 135 -> 129 us, with dropout 152 -> 138).
 template <int NB>
 struct AccCol {
-  static constexpr int W = NB * 4 < 32 ? NB * 4 : 32, NV = NB * 4 / W;
+  static constexpr int W = NB > 8 ? 4 : NB * 4 < 32 ? NB * 4 : 32, NV = NB * 4 / W;
   typedef float vec __attribute__((ext_vector_type(W)));
   vec v[NV];
   __device__ __forceinline__ float at(int db, int r) const { return v[db * 4 / W][db * 4 % W + r]; }
@@ -339,8 +341,10 @@ attn_fwd_kernel(FwdParams p) {
   constexpr int KBYTES = BKV * DP * 2;
   constexpr int STAGE = KBYTES + DP * 128;
   // fragment reads run ahead under an instruction-group schedule (registers allow it
-  // up to DP = 128 without the dropout hashing)
-  constexpr bool VPRE = DP <= 128 && !DROP;
+  // up to DP = 128 without the dropout hashing; past that it spills 23 registers and is
+  // still the faster form of a causal block, 8 x 4096 x 256 251 -> 218 us, not of the
+  // others, 209 -> 220)
+  constexpr bool VPRE = !DROP && (DP <= 128 || (CAUSAL && !HAS_BIAS));
   // K and V^T tiles go global -> LDS directly, 1 KB per wave instruction: BPW
   // such blocks per wave per tile, the first KPW of them K, the rest V^T
   constexpr int KBLK = KBYTES / 1024, NBLK = STAGE / 1024;
@@ -462,8 +466,11 @@ attn_fwd_kernel(FwdParams p) {
     // after its first K reads have gone out (its fragments were read before the
     // barrier), so the barrier's drain and those reads' latency hide behind its MFMAs.
     // It starts as zeros (adds nothing) and is flushed after the last tile.
-    constexpr int DQ = DB / 2;  // d blocks of the deferred quarter: DB - DQ .. of the second 32 keys
-    half8 dpf[2], dvf[DQ];
+    // (Without the reads ahead the held fragments cost more registers than the overlap
+    // gains, 8 x 4096 x 256 209 -> 203 us, but for the masked copies of causal blocks past
+    // 128 d, with dropout 256 -> 279.)
+    constexpr int DQ = VPRE || (CAUSAL && DP > 128) ? DB / 2 : 0;  // d blocks DB - DQ .. of the second 32 keys
+    half8 dpf[2], dvf[DQ > 0 ? DQ : 1];
     for (int e = 0; e < 8; ++e) dpf[0][e] = (_Float16)0.f;
     dpf[1] = dpf[0];
   #pragma unroll
