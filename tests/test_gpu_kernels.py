@@ -193,7 +193,7 @@ def test_linear_dispatch_splits_bit_exact(dev, M, N, K):
 
 
 @pytest.mark.parametrize("M,K,N", [(17, 6528, 832), (32, 4104, 264), (33, 6528, 832), (2048, 3200, 640), (1999, 3400, 520),
-                                   (640, 16384, 512)])
+                                   (640, 16384, 512), (16, 1000, 9000), (31, 1544, 8192), (32, 512, 8)])
 def test_linear_dispatch_few_rows_and_row_chunks(dev, M, K, N):
     """At most 32 rows whose tiles would split K (converted in the skinny kernel) and 33;
     x16 beyond the no-allocation array, which that entry point then takes in chunks of

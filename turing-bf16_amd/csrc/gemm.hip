@@ -1962,20 +1962,25 @@ int64_t scratch_rows(int64_t K, int64_t N, int splits) {
 }
 // The dispatcher's choice (cfg < 0): x quantised once and a kernel on fp16 operands,
 // also for wide tiles (4096^3: 101 us + 9 us of row pass against 118 + 5 with the
-// conversion in the GEMM). For at most 32 rows a kernel that would split K is not worth
-// its third launch: the skinny kernel converting x itself takes two (6x3712x2640: 17.2 us
-// a call against 18.9); ragged: N is not the caller's, which that kernel cannot take.
+// conversion in the GEMM).
+// At most 32 rows against fewer than 32 weight rows per CU, or at K <= 1024: the skinny
+// kernel, which converts x itself and splits K inside its blocks (device time, skinny
+// against the fp16 tiles: 16x512x2048 6.6 and 8.4 us, 8x2048x4096 12.0 and 13.0, 16x8192x4096
+// 25.4 and 30.9; a split over blocks takes a third launch). Above that the tiles, unsplit: 16
+// x 2048 x 8192 13.9 us against the skinny kernel's 14.9, 32 x 2560 x 10240 16.5 against 18.
+// ragged: N is not the caller's, which the skinny kernel cannot take.
 // Where that workspace would not fit the no-allocation entry point's array, a kernel
 // whose output that entry point reproduces bit for bit: the converting tiles do k
 // ascending, row chunks of the same configuration anything that takes 64 rows.
 LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg, bool ragged = false) {
   if (cfg >= 0) return layout_ws(M, K, N, cfg, pick_split(cfg, M, N, K), quantize_once(cfg, K));
+  const bool few = M <= 32 && !ragged;
+  if (few && (N < 32 * num_cus() || K <= 1024)) return layout_ws(M, K, N, pick_fused(M, N, false), 1, false);
   const size_t base = layout_ws(M, K, N, 20, 1, true).bytes;
   const bool over = base > TBF16_NOALLOC_SCRATCH_BYTES, bounded = over && scratch_rows(K, N, 1) == 0;
-  const F16Pick p = pick_f16(M, N, K, !over || bounded || scratch_rows(K, N, 8) > 0,
+  const F16Pick p = pick_f16(M, N, K, !few && (!over || bounded || scratch_rows(K, N, 8) > 0),
                              over ? kSplitPartBytes : std::min<size_t>(kSplitPartBytes, TBF16_NOALLOC_SCRATCH_BYTES - base),
                              bounded);
-  if (M <= 32 && p.splits > 1 && !ragged) return layout_ws(M, K, N, pick_fused(M, N, false), 1, false);
   return layout_ws(M, K, N, p.cfg, p.splits, true);
 }
 // The form that converts x inside the GEMM, the same output bits: the pinned
