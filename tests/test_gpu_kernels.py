@@ -193,10 +193,12 @@ def test_linear_dispatch_splits_bit_exact(dev, M, N, K):
 
 
 @pytest.mark.parametrize("M,K,N", [(17, 6528, 832), (32, 4104, 264), (33, 6528, 832), (2048, 3200, 640), (1999, 3400, 520),
-                                   (640, 16384, 512), (16, 1000, 9000), (31, 1544, 8192), (32, 512, 8)])
+                                   (640, 16384, 512), (16, 1000, 9000), (31, 1544, 8192), (32, 512, 8),
+                                   (33, 256, 72), (64, 328, 264), (64, 256, 10248), (300, 320, 1032), (4100, 768, 136),
+                                   (16390, 1032, 40)])
 def test_linear_dispatch_few_rows_and_row_chunks(dev, M, K, N):
-    """At most 32 rows whose tiles would split K (converted in the skinny kernel) and 33;
-    x16 beyond the no-allocation array, which that entry point then takes in chunks of
+    """At most 32 rows whose tiles would split K (converted in the skinny kernel) and 33; a
+    short K, or few columns for many rows (converted in the tiles); x16 beyond the no-allocation array, which that entry point then takes in chunks of
     rows (the last one short): exact products, and the same bits from both entry points."""
     g = torch.Generator().manual_seed(M)
     a, b = torch.randint(-1, 2, (M, K), generator=g), torch.randint(-1, 2, (N, K), generator=g)

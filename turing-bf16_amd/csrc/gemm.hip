@@ -1968,14 +1968,30 @@ int64_t scratch_rows(int64_t K, int64_t N, int splits) {
 // against the fp16 tiles: 16x512x2048 6.6 and 8.4 us, 8x2048x4096 12.0 and 13.0, 16x8192x4096
 // 25.4 and 30.9; a split over blocks takes a third launch). Above that the tiles, unsplit: 16
 // x 2048 x 8192 13.9 us against the skinny kernel's 14.9, 32 x 2560 x 10240 16.5 against 18.
-// ragged: N is not the caller's, which the skinny kernel cannot take.
+// More rows with a short K, or with few products for each value of x: the tile that
+// converts x itself (converts_x).
+// ragged: N is not the caller's, which those two cannot take.
 // Where that workspace would not fit the no-allocation entry point's array, a kernel
 // whose output that entry point reproduces bit for bit: the converting tiles do k
 // ascending, row chunks of the same configuration anything that takes 64 rows.
+// Whether a call of more than 32 rows converts x inside the GEMM. Up to 64 rows: with a short
+// K, in the skinny kernel (48x352x1872 7.7 us against 8.6). Else where what the separate
+// pass takes longer (2 us, and 0.54 us per million values of x for writing and reading x16)
+// exceeds what the conversion costs the tiles (0.33 us a k tile and round of 256 x 256
+// tiles; 0.45 with the selects of a K tail). Measured as x16 / converted, us: 16384x128 ->
+// 256 22.3 / 11.9, 8192x320 -> 1024 22.9 / 17.6, 4096x768 -> 256 14.0 / 12.9, 16384x1024 -> 256
+// 34.7 / 25.7, but 1024x512 -> 1024 9.8 / 10.0, 8192x4096 -> 512 59 / 66. On 460 shapes the
+// rule's choice is 0.8% off the better one on average and 15% at most.
+bool converts_x(int64_t M, int64_t K, int64_t N) {
+  if (M <= 64 && N < 32 * num_cus() && K <= (K % 64 ? 1024 : 512)) return true;
+  const int64_t rounds = cdiv(M * N, num_cus() * 65536);
+  return 2.0 + 0.54e-6 * (double)M * (double)K > (double)(rounds * K) / 64 * (K % 64 ? 0.45 : 0.33);
+}
 LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg, bool ragged = false) {
   if (cfg >= 0) return layout_ws(M, K, N, cfg, pick_split(cfg, M, N, K), quantize_once(cfg, K));
   const bool few = M <= 32 && !ragged;
-  if (few && (N < 32 * num_cus() || K <= 1024)) return layout_ws(M, K, N, pick_fused(M, N, false), 1, false);
+  if (few ? N < 32 * num_cus() || K <= 1024 : !ragged && converts_x(M, K, N))
+    return layout_ws(M, K, N, pick_fused(M, N, false), 1, false);
   const size_t base = layout_ws(M, K, N, 20, 1, true).bytes;
   const bool over = base > TBF16_NOALLOC_SCRATCH_BYTES, bounded = over && scratch_rows(K, N, 1) == 0;
   const F16Pick p = pick_f16(M, N, K, !few && (!over || bounded || scratch_rows(K, N, 8) > 0),
