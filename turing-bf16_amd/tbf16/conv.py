@@ -119,18 +119,19 @@ def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
     fp16 rounding: their results are pinned bit for bit to the reference's formula on
     that call. The native kernel is the faster one there too (64 -> 64 at 16 x 16: 22 us
     against 51)."""
-    if (x.dim() != 4 or conv.weight16.dim() != 4 or x.shape[1] != conv.weight16.shape[1] or conv.groups != 1
-            or isinstance(padding, str) or x.numel() == 0 or x.data_ptr() % 16
-            or conv.weight16.dtype != torch.float16 or not conv.weight16.is_contiguous()
+    w16 = conv.weight16  # (a module's buffers are slow to look up)
+    if (x.dim() != 4 or w16.dim() != 4 or conv.groups != 1 or isinstance(padding, str) or x.data_ptr() % 16
+            or w16.dtype != torch.float16 or not w16.is_contiguous()
             or (bias is not None and bias.dtype != torch.bfloat16)):
         return None
-    nchw, nhwc = x.is_contiguous(), x.is_contiguous(memory_format=torch.channels_last)
-    if nchw == nhwc or (nhwc and x.shape[1] % 8):
-        return None
     B, C, H, W = x.shape
-    O, _, KH, KW = conv.weight16.shape
+    O, Cw, KH, KW = w16.shape
+    nchw, nhwc = x.is_contiguous(), x.is_contiguous(memory_format=torch.channels_last)
+    if C != Cw or nchw == nhwc or (nhwc and C % 8):
+        return None
     ph, pw = (padding, padding) if isinstance(padding, int) else padding
-    pixels = B * H * W // (conv.stride[0] * conv.stride[1])  # the output's, up to its edges
+    sh, sw = conv.stride
+    pixels = B * H * W // (sh * sw)  # the output's, up to its edges
     if pixels * C * O * KH * KW < _NATIVE_MIN_MACS:
         return None
     # The kernels' copy of the input has its channels padded to a multiple of 64: it is the
@@ -145,7 +146,7 @@ def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int)
     """The whole scaled convolution on the library's own kernels, or None for sizes they
     do not take."""
     B, C, H, W = x.shape
-    w16 = conv.weight16
+    w16, scale = conv.weight16, conv.weight_scale
     O, Cw, KH, KW = w16.shape
     pad = (padding, padding) if isinstance(padding, int) else padding
     stride, dilation = conv.stride, conv.dilation
@@ -153,14 +154,14 @@ def _conv2d_native(conv: nn.Module, x: torch.Tensor, padding, bias, layout: int)
     wsb = lib().tbf16_conv2d_ws_bytes(B, C, H, W, O, KH, KW, *geom)
     if wsb == 0:
         return None
-    _dev_check(x, w16, conv.weight_scale, bias)
+    _dev_check(x, w16, scale, bias)
     Ho = (H + 2 * pad[0] - dilation[0] * (KH - 1) - 1) // stride[0] + 1
     Wo = (W + 2 * pad[1] - dilation[1] * (KW - 1) - 1) // stride[1] + 1
     y = torch.empty((B, O, Ho, Wo), device=x.device, dtype=torch.bfloat16,
                     memory_format=torch.channels_last if layout else torch.contiguous_format)
     ws = torch.empty(wsb, device=x.device, dtype=torch.uint8)
     b = None if bias is None else bias.detach().contiguous()
-    s = conv.weight_scale.float().contiguous()
+    s = scale.float().contiguous()
     launch("tbf16_conv2d", x, ptr(x), B, C, H, W, layout, int(conv._tbf16_plan.target_exp), ptr(w16), O, Cw, KH, KW,
            *geom, ptr(s), ptr(b), ptr(y), ptr(ws), wsb)
     return y
