@@ -218,6 +218,19 @@ def test_linear_dispatch_few_rows_and_row_chunks(dev, M, K, N):
 
 
 @pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("N", [50, 64])
+def test_linear_q_many_rows(dev, N):
+    """More rows than 65535 of the tiles that a few columns would get otherwise (128 x 64): a
+    taller tile takes them. Exact products."""
+    M, K = 65536 * 128 + 5, 8
+    g = torch.Generator(device=dev).manual_seed(N)
+    a, b = (torch.randint(-4, 5, (r, K), generator=g, device=dev).half() for r in (M, N))
+    y = ops.linear_q(a, torch.ones(M, device=dev), b, torch.ones(N, device=dev))
+    assert y.shape == (M, N)
+    for m in range(0, M, 1 << 21):
+        assert torch.equal(y[m:m + (1 << 21)], (a[m:m + (1 << 21)].float() @ b.float().t()).bfloat16()), m
+
+
 @pytest.mark.parametrize("M,N,K", [(2, 1, 64), (17, 9, 4096), (100, 515, 200), (300, 2049, 520), (64, 32001, 64), (2, 257, 16392)])
 def test_linear_any_n(dev, M, N, K, bias):
     """N that is no multiple of 8 without padding the weight, scale and bias views that

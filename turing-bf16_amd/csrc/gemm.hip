@@ -1639,6 +1639,7 @@ constexpr TileCfg kCfgs[] = {{256, 256, 32}, {128, 128, 64}, {64, 64, 64},      
                              {128, 128, 64, false, false, true, true}, {128, 64, 64, false, false, true, true},
                              {64, 128, 64, false, false, true, true}, {64, 64, 64, false, false, true, true}};
 constexpr int kNumCfgs = 31;
+constexpr int64_t kMaxRowTiles = 65536;  // fewer tiles than this along M
 
 // Compute units of the current device (cached per device).
 int64_t num_cus() {
@@ -1732,6 +1733,7 @@ F16Pick search_f16(int64_t M, int64_t N, int64_t K, int64_t cus, bool can_split,
   for (const F16Cand& c : kF16Cands) {
     const TileCfg& t = kCfgs[c.cfg];
     if (k_ascending && t.ksplit) continue;
+    if (cdiv(M, t.bm) >= kMaxRowTiles && t.bm < 256) continue;  // the launch refuses it; taller tiles take more rows
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
     for (int s = 1; s <= (!can_split ? 1 : k_ascending ? 2 : 8); s *= 2) {
       const int64_t kt = cdiv(KT, s);
@@ -1810,7 +1812,7 @@ int launch_gemm(int cfg, const void* A, int64_t lda, const int32_t* a_exp, const
   if (kCfgs[cfg].ksplit && M <= bm && splits == 1 && cdiv(N, bn) < num_cus())
     rows = (int)std::min<int64_t>(bn, std::max<int64_t>(8, cdiv(cdiv(N, num_cus()), 8) * 8));
   const int64_t blocks = cdiv(N, rows) * (kCfgs[cfg].skinny || kCfgs[cfg].stream ? 1 : cdiv(M, bm));
-  TB_CHECK(blocks < (int64_t)1 << 31 && cdiv(M, bm) < 65536, "gemm: grid too large");
+  TB_CHECK(blocks < (int64_t)1 << 31 && cdiv(M, bm) < kMaxRowTiles, "gemm: grid too large");
   const bool even = K % kCfgs[cfg].bk == 0;  // no k-tail selects on loaded values
   const auto a = (const uint16_t*)A;
   const auto b = (const uint16_t*)B;
