@@ -80,6 +80,19 @@ def test_linear_input_gradient_of_any_n(linear_calls, N):
     assert name == "tbf16_gemm_f16" and args[1:4] == (10, N + -N % 8, N + -N % 8)
 
 
+@pytest.mark.parametrize("N", [12, 1025])
+def test_linear_of_any_n_takes_a_misaligned_weight(linear_calls, N):
+    """A weight that does not start on 16 bytes (a view into a packed buffer) is copied for the
+    kernels, whose entry points refuse it."""
+    from tbf16 import ops
+    w16 = torch.zeros(N * 16 + 1, dtype=torch.float16)[1:].view(N, 16)
+    assert w16.data_ptr() % 16
+    x16 = torch.zeros(40, 16, dtype=torch.float16)
+    y = ops.linear_q(x16, torch.ones(40), w16, torch.ones(N))
+    (name, args), = linear_calls
+    assert y.shape == (40, N) and name == "tbf16_gemm_f16_any_n" and args[5] not in (0, None) and args[5] % 16 == 0
+
+
 @pytest.mark.parametrize("K,N", [(16, 12), (30, 40), (13, 1025)])
 def test_linear_gradients_have_their_leaves_shapes(linear_calls, K, N):
     from tbf16 import autograd

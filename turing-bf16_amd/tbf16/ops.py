@@ -132,6 +132,8 @@ def _prep_gemm_operands(x2, w16, w_sinv, bias):
         ws = F.pad(ws, (0, Np - N), value=1.0)
         if b is not None:
             b = F.pad(b, (0, Np - N))
+    elif Np != N and w16.data_ptr() % 16:  # (the padded copy used to put such weights in order)
+        w16 = w16.clone()
     return x2, w16, ws, b, N, Np
 
 
