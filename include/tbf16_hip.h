@@ -75,9 +75,10 @@ int tbf16_quantize_cols_t(const void* x, int64_t R, int64_t K, int64_t ldx, int 
  * x bf16 (M, K); w16 fp16 (N, K); ws fp32 (N,); bias bf16 (N,) or NULL; y bf16
  * (M, N). cfg < 0 picks the tile shape. workspace: tbf16_linear_ws_bytes(M, K, N,
  * cfg) bytes, 16-byte aligned; its first M int32 receive the row exponents p.
- * x is quantised once, as the reference's small-M path does: the row inverse scales
- * and x's scaled fp16 copy go into the workspace too, and the GEMM runs on fp16
- * operands (some pinned configurations convert x inside the GEMM instead). Where the
+ * As a rule x is quantised once, as the reference's small-M path does: the row inverse
+ * scales and x's scaled fp16 copy go into the workspace too, and the GEMM runs on fp16
+ * operands. Few rows, a short K or few columns for many rows (and some pinned
+ * configurations) convert x inside the GEMM instead. Where the
  * tiles would leave CUs idle and K is long (at most 8 MiB of partial sums), K is split
  * in up to eight: fp32 partial sums go into the workspace and a second kernel adds
  * them in a fixed order and applies the epilogue. Replaces linear (tbf16/csrc/gemm_sm75.cu:257-284) and, at
@@ -191,8 +192,8 @@ int tbf16_conv_epilogue(const void* y16, int64_t B, int64_t O, int64_t P, int ch
 /* The whole scaled 2-D convolution (tbf16/conv.py:39-60; one group, zero padding): x bf16
  * (B, C, H, W), contiguous or (channels_last, C % 8 == 0) channels last, each sample scaled
  * as tbf16_conv_input does at t; w16 fp16 (O, Cw, KH, KW) contiguous, Cw = C (anything else is
- * rejected), with its inverse scales per channel; bias bf16 (O,) or NULL; y bf16 in x's layout, rounded once from fp32. stride,
- * pad and dilation: two each. Replaces the reference's cuDNN call and the passes
+ * rejected), with its inverse scales per channel; bias bf16 (O,) or NULL; y bf16 in x's
+ * layout, rounded once from fp32. stride, pad and dilation: two each. Replaces the reference's cuDNN call and the passes
  * around it. A size query returns 0 for sizes the kernels do not take. */
 size_t tbf16_conv2d_ws_bytes(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW,
                              const int64_t* stride, const int64_t* pad, const int64_t* dilation);

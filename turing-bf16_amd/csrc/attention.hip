@@ -60,7 +60,7 @@ struct FwdParams {
   const uint16_t *q, *k, *v;
   uint16_t *k16, *vt16;  // workspace copies: (B, Hkv, Skp, DP) and (B, Hkv, Skp / BKV, DP, BKV)
   int32_t* ex;           // workspace exponents {a, 0, ev[b * Hkv + hk]...}
-  int Skp, DPc;
+  int Skp;
   int64_t q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss;
   const uint16_t* bias;
   int64_t bias_sb, bias_sh, bias_sq;
@@ -722,7 +722,7 @@ attn_fwd_kernel(FwdParams p) {
     deferred();
 
     if constexpr (SPLIT) {
-      // Group 1's partial O^T (lane-major, DB x 16 values per lane), running max
+      // Group 1's partial O^T (lane-major, DB x 8 values per lane), running max
       // and row sums go through the idle stages; group 0 merges them into its own:
       // m = max(m0, m1), O = O0 2^(m0 - m) + O1 2^(m1 - m), l likewise.
       float* xo = reinterpret_cast<float*>(rw < 2 ? smem0 : smem1) + (rw & 1) * (DB * 8 * 64);
@@ -1010,7 +1010,6 @@ extern "C" int tbf16_attn_fwd(const void* q, const void* k, const void* v, int64
   p.k16 = reinterpret_cast<uint16_t*>(wsb + w.off_k16);
   p.vt16 = reinterpret_cast<uint16_t*>(wsb + w.off_vt16);
   p.Skp = (int)w.Skp;
-  p.DPc = (int)w.DP;
   {
     const dim3 g((unsigned)(w.Skp / BKV), (unsigned)(B * Hkv));
     if (w.DP == 64) kv_prep_kernel<64><<<g, 256, 0, st>>>(p);

@@ -10,7 +10,8 @@
 // Memory layout: a sample is n = C * prod(spatial) elements stored back to back
 // (contiguous NC... or channels-last, both keep the batch outermost), so the
 // input passes run over B * n elements in memory order and find the sample as
-// index / n. All three kernels are HBM-bound streams of 16-byte vectors.
+// index / n. The passes of this file are HBM-bound streams of 16-byte vectors; the
+// implicit GEMM that they feed is bound by its products.
 #include <algorithm>
 
 #include "abi_util.h"

@@ -11,9 +11,10 @@
 //  - pingpong_kernel, fp16 a: large tiles, two wave groups alternating MFMAs and loads.
 //  - ksplit_kernel, fp16 a: small tiles (decode to mid-size M), the groups on alternate k
 //    tiles; also the implicit convolutions.
-//  - gemm_kernel: the form that converts bf16 a in its staging (tbf16_linear_exps, and
-//    the no-allocation entry point where x16 does not fit its array).
-//  - skinny_kernel: the same at M <= 32, K split across waves.
+//  - gemm_kernel: the form that converts bf16 a in its staging (a short K, or few columns
+//    for many rows; tbf16_linear_exps; the no-allocation entry point where x16 does not
+//    fit its array).
+//  - skinny_kernel: the same at M <= 64, K split across waves.
 //  - stream_kernel: decode on fp16 a with plain waves, by configuration number only:
 //    ksplit_kernel's 64-row tiles replaced it in the dispatch (16 x 2560 -> 10240: 17.3
 //    -> 15.5 us a call).
@@ -1668,8 +1669,7 @@ int pick_split(int cfg, int64_t M, int64_t N, int64_t K) {
   return 2;
 }
 
-// Tile configuration that converts bf16 a inside the GEMM (tbf16_linear_exps, and the
-// no-allocation entry point where x16 does not fit its array). For M <= 64 with enough
+// Configuration that converts bf16 a inside the GEMM. For M <= 64 with enough
 // b rows for 160 blocks, the 64-row skinny block up to M = 32 and the LDS-staged 64x64
 // tile above (every skinny block re-reads all of a). Otherwise the tile that maximises
 // eff x (blocks / whole rounds of CU-count blocks) x (M / M rounded up to the tile):
@@ -1962,6 +1962,19 @@ int64_t scratch_rows(int64_t K, int64_t N, int splits) {
   const int64_t per_row = 2 * K + 12 + (splits > 1 ? (int64_t)splits * N * 4 : 0);
   return (TBF16_NOALLOC_SCRATCH_BYTES - 1024) / per_row / 64 * 64;
 }
+// Whether a call of more than 32 rows converts x inside the GEMM. Up to 64 rows: with a short
+// K, in the skinny kernel (48x352x1872 7.7 us against 8.6). Else where what the separate
+// pass takes longer (2 us, and 0.54 us per million values of x for writing and reading x16)
+// exceeds what the conversion costs the tiles (0.33 us a k tile and round of 256 x 256
+// tiles; 0.45 with the selects of a K tail). Measured as x16 / converted, us: 16384x128 ->
+// 256 22.3 / 11.9, 8192x320 -> 1024 22.9 / 17.6, 4096x768 -> 256 14.0 / 12.9, 16384x1024 -> 256
+// 34.7 / 25.7, but 1024x512 -> 1024 9.8 / 10.0, 8192x4096 -> 512 59 / 66. On 460 shapes the
+// rule's choice is 0.8% off the better one on average and 15% at most.
+bool converts_x(int64_t M, int64_t K, int64_t N) {
+  if (M <= 64 && N < 32 * num_cus() && K <= (K % 64 ? 1024 : 512)) return true;
+  const int64_t rounds = cdiv(M * N, num_cus() * 65536);
+  return 2.0 + 0.54e-6 * (double)M * (double)K > (double)(rounds * K) / 64 * (K % 64 ? 0.45 : 0.33);
+}
 // The dispatcher's choice (cfg < 0): x quantised once and a kernel on fp16 operands,
 // also for wide tiles (4096^3: 101 us + 9 us of row pass against 118 + 5 with the
 // conversion in the GEMM).
@@ -1976,19 +1989,6 @@ int64_t scratch_rows(int64_t K, int64_t N, int splits) {
 // Where that workspace would not fit the no-allocation entry point's array, a kernel
 // whose output that entry point reproduces bit for bit: the converting tiles do k
 // ascending, row chunks of the same configuration anything that takes 64 rows.
-// Whether a call of more than 32 rows converts x inside the GEMM. Up to 64 rows: with a short
-// K, in the skinny kernel (48x352x1872 7.7 us against 8.6). Else where what the separate
-// pass takes longer (2 us, and 0.54 us per million values of x for writing and reading x16)
-// exceeds what the conversion costs the tiles (0.33 us a k tile and round of 256 x 256
-// tiles; 0.45 with the selects of a K tail). Measured as x16 / converted, us: 16384x128 ->
-// 256 22.3 / 11.9, 8192x320 -> 1024 22.9 / 17.6, 4096x768 -> 256 14.0 / 12.9, 16384x1024 -> 256
-// 34.7 / 25.7, but 1024x512 -> 1024 9.8 / 10.0, 8192x4096 -> 512 59 / 66. On 460 shapes the
-// rule's choice is 0.8% off the better one on average and 15% at most.
-bool converts_x(int64_t M, int64_t K, int64_t N) {
-  if (M <= 64 && N < 32 * num_cus() && K <= (K % 64 ? 1024 : 512)) return true;
-  const int64_t rounds = cdiv(M * N, num_cus() * 65536);
-  return 2.0 + 0.54e-6 * (double)M * (double)K > (double)(rounds * K) / 64 * (K % 64 ? 0.45 : 0.33);
-}
 LinearWs linear_ws(int64_t M, int64_t K, int64_t N, int cfg, bool ragged = false) {
   if (cfg >= 0) return layout_ws(M, K, N, cfg, pick_split(cfg, M, N, K), quantize_once(cfg, K));
   const bool few = M <= 32 && !ragged;
