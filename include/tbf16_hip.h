@@ -139,12 +139,12 @@ int tbf16_gemm_f16(const void* a16, int64_t M, int64_t K, int64_t lda, const flo
  * xT NULL (exps_ws too): no transposed copy, for the further layers that read one x.
  * Backward: dx = dY W from dY rows by L1 norm at t_rows and W columns at t_w; dw = dY^T X
  * from dY's columns (with sx folded in) at t_dy and xT; db = the columns' fp32 sums, bf16.
- * Each of dx (M, K), dw (N, K), db (N,) may be NULL. */
+ * Each of dx (M, K), dw (N, K), db (N,) may be NULL; its workspace query says which are not. */
 size_t tbf16_train_linear_fwd_ws_bytes(int64_t N, int64_t K);
 int tbf16_train_linear_fwd(const void* x, int64_t M, int64_t K, int64_t ldx, const void* w, int64_t N, int64_t ldw,
                            const void* bias, int t, void* x16, void* xT, int64_t ldT, float* sx, int32_t* exps_ws,
                            void* y, int64_t ldy, void* ws, int64_t ws_bytes, void* stream);
-size_t tbf16_train_linear_bwd_ws_bytes(int64_t M, int64_t N, int64_t K);
+size_t tbf16_train_linear_bwd_ws_bytes(int64_t M, int64_t N, int64_t K, int dx, int dw, int db);
 int tbf16_train_linear_bwd(const void* dy, int64_t M, int64_t N, int64_t lddy, const void* w, int64_t K, int64_t ldw,
                            const void* xT, int64_t ldT, const float* sx, int t_w, int t_rows, int t_dy, void* dx,
                            void* dw, void* db, void* ws, int64_t ws_bytes, void* stream);

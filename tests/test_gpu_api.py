@@ -433,13 +433,14 @@ def _to_double(m):
 
 
 @pytest.mark.parametrize("layout", ["whole", "view"])
-@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (37, 264, 72), (130, 520, 1032), (1000, 768, 256)])
+@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (37, 264, 72), (130, 520, 1032), (1000, 768, 256), (4100, 72, 8200)])
 @pytest.mark.parametrize("grads", ["xwb", "x", "w", "b", "xb"])
 def test_autograd_linear_one_call_matches_passes(dev, monkeypatch, M, K, N, grads, layout):
     """The training linear in one native call each way against the pass-by-pass route:
     the same bits (db: fp32 sums in another order, so within one bf16 rounding and the
     sum's own error), for every set of wanted gradients, row strides wider than the
-    matrix, and an activation that two layers read."""
+    matrix, an activation that two layers read, and a dY so large that its two fp16 copies
+    share a buffer."""
     import tbf16.autograd as ag
     from tbf16 import routing
     g = torch.Generator().manual_seed(M + N)

@@ -178,6 +178,19 @@ def test_linear_keeps_one_copy_of_an_activation(linear_calls, N):
     assert kept[0].data_ptr() not in [a for _, args in linear_calls[first:] for a in args]
 
 
+@pytest.mark.parametrize("M,N,K", [(8193, 2048, 768), (4096, 32000, 768), (8193, 4096, 64)])
+def test_linear_backward_workspace_holds_what_is_wanted(M, N, K):
+    """The backward's workspace: W's fp16 columns and dY's rows for dX, dY's columns for dW, and
+    where dY is large its two copies in one place; the rest is vectors and three sets of at most 2^21 partial results."""
+    ws = lambda *want: _ext.lib().tbf16_train_linear_bwd_ws_bytes(M, N, K, *want)
+    W, dY = 2 * N * K, 2 * N * (M + -M % 8)
+    rest = 32 * (M + N + K) + 3 * (9 << 20)
+    assert W + dY <= ws(1, 0, 0) + 16 * N <= W + dY + rest
+    assert dY <= ws(0, 1, 0) <= dY + rest
+    assert ws(0, 0, 1) <= rest
+    assert W + dY <= ws(1, 1, 1) <= W + dY + rest + (dY if 2 * M * N < 64 << 20 else 0)
+
+
 @pytest.mark.parametrize("B,C,O,side,k,native", [
     (1, 8, 8, 1024, 3, False), (1, 16, 16, 512, 3, False),     # 8 and 4 times the input's memory
     (1, 3, 64, 512, 5, False), (1, 4, 320, 512, 3, False),     # few channels, large images

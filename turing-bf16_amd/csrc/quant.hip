@@ -649,37 +649,44 @@ extern "C" int tbf16_train_linear_fwd(const void* x, int64_t M, int64_t K, int64
 }
 
 namespace {
+// Bytes of dY from which dX's rows and dW's columns of it take turns in one buffer, dW's
+// written after dX's product: a launch more, and a copy of dY less at the peak.
+constexpr int64_t kTurnBytes = (int64_t)64 << 20;
 struct TrainBwdWs {
   size_t wpart, dpart, dsum, wexp, dexp, swc, sdyc, sdy, ones, wcT, dycT, dy16, total;
+  bool turns;
 };
-TrainBwdWs train_bwd_ws(int64_t M, int64_t N, int64_t K) {
+// what the wanted outputs need, and no more
+TrainBwdWs train_bwd_ws(int64_t M, int64_t N, int64_t K, bool dx, bool dw, bool db) {
   TrainBwdWs w{};
   size_t at = 0;
-  auto take = [&](size_t bytes) {
+  auto take = [&](bool want, size_t bytes) {
     const size_t o = at;
-    at += align_up(bytes, 256);
+    if (want) at += align_up(bytes, 256);
     return o;
   };
   const int64_t M8 = cdiv(M, 8) * 8, wch = col_chunks(N, K), dch = col_chunks(M, N);
-  w.wpart = take((size_t)(wch * K) * 4);
-  w.dpart = take((size_t)(dch * N) * 4);
-  w.dsum = take((size_t)(dch * N) * 4);
-  w.wexp = take((size_t)K * 4);
-  w.dexp = take((size_t)N * 4);
-  w.swc = take((size_t)K * 4);
-  w.sdyc = take((size_t)N * 4);
-  w.sdy = take((size_t)M * 4);
-  w.ones = take((size_t)K * 4);
-  w.wcT = take((size_t)K * (size_t)N * 2);
-  w.dycT = take((size_t)N * (size_t)M8 * 2);
-  w.dy16 = take((size_t)M * (size_t)N * 2);
-  w.total = at;
+  const bool cols = dw || db;
+  w.wpart = take(dx, (size_t)(wch * K) * 4);
+  w.dpart = take(cols, (size_t)(dch * N) * 4);
+  w.dsum = take(db, (size_t)(dch * N) * 4);
+  w.wexp = take(dx, (size_t)K * 4);
+  w.dexp = take(cols, (size_t)N * 4);
+  w.swc = take(dx, (size_t)K * 4);
+  w.sdyc = take(cols, (size_t)N * 4);
+  w.sdy = take(dx, (size_t)M * 4);
+  w.ones = take(dw, (size_t)K * 4);
+  w.wcT = take(dx, (size_t)K * (size_t)N * 2);
+  w.turns = dx && dw && M * N * 2 >= kTurnBytes;
+  w.dycT = take(dw, (size_t)N * (size_t)M8 * 2);  // no smaller than dy16
+  w.dy16 = w.turns ? w.dycT : take(dx, (size_t)M * (size_t)N * 2);
+  w.total = std::max<size_t>(at, 256);
   return w;
 }
 }  // namespace
 
-extern "C" size_t tbf16_train_linear_bwd_ws_bytes(int64_t M, int64_t N, int64_t K) {
-  return M <= 0 || N <= 0 || K <= 0 ? 0 : train_bwd_ws(M, N, K).total;
+extern "C" size_t tbf16_train_linear_bwd_ws_bytes(int64_t M, int64_t N, int64_t K, int dx, int dw, int db) {
+  return M <= 0 || N <= 0 || K <= 0 ? 0 : train_bwd_ws(M, N, K, dx != 0, dw != 0, db != 0).total;
 }
 extern "C" int tbf16_train_linear_bwd(const void* dy, int64_t M, int64_t N, int64_t lddy, const void* w, int64_t K,
                                       int64_t ldw, const void* xT, int64_t ldT, const float* sx, int t_w, int t_rows,
@@ -690,10 +697,9 @@ extern "C" int tbf16_train_linear_bwd(const void* dy, int64_t M, int64_t N, int6
   TB_CHECK(dx == nullptr || aligned16(dx), "train_linear_bwd: misaligned dx");
   TB_CHECK(dw == nullptr || (aligned16(dw) && xT && aligned16(xT) && ldT == cdiv(M, 8) * 8 && sx),
            "train_linear_bwd: dw needs the transposed x16, its row stride and scales");
-  TB_CHECK(ws && aligned16(ws) && ws_bytes >= (int64_t)tbf16_train_linear_bwd_ws_bytes(M, N, K),
-           "train_linear_bwd: workspace too small");
+  const TrainBwdWs o = train_bwd_ws(M, N, K, dx != nullptr, dw != nullptr, db != nullptr);
+  TB_CHECK(ws && aligned16(ws) && ws_bytes >= (int64_t)o.total, "train_linear_bwd: workspace too small");
   hipStream_t st = as_stream(stream);
-  const TrainBwdWs o = train_bwd_ws(M, N, K);
   uint8_t* const b = static_cast<uint8_t*>(ws);
   TrainBwd p{};
   p.dy = (const uint16_t*)dy;
@@ -721,12 +727,17 @@ extern "C" int tbf16_train_linear_bwd(const void* dy, int64_t M, int64_t N, int6
   train_exps_kernel<<<(unsigned)(de + we + (dw ? cdiv(K, 256) : 0)), 256, 0, st>>>(p, de, we);
   TB_LAUNCH_CHECK("train_linear_bwd/exps");
   const int64_t tdx = cdiv(N, 256), td = dw ? tdx * cdiv(ldT, 64) : 0, twx = cdiv(K, 256), tw = dx ? twx * cdiv(N, 64) : 0;
-  if (td + tw > 0) {
-    train_transpose_kernel<<<(unsigned)(td + tw), 256, 0, st>>>(p, tdx, td, twx);
+  const int64_t td0 = o.turns ? 0 : td;  // dY's columns in the launch of W's
+  if (td0 + tw > 0) {
+    train_transpose_kernel<<<(unsigned)(td0 + tw), 256, 0, st>>>(p, tdx, td0, twx);
     TB_LAUNCH_CHECK("train_linear_bwd/transpose");
   }
   if (dx)
     if (int rc = tbf16_gemm_f16(p.dy16, M, N, N, p.sdy, p.wcT, K, N, p.swc, nullptr, dx, K, -1, stream)) return rc;
+  if (o.turns) {
+    train_transpose_kernel<<<(unsigned)td, 256, 0, st>>>(p, tdx, td, twx);
+    TB_LAUNCH_CHECK("train_linear_bwd/transpose dY");
+  }
   if (dw)
     if (int rc = tbf16_gemm_f16(p.dycT, N, ldT, ldT, p.sdyc, xT, K, ldT, p.ones, nullptr, dw, K, -1, stream)) return rc;
   return 0;

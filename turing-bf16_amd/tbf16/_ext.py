@@ -47,7 +47,7 @@ _SIGS = {
     "tbf16_gemm_f16": (I, [P, I64, I64, I64, P, P, I64, I64, P, P, P, I64, I, P]),
     "tbf16_train_linear_fwd_ws_bytes": (SZ, [I64, I64]),
     "tbf16_train_linear_fwd": (I, [P, I64, I64, I64, P, I64, I64, P, I, P, P, I64, P, P, P, I64, P, I64, P]),
-    "tbf16_train_linear_bwd_ws_bytes": (SZ, [I64, I64, I64]),
+    "tbf16_train_linear_bwd_ws_bytes": (SZ, [I64, I64, I64, I, I, I]),
     "tbf16_train_linear_bwd": (I, [P, I64, I64, I64, P, I64, I64, P, I64, P, I, I, I, P, P, P, P, I64, P]),
     "tbf16_gemv": (I, [P, P, I64, I64, I64, P, P, P, P]),
     "tbf16_head_amax": (I, [P, I, I64, I64, I64, I64, I64, I64, I64, P, P]),
