@@ -454,6 +454,24 @@ def test_attention_bias_forms(dev, monkeypatch, Sq, Sk, D, causal, split):
         assert rel(got.cpu(), torch.softmax(s, -1) @ v.double()) < TOL
 
 
+@pytest.mark.parametrize("B,H,Sq,Sk,D", [(1, 8, 100, 64, 64), (1, 8, 200, 512, 128), (1, 8, 200, 513, 128),
+                                         (2, 4, 130, 256, 64), (2, 4, 130, 257, 64), (9, 16, 128, 128, 64),
+                                         (9, 16, 129, 70, 128), (33, 8, 33, 33, 64), (1, 3, 7, 1, 128)])
+def test_attention_block_forms_of_short_calls(dev, B, H, Sq, Sk, D):
+    """Few keys or few queries on both sides of the lines between 4-wave blocks, split-key
+    blocks and 256-row blocks, with and without bias rows: fp64 softmax(q k^T scale + bias) v
+    within the bound of the other forms."""
+    g = torch.Generator().manual_seed(Sq + Sk)
+    q = torch.randn(B, H, Sq, D, generator=g).bfloat16().to(dev)
+    k, v = (torch.randn(B, H, Sk, D, generator=g).bfloat16().to(dev) for _ in range(2))
+    s = (q.double() @ k.double().transpose(-1, -2).contiguous()) * D ** -0.5
+    bias = torch.randn(B, 1, 1, Sk, generator=g).half().to(dev)
+    tri = torch.ones(Sq, Sk, dtype=torch.bool, device=dev).triu(1)
+    for mask, causal, ref in ((None, False, s), (bias, False, s + bias.double()), (None, True, s.masked_fill(tri, -math.inf))):
+        got = tbf16.sdpa(q, k, v, attn_mask=mask, is_causal=causal)
+        assert rel(got, torch.softmax(ref, -1) @ v.double()) < TOL
+
+
 @pytest.mark.parametrize("split", ["0", "1"])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("D", [64, 128, 192])

@@ -906,9 +906,17 @@ int launch_fwd_dp(FwdParams p, bool causal, bool has_bias, hipStream_t st, int n
   const bool pair = few && !single && getenv("TBF16_ATTN_NOPAIR") == nullptr;
   // the paired and single causal grids, and any grid whose 128-row tiles are no more than
   // the CUs, run as split-key blocks (key-padding mask, 24 heads, S = 1111, D = 64: kernel
-  // 36.6 -> 29.2 us); TBF16_ATTN_SPLIT=0 / 1 turns that off / on for any grid (benchmarking)
-  const bool split = split_ok && (sv || pair || (few && single) || tiles4 <= cus);
-  int nw = nw_override > 0 ? nw_override : pair ? 4 : (tiles8 >= 128 ? 8 : 4);
+  // 36.6 -> 29.2 us), the latter only where the keys are more than a few tiles: the merge
+  // and the larger prologue cost about 1.5 us, so fewer keys take 4-wave blocks. Device
+  // time of a call, 4-wave -> split-key blocks, 24 heads, 128 x keys, D = 128: 64 keys 13.8 ->
+  // 15.8 us, 512 21.5 -> 22.3, 1024 31.7 -> 31.0; with bias rows 64 keys 14.5 -> 16.5, 256 19.3
+  // -> 19.9, 512 25.6 -> 25.1. At most 128 queries a head leave half of a 256-row block
+  // idle: 4-wave blocks (1024 heads of 128 x 128, D = 64: 68.4 -> 50.0 us).
+  // TBF16_ATTN_SPLIT=0 / 1 turns split keys off / on for any grid (benchmarking)
+  const int64_t ktiles = cdiv(causal ? std::min(p.Sk, p.Sq) : p.Sk, BKV);
+  const bool one_round = tiles4 <= cus, short_keys = ktiles <= (has_bias ? 4 : 8);
+  const bool split = split_ok && (sv || pair || (few && single) || (one_round && !short_keys));
+  int nw = nw_override > 0 ? nw_override : pair || tiles8 < 128 || (one_round && short_keys) || p.Sq <= 128 ? 4 : 8;
   if (DP > 128 || p.drop_thr) nw = 4;
   if (split) nw = 8;
   const int64_t ntiles = cdiv(p.Sq, nw == 8 && !split ? 256 : 128);
