@@ -432,7 +432,7 @@ def _to_double(m):
     return d
 
 
-@pytest.mark.parametrize("layout", ["whole", "view"])
+@pytest.mark.parametrize("layout", ["whole", "view", "transposed"])
 @pytest.mark.parametrize("M,K,N", [(1, 8, 8), (37, 264, 72), (130, 520, 1032), (1000, 768, 256), (4100, 72, 8200)])
 @pytest.mark.parametrize("grads", ["xwb", "x", "w", "b", "xb"])
 def test_autograd_linear_one_call_matches_passes(dev, monkeypatch, M, K, N, grads, layout):
@@ -447,7 +447,7 @@ def test_autograd_linear_one_call_matches_passes(dev, monkeypatch, M, K, N, grad
 
     def mat(r, c):
         t = (torch.randn(r, c, generator=g) * torch.exp2(torch.randint(-9, 9, (r, 1), generator=g).float())).bfloat16().to(dev)
-        return torch.cat([t, t], 1)[:, :c] if layout == "view" else t
+        return torch.cat([t, t], 1)[:, :c] if layout == "view" else t.t().contiguous().t() if layout == "transposed" else t
 
     x, w1, w2, dy = mat(M, K), mat(N, K), mat(N, K), mat(M, N)
     b = torch.randn(N, generator=g).bfloat16().to(dev)

@@ -102,6 +102,17 @@ def test_linear_gradients_have_their_leaves_shapes(linear_calls, K, N):
     assert [g.shape for g in grads] == [t.shape for t in leaves]
 
 
+@pytest.mark.parametrize("M,K,N", [(40, 64, 24), (33, 1, 16), (10, 30, 12)])
+def test_linear_takes_an_activation_of_any_strides(linear_calls, M, K, N):
+    """A transposed activation, or one whose columns are not side by side."""
+    from tbf16 import autograd
+    for x in (torch.zeros(K, M, dtype=torch.bfloat16).t(), torch.zeros(M, 3 * K, dtype=torch.bfloat16)[:, ::3]):
+        x = x.detach().requires_grad_()
+        y = autograd.linear(x, torch.zeros(N, K, dtype=torch.bfloat16))
+        (dx,) = torch.autograd.grad(y, [x], torch.zeros_like(y))
+        assert y.shape == (M, N) and dx.shape == x.shape
+
+
 def test_linear_refuses_host_tensors(linear_calls, monkeypatch):
     """A weight (or a saved tensor that a hook unpacked) in host memory raises before any
     launch: its address must not reach a kernel."""
