@@ -206,12 +206,15 @@ def test_linear_backward_workspace_holds_what_is_wanted(M, N, K):
     (1, 8, 8, 1024, 3, False), (1, 16, 16, 512, 3, False),     # 8 and 4 times the input's memory
     (1, 3, 64, 512, 5, False), (1, 4, 320, 512, 3, False),     # few channels, large images
     (1, 96, 16, 1024, 3, False), (1, 96, 64, 1024, 3, True),   # 128 channels against 96 + O
+    (1, 3, 320, 450, 11, False), (1, 8, 320, 450, 7, False), (1, 16, 320, 400, 5, False),  # products with zeros
+    (1, 4, 64, 300, 5, True), (1, 24, 320, 400, 7, True), (1, 32, 320, 400, 5, True),
     (1, 16, 64, 256, 3, True), (2, 16, 64, 224, 7, True), (1, 512, 512, 128, 3, True), (1, 64, 64, 512, 3, True),
 ])
 @pytest.mark.parametrize("cl", [False, True])
 def test_conv2d_route_by_the_padded_copy(B, C, O, side, k, native, cl):
     """The native kernels pad the input's channels to a multiple of 64. They are used where
-    that copy is small, or no larger than the library path's own fp16 copies."""
+    that copy is small, or no larger than the library path's own fp16 copies, and not too many
+    products are with zeros."""
     if cl and C % 8:
         pytest.skip("channels last takes channels in multiples of 8")
     m = _converted(C, O, k, padding=k // 2)

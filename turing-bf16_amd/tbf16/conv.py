@@ -104,10 +104,17 @@ def _pair(v) -> ctypes.Array:
 _NATIVE_MIN_MACS = 1 << 29
 # Bytes of a padded input copy that are taken whatever the channels. Of 491 convolutions of
 # 3 to 96 channels (3x3, strided 3x3, 5x5, strided 7x7; 128 to 1024 pixels a side; both
-# layouts), native against library, 298 are taken, none more than 4% slower and the median
+# layouts), native against library, this takes 298, none more than 4% slower and the median
 # half the time (16 -> 64 at 256 x 256: 28 us against 55). At 32 MiB they begin to lose (16 -> 16
 # at 512 x 512: 70 us against 55; 8 -> 8 at 1024 x 1024: 222 against 98).
 _NATIVE_MAX_PADDED = 28 << 20
+# Products spent on padding that the native kernel is given, after what the library path
+# costs more: per output pixel its own slower products (1.5 for each real one), im2col (as 32
+# products a value) and the fp16 output (256 a value). Of 720 convolutions of 2 to 48 channels
+# (taps 2x2 to 11x11, 24 to 768 outputs, copies to 60 MiB) this leaves 372, the worst 19%
+# slower than the library, 7 by more than 5%; without it 3 -> 320 at 460 x 460, 11 x 11, takes
+# 944 us against 243, 8 -> 320 at 464 x 464, 7 x 7, twice the library's time.
+_NATIVE_MAX_WASTE = 8_000_000_000
 
 
 def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
@@ -135,9 +142,13 @@ def _native_layout(conv: nn.Module, x: torch.Tensor, padding, bias):
     if pixels * C * O * KH * KW < _NATIVE_MIN_MACS:
         return None
     # The kernels' copy of the input has its channels padded to a multiple of 64: it is the
-    # memory of the call, and with few channels its time too. It is taken where it is small
-    # or no larger than the two fp16 tensors around the library's convolution.
+    # memory of the call, and with few channels its products are most of the time. It is
+    # taken where it is small or no larger than the two fp16 tensors around the library's
+    # convolution, and the products with zeros are few enough.
     padded = B * (H + 2 * ph) * (W + 2 * pw) * (C + -C % 64)
+    taps = KH * KW
+    if pixels * ((O + -O % 64) * taps * (C + -C % 64 - 2.5 * C) - 32 * taps * C - 256 * O) > _NATIVE_MAX_WASTE:
+        return None
     small = 2 * padded <= _NATIVE_MAX_PADDED
     return int(nhwc) if small or (C >= 16 and padded <= B * C * H * W + pixels * O) else None
 
